@@ -191,6 +191,8 @@ extern "C" void pic_destroy(pic_ctx* ctx) {
     if (ctx->pin) (void)hipHostFree(ctx->pin);
     for (auto e : ctx->solve_ev)
         if (e) (void)hipEventDestroy(e);
+    for (auto e : ctx->pcg_ev)
+        if (e) (void)hipEventDestroy(e);
     for (auto& r : ctx->prof.recs) {
         (void)hipEventDestroy(r.a);
         (void)hipEventDestroy(r.b);

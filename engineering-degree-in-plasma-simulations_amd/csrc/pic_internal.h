@@ -269,6 +269,7 @@ struct pic_ctx {
     double* pin = nullptr;     // pinned host memory for the solvers' convergence reads
     size_t pin_bytes = 0;
     hipEvent_t solve_ev[2] = {nullptr, nullptr};  // pic_poisson's timing events
+    hipEvent_t pcg_ev[2] = {nullptr, nullptr};    // ends of PCG's queued batches
 };
 
 // ---- host helpers shared between translation units ----
@@ -391,7 +392,9 @@ inline double shost(const double* s) {
     for (int q = 0; q < NSTRIPE; q++) t += s[q * SSTRIDE];
     return t;
 }
-constexpr size_t SCRATCH_DOUBLES = 16384;  // ctx->scratch: [0, 4096) plain, [4096, ...) striped
+// ctx->scratch: [0, 4096) plain, [4096, 16384) striped, then the linear
+// solvers' partial sums
+constexpr size_t SCRATCH_DOUBLES = 32768;
 // learned preconditioner's striped scalars in ctx->scratch: restriction sums
 // {x^2, count}, line-search sums {c.res, c.A c}, then one spare (rz)
 constexpr int LEARNED_WS = 4096;

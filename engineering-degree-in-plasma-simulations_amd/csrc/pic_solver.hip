@@ -287,38 +287,147 @@ __global__ void __launch_bounds__(BLOCK)
     phi[u] = nbr_of<double>(t, phi, u, s);
 }
 
-// residual of the (Boltzmann) Poisson problem, three striped scalars at
-// out, out + SSIZE, out + 2 SSIZE: sum R^2 over all non-Dirichlet rows
-// (reference RMS numerator), sum R^2 over regular rows, sum b^2 over
-// regular rows.
+// Grid-wide sums of the linear solvers: every workgroup stores its partial
+// sum at part[blockIdx.x] (a plain store, nothing to clear and no atomics:
+// 1000 workgroups adding to one FP64 word took longer than the PCG kernels'
+// loads), and every workgroup of the kernel that needs the total adds the
+// partials up itself, while its first loads are in flight.
+// PART_MAX workgroups at most: four per CU, all resident at once at these
+// kernels' 44..107 registers (128^3 FP64 solve of 424 iterations: 20.0 ms with
+// up to 2048 workgroups, whose last ones ran as a second, nearly empty wave,
+// 18.8 with 1280, 16.1 with 1024, 16.3 with 512)
+constexpr int PART_MAX = 1024;
+// ctx->scratch offsets of the partials: three residual sums, then PCG's g.s,
+// g.g and d.z; the stop flag and the g.s ring follow
+constexpr int PART_F = 16384, PART_GS = PART_F + 3 * PART_MAX, PART_GG = PART_GS + PART_MAX,
+              PART_DZ = PART_GG + PART_MAX, PCG_FLAG = PART_DZ + PART_MAX, PCG_GS = PCG_FLAG + 8;
+static_assert(PCG_GS + 4 <= (int)SCRATCH_DOUBLES, "scratch layout");
+__device__ inline double sum_parts(const double* __restrict__ part, int n) {
+    __shared__ double red[BLOCK / 64];
+    double v = 0;
+    for (int q = threadIdx.x; q < n; q += BLOCK) v += part[q];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; w++) t += red[w];
+    __syncthreads();
+    return t;  // valid in every thread
+}
+// out[q] = the sum of part[q * PART_MAX ..] (one workgroup per q); out may
+// be pinned host memory
+__global__ void __launch_bounds__(BLOCK) k_sum_parts(const double* __restrict__ part, int n, double* out) {
+    const double t = sum_parts(part + (size_t)blockIdx.x * PART_MAX, n);
+    if (threadIdx.x == 0) out[blockIdx.x] = t;
+}
+
+// Four consecutive nodes u0 .. u0 + 3 (u0 a multiple of 4) per thread, in
+// flat order: a vector's own values in one 16-byte load (two in FP64), the
+// rows on either side likewise (unaligned where a row is not a multiple of 4
+// long), the i-neighbours beyond the group as single words.  Rows need no
+// special care: a group that straddles two i-lines holds face nodes there,
+// and face nodes do not use the 7-point stencil.  Addresses are clamped into
+// the array for the groups on its first and last planes.
+template <typename T>
+struct Q4 {
+    T a[4];
+};
+template <typename T>
+__device__ inline Q4<T> load4(const T* __restrict__ p) {
+    typedef T V __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    const V v = *reinterpret_cast<const V*>(p);
+    return Q4<T>{{v[0], v[1], v[2], v[3]}};
+}
+template <typename T>
+__device__ inline void store4(T* __restrict__ p, const T (&a)[4]) {
+    typedef T V __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    *reinterpret_cast<V*>(p) = V{a[0], a[1], a[2], a[3]};
+}
+template <typename T>
+struct Ring4 {
+    Q4<T> c, ym, yp, zm, zp;
+    T l, r;
+};
+template <typename T>
+__device__ inline void load_ring4(const T* __restrict__ v, unsigned u0, const Stencil& s, Ring4<T>& g) {
+    const unsigned n = (unsigned)s.nn, sj = (unsigned)s.sj, sk = (unsigned)s.sk, last = n - 4u;
+    g.c = load4(v + u0);
+    g.ym = load4(v + (u0 >= sj ? u0 - sj : 0u));
+    g.yp = load4(v + (u0 + sj <= last ? u0 + sj : last));
+    g.zm = load4(v + (u0 >= sk ? u0 - sk : 0u));
+    g.zp = load4(v + (u0 + sk <= last ? u0 + sk : last));
+    g.l = v[u0 >= 1u ? u0 - 1u : 0u];
+    g.r = v[u0 + 4u < n ? u0 + 4u : n - 1u];
+}
+// the 7-point operator at the group's node q (apply_A's order)
+template <typename T>
+__device__ inline T ring_A(const Ring4<T>& g, int q, const Stencil& s) {
+    const T xm = q == 0 ? g.l : g.c.a[q == 0 ? 0 : q - 1];
+    const T xp = q == 3 ? g.r : g.c.a[q == 3 ? 3 : q + 1];
+    return (T)s.cz * (g.zm.a[q] + g.zp.a[q]) + (T)s.cy * (g.ym.a[q] + g.yp.a[q]) + (T)s.cx * (xm + xp) -
+           (T)s.twos * g.c.a[q];
+}
+__device__ inline uint32_t load_types4(const uint8_t* __restrict__ nt, unsigned u0) {
+    return *reinterpret_cast<const uint32_t*>(nt + u0);
+}
+__device__ inline uint8_t type_at(uint32_t t4, int q) { return (uint8_t)((t4 >> (8 * q)) & 0xFFu); }
+
+// workgroups of the four-node kernels with partial sums: one group per
+// thread up to PART_MAX workgroups
+unsigned part_blocks(long long nn) {
+    long long b = (nn / 4 + BLOCK - 1) / BLOCK;
+    if (b > PART_MAX) b = PART_MAX;
+    return (unsigned)((b + NXCD - 1) / NXCD * NXCD);
+}
+
+// residual of the (Boltzmann) Poisson problem, three partial sums: sum R^2
+// over all non-Dirichlet rows (reference RMS numerator), sum R^2 over
+// regular rows, sum b^2 over regular rows.
 __global__ void __launch_bounds__(BLOCK)
     k_resid(Stencil s, SorArgs a, const uint8_t* __restrict__ nt, const double* __restrict__ phi,
-            const double* __restrict__ rho, double* __restrict__ out) {
+            const double* __restrict__ rho, double* __restrict__ part) {
     double r_all = 0, r_reg = 0, b_reg = 0;
-    long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        uint8_t t = nt[u];
-        if (t == NT_DIR) continue;
-        double p = phi[u];
-        if (t != NT_REG) {
-            double R = p - nbr_of<double>(t, phi, u, s);
-            r_all += R * R;
-            continue;
-        }
-        double q = rho[u];
+    auto regular = [&](double p, double rho_u, double sx, double sy, double sz) {
+        double q = rho_u;
         if (a.n0 != 0.0) q -= QE * (a.n0 * exp((p - a.phi0) * a.inv_te0));
-        double R = -p * s.twos + q * a.ieps + (phi[u - 1] + phi[u + 1]) * s.cx +
-                   (phi[u - s.sj] + phi[u + s.sj]) * s.cy + (phi[u - s.sk] + phi[u + s.sk]) * s.cz;
+        const double R = -p * s.twos + q * a.ieps + sx * s.cx + sy * s.cy + sz * s.cz;
+        const double b = rho_u * a.ieps;
         r_all += R * R;
         r_reg += R * R;
-        double b = rho[u] * a.ieps;
         b_reg += b * b;
+    };
+    auto face = [&](uint8_t t, long long u) {
+        const double R = phi[u] - nbr_of<double>(t, phi, u, s);
+        r_all += R * R;
+    };
+    long long end;
+    for (long long m = chunk_begin(s.nn / 4, end) + threadIdx.x; m < end; m += BLOCK) {
+        const unsigned u0 = 4u * (unsigned)m;
+        const uint32_t t4 = load_types4(nt, u0);
+        Ring4<double> g;
+        load_ring4(phi, u0, s, g);
+        const Q4<double> rh = load4(rho + u0);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint8_t t = type_at(t4, q);
+            if (t == NT_REG)
+                regular(g.c.a[q], rh.a[q], (q == 0 ? g.l : g.c.a[q == 0 ? 0 : q - 1]) +
+                                               (q == 3 ? g.r : g.c.a[q == 3 ? 3 : q + 1]),
+                        g.ym.a[q] + g.yp.a[q], g.zm.a[q] + g.zp.a[q]);
+            else if (t != NT_DIR)
+                face(t, u0 + q);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
+        const long long u = (s.nn & ~3ll) + threadIdx.x;
+        if (nt[u] != NT_REG && nt[u] != NT_DIR) face(nt[u], u);
     }
     double t0 = block_sum(r_all), t1 = block_sum(r_reg), t2 = block_sum(b_reg);
-    if (threadIdx.x == 0) {  // three striped scalars
-        sadd(out, t0);
-        sadd(out + SSIZE, t1);
-        sadd(out + 2 * SSIZE, t2);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = t0;
+        part[PART_MAX + blockIdx.x] = t1;
+        part[2 * PART_MAX + blockIdx.x] = t2;
     }
 }
 
@@ -327,159 +436,295 @@ __global__ void __launch_bounds__(BLOCK)
 //   b_u = 0 (Neumann), phi_u (Dirichlet), -rho_u/eps0 (regular)
 //   F = A phi - b - [regular] q n0 exp((phi-phi0)/Te0)/eps0
 //   P = [regular] q n0/(eps0 Te0) exp((phi-phi0)/Te0)
-// out[0] += F.F (all rows), out[1] += F.F (regular), out[2] += b.b (regular)
+// partial sums F.F (all rows), F.F (regular), b.b (regular)
+// START: the set-up of PCG on J y = F from y = 0 instead of F itself: g = -F
+// (TF), its Jacobi-scaled s = M g (NEU), and the partial sums g.s and g.g;
+// the stop flag of the iterations that follow is cleared.
 // ------------------------------------------------------------------------
 struct NewtonArgs {
     double ieps, phi0, n0, inv_te0;
 };
 
-template <typename TF>
+template <typename TF, bool START, bool NEU>
 __global__ void __launch_bounds__(BLOCK)
     k_F(Stencil s, NewtonArgs a, const uint8_t* __restrict__ nt, const double* __restrict__ phi,
-        const double* __restrict__ rho, TF* __restrict__ F, double* __restrict__ P,
-        double* __restrict__ out) {
-    double f_all = 0, f_reg = 0, b_reg = 0;
-    long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        uint8_t t = nt[u];
-        double Ap = apply_A<double>(t, u, s, [&](long long v) { return phi[v]; });
-        double b;
-        if (t == NT_REG)
-            b = -rho[u] * a.ieps;
-        else if (t == NT_DIR)
-            b = phi[u];
-        else
-            b = 0.0;
-        double f = Ap - b;
-        if (t == NT_REG && a.n0 != 0.0) {
-            double ex = exp((phi[u] - a.phi0) * a.inv_te0);
-            f -= QE * a.n0 * ex * a.ieps;
-            P[u] = QE * a.n0 * a.ieps * a.inv_te0 * ex;
-        } else if (P) {
-            P[u] = 0.0;
-        }
-        F[u] = (TF)f;
-        f_all += f * f;
+        const double* __restrict__ rho, TF* __restrict__ F, TF* __restrict__ sv, double* __restrict__ P,
+        double* __restrict__ scratch) {
+    double f_all = 0, f_reg = 0, b_reg = 0, gs = 0, gg = 0;
+    // one node: its row of F, and what START keeps of it
+    auto row = [&](uint8_t t, double Ap, double pu, double rho_u, double& Pu, TF& Fu, TF& su) {
+        Pu = 0.0;
+        double f;
         if (t == NT_REG) {
+            const double b = -rho_u * a.ieps;
+            f = Ap - b;
+            if (a.n0 != 0.0) {
+                const double ex = exp((pu - a.phi0) * a.inv_te0);
+                f -= QE * a.n0 * ex * a.ieps;
+                Pu = QE * a.n0 * a.ieps * a.inv_te0 * ex;
+            }
             f_reg += f * f;
             b_reg += b * b;
+        } else {
+            f = t == NT_DIR ? 0.0 : Ap;  // a Dirichlet row is phi - phi
         }
+        f_all += f * f;
+        Fu = START ? -(TF)f : (TF)f;
+        if (START) {
+            su = (TF)(1.0 / diagA(t, s)) * Fu;
+            gs += (double)Fu * (double)su;
+            gg += (double)Fu * (double)Fu;
+        }
+    };
+    long long end;
+    for (long long m = chunk_begin(s.nn / 4, end) + threadIdx.x; m < end; m += BLOCK) {
+        const unsigned u0 = 4u * (unsigned)m;
+        const uint32_t t4 = load_types4(nt, u0);
+        Ring4<double> g;
+        load_ring4(phi, u0, s, g);
+        const Q4<double> rh = load4(rho + u0);
+        TF f4[4], s4[4];
+        double P4[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint8_t t = type_at(t4, q);
+            double Ap = 0.0;
+            if (t == NT_REG)
+                Ap = ring_A(g, q, s);
+            else if (NEU && t != NT_DIR)
+                Ap = apply_A<double>(t, u0 + q, s, [&](long long v) { return phi[v]; });
+            s4[q] = 0;
+            row(t, Ap, g.c.a[q], rh.a[q], P4[q], f4[q], s4[q]);
+        }
+        store4(F + u0, f4);
+        if (START && NEU) store4(sv + u0, s4);
+        if (P) store4(P + u0, P4);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
+        const long long u = (s.nn & ~3ll) + threadIdx.x;
+        const uint8_t t = nt[u];
+        double Pu;
+        TF Fu, su = 0;
+        row(t, NEU ? apply_A<double>(t, u, s, [&](long long v) { return phi[v]; }) : 0.0, phi[u], rho[u], Pu, Fu, su);
+        F[u] = Fu;
+        if (START && NEU) sv[u] = su;
+        if (P) P[u] = Pu;
     }
     double t0 = block_sum(f_all), t1 = block_sum(f_reg), t2 = block_sum(b_reg);
     if (threadIdx.x == 0) {
-        atomicAdd(&out[0], t0);
-        atomicAdd(&out[1], t1);
-        atomicAdd(&out[2], t2);
+        scratch[PART_F + blockIdx.x] = t0;
+        scratch[PART_F + PART_MAX + blockIdx.x] = t1;
+        scratch[PART_F + 2 * PART_MAX + blockIdx.x] = t2;
+    }
+    if (START) {
+        double t3 = block_sum(gs), t4 = block_sum(gg);
+        if (threadIdx.x == 0) {
+            scratch[PART_GS + blockIdx.x] = t3;
+            scratch[PART_GG + blockIdx.x] = t4;
+            if (blockIdx.x == 0) scratch[PCG_FLAG] = 0.0;
+        }
     }
 }
 
 // ------------------------------------------------------------------------
-// PCG on J y = F, J = A - diag(P), M = 1/diag(A).  History arrays hold
-// dz[t] = d_t.z_t, gs[t] = g_t.s_t, gg[t] = g_t.g_t.
+// PCG on J y = F, J = A - diag(P), M = 1/diag(A), two kernels per iteration
+// over groups of four nodes, sums by partials.  Without Neumann faces M is
+// one constant on every row where g is not 0 (Dirichlet rows of F vanish),
+// so s = M g is formed from g where it is read; with them (NEU) s is kept.
+//
+// 128^3 nodes, FP64: k_pcg1 moves 41 B and k_pcg2 48 B per node of
+// cache-resident vectors, about 18 us each (5 TB/s); with one node per load,
+// eight nodes per thread, s stored and atomics on single words they took 27.8
+// and 30.2 us.  97^3 FP32: 5.6 and 5.0 us, close to an empty launch's 4 us,
+// against 14.1 and 13.5 us.
 // ------------------------------------------------------------------------
-struct PcgHist {
-    double* dz;
-    double* gs;
-    double* gg;
-};
-
 template <typename T>
 struct PcgVec {
-    T *y, *g, *s, *d0, *d1, *z;
-    const T* F;
-    const double* P;  // may be null
+    T *y, *g, *s, *z;  // s: NEU only
+    const double* P;   // may be null
 };
-
-// g = -F (y = 0), s = M g, d = -s, gs[0], gg[0]
-template <typename T>
-__global__ void __launch_bounds__(BLOCK)
-    k_pcg0(Stencil s, const uint8_t* __restrict__ nt, PcgVec<T> v, PcgHist h) {
-    double gs = 0, gg = 0;
-    long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        T g = -v.F[u];
-        T m = (T)(1.0 / diagA(nt[u], s));
-        T sv = m * g;
-        v.y[u] = 0;
-        v.g[u] = g;
-        v.s[u] = sv;
-        v.d0[u] = 0;
-        gs += (double)g * (double)sv;
-        gg += (double)g * (double)g;
-    }
-    double a = block_sum(gs), b = block_sum(gg);
-    if (threadIdx.x == 0) {
-        atomicAdd(&h.gs[0], a);
-        atomicAdd(&h.gg[0], b);
-    }
-}
 
 // d_new = beta d_old - s (beta = gs[t]/gs[t-1], 0 at t = 0); z = J d_new,
 // by the recurrence J d_new = beta J d_old - J s: the stencil of s alone
-// (seven loads instead of fourteen), the previous z in place
-template <typename T>
+// (one operand's neighbours instead of two), the previous z in place.
+// gg[t] is kept for the host's check.  Returns at once when the stop flag is
+// set (an earlier iteration converged).
+template <typename T, bool NEU>
 __global__ void __launch_bounds__(BLOCK)
-    k_pcg1(Stencil s, const uint8_t* __restrict__ nt, const T* __restrict__ dold,
-           T* __restrict__ dnew, const T* __restrict__ sv, T* __restrict__ z,
-           const double* __restrict__ P, PcgHist h, int t) {
+    k_pcg1(Stencil s, const uint8_t* __restrict__ nt, PcgVec<T> v, const T* __restrict__ dold,
+           T* __restrict__ dnew, double* __restrict__ scratch, double* __restrict__ ggh, int t) {
+    if (scratch[PCG_FLAG] != 0.0) return;  // (the whole grid)
+    const T* __restrict__ src = NEU ? v.s : v.g;
+    const T mreg = (T)(1.0 / diagA(NT_REG, s));  // M of a regular row (k_pcg2's s, rounded alike)
+    long long end;
+    long long m = chunk_begin(s.nn / 4, end) + threadIdx.x;
+    Ring4<T> r;
+    Q4<T> d4{}, z4{};
+    uint32_t t4 = 0;
+    auto load = [&]() {
+        const unsigned u0 = 4u * (unsigned)m;
+        t4 = load_types4(nt, u0);
+        load_ring4(src, u0, s, r);
+        if (t > 0) {
+            d4 = load4(dold + u0);
+            z4 = load4(v.z + u0);
+        }
+    };
+    if (m < end) load();
+    const double gs = sum_parts(scratch + PART_GS, gridDim.x);
     double beta = 0.0;
     if (t > 0) {
-        double den = h.gs[t - 1];
-        beta = den != 0.0 ? h.gs[t] / den : 0.0;
+        const double den = scratch[PCG_GS + ((t - 1) & 3)];
+        beta = den != 0.0 ? gs / den : 0.0;
     }
-    T bt = (T)beta;
+    const T bt = (T)beta;
     double acc = 0;
-    long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        uint8_t ty = nt[u];
-        const T su = sv[u];
-        T js = apply_A<T>(ty, u, s, [&](long long q) { return sv[q]; });
-        if (P) js -= (T)P[u] * su;
+    while (m < end) {
+        const unsigned u0 = 4u * (unsigned)m;
+        if (!NEU) {  // s = M g
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                r.c.a[q] *= mreg;
+                r.ym.a[q] *= mreg;
+                r.yp.a[q] *= mreg;
+                r.zm.a[q] *= mreg;
+                r.zp.a[q] *= mreg;
+            }
+            r.l *= mreg;
+            r.r *= mreg;
+        }
+        T dn[4], zn[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint8_t ty = type_at(t4, q);
+            const T su = r.c.a[q];
+            T js = su;  // a Dirichlet row
+            if (ty == NT_REG)
+                js = ring_A(r, q, s);
+            else if (NEU && ty != NT_DIR)
+                js = apply_A<T>(ty, u0 + q, s, [&](long long w) { return src[w]; });
+            if (v.P) js -= (T)v.P[u0 + q] * su;
+            dn[q] = -su + bt * d4.a[q];
+            zn[q] = -js + bt * z4.a[q];
+            acc += (double)dn[q] * (double)zn[q];
+        }
+        store4(dnew + u0, dn);
+        store4(v.z + u0, zn);
+        m += BLOCK;
+        if (m < end) load();
+    }
+    if (NEU && blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
+        const long long u = (s.nn & ~3ll) + threadIdx.x;
+        const T su = src[u];
+        T js = apply_A<T>(nt[u], u, s, [&](long long w) { return src[w]; });
+        if (v.P) js -= (T)v.P[u] * su;
         T du = -su, zu = -js;
         if (t > 0) {
             du += bt * dold[u];
-            zu += bt * z[u];
+            zu += bt * v.z[u];
         }
         dnew[u] = du;
-        z[u] = zu;
+        v.z[u] = zu;
         acc += (double)du * (double)zu;
     }
-    double a = block_sum(acc);
-    if (threadIdx.x == 0) atomicAdd(&h.dz[t], a);
+    const double a = block_sum(acc);
+    if (threadIdx.x == 0) scratch[PART_DZ + blockIdx.x] = a;
+    if (blockIdx.x == 0) {
+        const double gg = sum_parts(scratch + PART_GG, gridDim.x);
+        if (threadIdx.x == 0) {
+            scratch[PCG_GS + (t & 3)] = gs;
+            ggh[t] = gg;
+        }
+    }
 }
 
-// alpha = gs[t]/dz[t]; y += alpha d; g += alpha z; s = M g; gs[t+1], gg[t+1]
-template <typename T>
+// alpha = gs[t]/dz[t]; y += alpha d (y = 0 before t = 0); g += alpha z;
+// s = M g; gs[t+1], gg[t+1]
+template <typename T, bool NEU>
 __global__ void __launch_bounds__(BLOCK)
-    k_pcg2(Stencil s, const uint8_t* __restrict__ nt, T* __restrict__ y, T* __restrict__ g,
-           T* __restrict__ sv, const T* __restrict__ d, const T* __restrict__ z, PcgHist h,
-           int t) {
-    double den = h.dz[t];
-    T alpha = (T)(den != 0.0 ? h.gs[t] / den : 0.0);
-    double gs = 0, gg = 0;
+    k_pcg2(Stencil s, const uint8_t* __restrict__ nt, PcgVec<T> v, const T* __restrict__ d,
+           double* __restrict__ scratch, int t) {
+    if (scratch[PCG_FLAG] != 0.0) return;  // (the whole grid)
+    const T mreg = (T)(1.0 / diagA(NT_REG, s));
     long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        T gu = g[u] + alpha * z[u];
-        y[u] += alpha * d[u];
-        T m = (T)(1.0 / diagA(nt[u], s));
-        T su = m * gu;
-        g[u] = gu;
-        sv[u] = su;
+    long long m = chunk_begin(s.nn / 4, end) + threadIdx.x;
+    Q4<T> g4, z4, y4{}, d4;
+    uint32_t t4 = 0;
+    auto load = [&]() {
+        const unsigned u0 = 4u * (unsigned)m;
+        g4 = load4(v.g + u0);
+        z4 = load4(v.z + u0);
+        if (t > 0) y4 = load4(v.y + u0);
+        d4 = load4(d + u0);
+        if (NEU) t4 = load_types4(nt, u0);
+    };
+    if (m < end) load();
+    const double den = sum_parts(scratch + PART_DZ, gridDim.x);
+    const T alpha = (T)(den != 0.0 ? scratch[PCG_GS + (t & 3)] / den : 0.0);
+    double gs = 0, gg = 0;
+    auto sums = [&](T gu, T su) {
         gs += (double)gu * (double)su;
         gg += (double)gu * (double)gu;
+    };
+    while (m < end) {
+        const unsigned u0 = 4u * (unsigned)m;
+        T gn[4], yn[4], sn[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            gn[q] = g4.a[q] + alpha * z4.a[q];
+            yn[q] = y4.a[q] + alpha * d4.a[q];
+            sn[q] = (NEU ? (T)(1.0 / diagA(type_at(t4, q), s)) : mreg) * gn[q];
+            sums(gn[q], sn[q]);
+        }
+        store4(v.g + u0, gn);
+        store4(v.y + u0, yn);
+        if (NEU) store4(v.s + u0, sn);
+        m += BLOCK;
+        if (m < end) load();
     }
-    double a = block_sum(gs), b = block_sum(gg);
+    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
+        const long long u = (s.nn & ~3ll) + threadIdx.x;
+        if (NEU) {
+            const T gu = v.g[u] + alpha * v.z[u];
+            const T su = (T)(1.0 / diagA(nt[u], s)) * gu;
+            v.y[u] = (t > 0 ? v.y[u] : (T)0) + alpha * d[u];
+            v.g[u] = gu;
+            v.s[u] = su;
+            sums(gu, su);
+        }
+    }
+    const double a = block_sum(gs), b = block_sum(gg);
     if (threadIdx.x == 0) {
-        atomicAdd(&h.gs[t + 1], a);
-        atomicAdd(&h.gg[t + 1], b);
+        scratch[PART_GS + blockIdx.x] = a;
+        scratch[PART_GG + blockIdx.x] = b;
     }
 }
 
-// phi -= y on non-Dirichlet rows (PotentialSolver.cpp:225-228)
+// The end of a batch of iterations (t0, t1]: g.g of each to the host (pinned
+// memory), and the stop flag when one is within the target.
+__global__ void __launch_bounds__(BLOCK)
+    k_pcg_check(double* __restrict__ scratch, const double* __restrict__ ggh, int nb, int t0, int t1,
+                double target2, double* host) {
+    if (scratch[PCG_FLAG] != 0.0) return;
+    const double gg = sum_parts(scratch + PART_GG, nb);
+    __shared__ int hit;
+    if (threadIdx.x == 0) hit = 0;
+    __syncthreads();
+    for (int q = t0 + 1 + threadIdx.x; q <= t1; q += BLOCK) {
+        const double x = q == t1 ? gg : ggh[q];
+        host[q - t0 - 1] = x;
+        if (x <= target2) hit = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && hit) scratch[PCG_FLAG] = 1.0;
+}
+
+// phi -= y on non-Dirichlet rows (PotentialSolver.cpp:225-228); with part,
+// the partial sums of y.y over them
 template <typename T>
 __global__ void __launch_bounds__(BLOCK)
     k_update_phi(Stencil s, const uint8_t* __restrict__ nt, double* __restrict__ phi,
-                 const T* __restrict__ y, double* __restrict__ out) {
+                 const T* __restrict__ y, double* __restrict__ part) {
     double yy = 0;
     long long end;
     for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
@@ -488,8 +733,9 @@ __global__ void __launch_bounds__(BLOCK)
         phi[u] -= yv;
         yy += yv * yv;
     }
+    if (!part) return;
     double a = block_sum(yy);
-    if (threadIdx.x == 0) atomicAdd(out, a);
+    if (threadIdx.x == 0) part[blockIdx.x] = a;
 }
 
 Stencil make_stencil(const GridC& g, bool axis_swap) {
@@ -554,18 +800,20 @@ static bool has_neumann(pic_ctx* ctx) {
     return ctx->has_neumann;
 }
 
-static int residual_norms(pic_ctx* ctx, const Stencil& st, const SorArgs& a, double out[3],
-                          const double* phi = nullptr) {
-    double* sums = ctx->scratch + LEARNED_WS + 5 * SSIZE;  // three striped scalars
-    PIC_HIP(ctx, hipMemsetAsync(sums, 0, 3 * SSIZE * sizeof(double), ctx->stream));
-    k_resid<<<stencil_blocks(st.nn), BLOCK, 0, ctx->stream>>>(st, a, ctx->ntype, phi ? phi : ctx->phi,
-                                                             ctx->rho, sums);
+// queues the residual sums of phi (k_resid's three) into out (pinned memory)
+static int queue_residual(pic_ctx* ctx, const Stencil& st, const SorArgs& a, double* out) {
+    const unsigned nb = part_blocks(st.nn);
+    k_resid<<<nb, BLOCK, 0, ctx->stream>>>(st, a, ctx->ntype, ctx->phi, ctx->rho, ctx->scratch + PART_F);
+    k_sum_parts<<<3, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nb, out);
     PIC_HIP(ctx, hipGetLastError());
-    std::vector<double> h(3 * SSIZE);
-    PIC_HIP(ctx, hipMemcpyAsync(h.data(), sums, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                                ctx->stream));
+    return PIC_OK;
+}
+static int residual_norms(pic_ctx* ctx, const Stencil& st, const SorArgs& a, double out[3]) {
+    int rc = pic_ensure_pin(ctx, 3 * sizeof(double));
+    if (!rc) rc = queue_residual(ctx, st, a, ctx->pin);
+    if (rc) return rc;
     PIC_HIP(ctx, pic_spin_wait(ctx->stream));
-    for (int q = 0; q < 3; q++) out[q] = shost(h.data() + q * SSIZE);
+    for (int q = 0; q < 3; q++) out[q] = ctx->pin[q];
     return PIC_OK;
 }
 
@@ -657,117 +905,110 @@ static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
     return conv ? PIC_OK : PIC_NOT_CONVERGED;
 }
 
-// inner PCG on J y = F (vectors of type T); stops when ||g|| <= target or at
-// max_it; returns iterations used.
-template <typename T>
-static int pcg_inner(pic_ctx* ctx, const Stencil& s, T* base, const double* P, double target2,
-                     int max_it, int check, int* iters, double* gg_last) {
-    size_t nn = (size_t)s.nn;
-    PcgVec<T> v;
-    v.F = base;
-    v.y = base + nn;
-    v.g = base + 2 * nn;
-    v.s = base + 3 * nn;
-    v.d0 = base + 4 * nn;
-    v.d1 = base + 5 * nn;
-    v.z = base + 6 * nn;
-    v.P = P;
-    double* hist = (double*)(base + 7 * nn);
-    hist = (double*)(((uintptr_t)hist + 255) & ~(uintptr_t)255);
-    PcgHist h;
-    h.dz = hist;
-    h.gs = hist + (max_it + 2);
-    h.gg = hist + 2 * (max_it + 2);
-    PIC_HIP(ctx, hipMemsetAsync(hist, 0, 3 * (size_t)(max_it + 2) * sizeof(double), ctx->stream));
-    unsigned nb = stencil_blocks_red(s.nn);
-    {
-        // set-up launches are not counted as PCG iterations
-        k_pcg0<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v, h);
-    }
-    PIC_HIP(ctx, hipGetLastError());
-    std::vector<double> hg(max_it + 2);
-    PIC_HIP(ctx, hipMemcpyAsync(hg.data(), h.gg, sizeof(double), hipMemcpyDeviceToHost,
-                                ctx->stream));
-    PIC_HIP(ctx, pic_spin_wait(ctx->stream));
-    *gg_last = hg[0];
-    if (hg[0] <= target2) {  // already converged (zero RHS included)
-        *iters = 0;
-        return PIC_OK;
-    }
-    T* dold = v.d0;
-    T* dnew = v.d1;
-    int t = 0, last_checked = 0;
-    while (t < max_it) {
-        int upto = std::min(max_it, t + check);
-        for (; t < upto; t++) {  // one profiled "launch" = one PCG iteration (2 kernels)
-            PicProfScope ps(ctx, PIC_K_PCG);
-            k_pcg1<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, dold, dnew, v.s, v.z, P, h,
-                                                     t);
-            k_pcg2<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v.y, v.g, v.s, dnew, v.z, h,
-                                                     t);
-            std::swap(dold, dnew);
+// The iterations of PCG on J y = F after k_F's set-up (vectors of type T, g.g
+// = gg0 > target2); stops at the end of the first batch of `check` iterations
+// in which g.g reached target2, or at max_it.  The host queues one batch
+// ahead of the one it waits for, so the device never idles during a check;
+// once a batch has converged the kernels of the next return at once (the
+// stop flag), so y is the one of the batch that converged.  hp: 2 * check
+// doubles of pinned memory; ggh: max_it + 1 doubles on the device.
+template <typename T, bool NEU>
+static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, T* d1, double* ggh, double* hp,
+                     double target2, int max_it, int check, int* iters) {
+    const unsigned nb = part_blocks(s.nn);
+    for (auto& e : ctx->pcg_ev)
+        if (!e) PIC_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    // profiled runs wait for every batch, so that no returned-at-once
+    // iteration is counted
+    const int ahead = ctx->prof.on ? 1 : 2;
+    int t = 0;                        // iterations queued
+    int beg[2], end[2], queued = 0, done = 0;  // batches queued and waited for
+    T *dold = d0, *dnew = d1;
+    for (;;) {
+        while (t < max_it && queued - done < ahead) {
+            const int q = queued & 1, t0 = t, upto = std::min(max_it, t + check);
+            for (; t < upto; t++) {  // one profiled "launch" = one PCG iteration (2 kernels)
+                PicProfScope ps(ctx, PIC_K_PCG);
+                k_pcg1<T, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v, dold, dnew, ctx->scratch, ggh, t);
+                k_pcg2<T, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v, dnew, ctx->scratch, t);
+                std::swap(dold, dnew);
+            }
+            k_pcg_check<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch, ggh, (int)nb, t0, t, target2,
+                                                      hp + (size_t)q * check);
+            PIC_HIP(ctx, hipGetLastError());
+            PIC_HIP(ctx, hipEventRecord(ctx->pcg_ev[q], ctx->stream));
+            beg[q] = t0;
+            end[q] = t;
+            queued++;
         }
-        PIC_HIP(ctx, hipGetLastError());
-        PIC_HIP(ctx, hipMemcpyAsync(hg.data() + last_checked + 1, h.gg + last_checked + 1,
-                                    (size_t)(t - last_checked) * sizeof(double),
-                                    hipMemcpyDeviceToHost, ctx->stream));
-        PIC_HIP(ctx, pic_spin_wait(ctx->stream));
-        for (int q = last_checked + 1; q <= t; q++) {
-            if (!(hg[q] == hg[q])) return pic_fail(ctx, PIC_ERR_NUMERIC, "PCG produced NaN");
-            if (hg[q] <= target2) {
-                *iters = t;
-                *gg_last = hg[q];
+        if (done == queued) {
+            *iters = t;
+            return PIC_NOT_CONVERGED;
+        }
+        const int q = done & 1;
+        PIC_HIP(ctx, pic_spin_event(ctx->pcg_ev[q]));
+        done++;
+        const volatile double* h = hp + (size_t)q * check;
+        for (int e = 0; e < end[q] - beg[q]; e++) {
+            if (!(h[e] == h[e])) return pic_fail(ctx, PIC_ERR_NUMERIC, "PCG produced NaN");
+            if (h[e] <= target2) {
+                *iters = end[q];
                 return PIC_OK;
             }
         }
-        last_checked = t;
-        *gg_last = hg[t];
     }
-    *iters = t;
-    return PIC_NOT_CONVERGED;
 }
 
 // Newton + PCG (PotentialSolver.cpp:178-241).  The linear case (n0 == 0)
 // needs a single Newton step; each Newton step restarts PCG from y = 0.
-static int solve_pcg(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st, bool mixed) {
+template <typename T, bool NEU>
+static int solve_pcg_t(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st) {
     const GridC& g = ctx->g;
+    constexpr bool mixed = sizeof(T) == sizeof(float);
     size_t nn = (size_t)g.nn;
     Stencil s = make_stencil(g, (p->flags & PIC_SOLVE_AXIS_SWAP) != 0);
     bool nonlinear = p->n0 != 0.0;
     int max_it = p->max_it > 0 ? p->max_it : 10000;
-    int check = p->check_every > 0 ? p->check_every : 8;
-    size_t tsz = mixed ? sizeof(float) : sizeof(double);
-    size_t bytes = 7 * nn * tsz + 256 + 3 * (size_t)(max_it + 2) * sizeof(double);
-    size_t pbytes = nonlinear ? nn * sizeof(double) : 0;
-    int rc = pic_ensure_work(ctx, bytes + pbytes + 256);
+    int check = std::min(p->check_every > 0 ? p->check_every : 8, max_it);
+    // y, g, d0, d1, z (s), P, the g.g history; each vector on a 256-byte line
+    const size_t vs = (nn * sizeof(T) + 255) & ~(size_t)255;
+    const size_t ps = nonlinear ? (nn * sizeof(double) + 255) & ~(size_t)255 : 0;
+    const int nvec = NEU ? 6 : 5;
+    int rc = pic_ensure_work(ctx, nvec * vs + ps + ((size_t)max_it + 2) * sizeof(double));
+    if (rc) return rc;
+    rc = pic_ensure_pin(ctx, (8 + 2 * (size_t)check) * sizeof(double));
     if (rc) return rc;
     char* wbase = (char*)ctx->work;
-    double* P = nonlinear ? (double*)(wbase + ((bytes + 255) & ~(size_t)255)) : nullptr;
+    auto vec = [&](int q) { return reinterpret_cast<T*>(wbase + q * vs); };
+    double* P = nonlinear ? (double*)(wbase + nvec * vs) : nullptr;
+    double* ggh = (double*)(wbase + nvec * vs + ps);
+    PcgVec<T> v;
+    v.y = vec(0);
+    v.g = vec(1);
+    v.z = vec(4);
+    v.s = NEU ? vec(5) : nullptr;
+    v.P = P;
+    volatile double* hp = ctx->pin;  // [0, 5) sums of k_F, [5] y.y, [8, ...) g.g of the batches
     NewtonArgs na;
     na.ieps = 1.0 / EPS0;
     na.phi0 = p->phi0;
     na.n0 = p->n0;
     na.inv_te0 = 1.0 / (p->Te0 != 0 ? p->Te0 : 1.0);
-    unsigned nb = stencil_blocks_red(s.nn);
+    const unsigned nb = part_blocks(s.nn);
     int total_it = 0, newton = 0;
-    bool conv = false;
+    bool conv = false, have_r = false;
     double fr[3];
     const int newton_max = nonlinear ? 20 : 1000;  // PotentialSolver.cpp:179
     for (newton = 0; newton < newton_max; newton++) {
-        PIC_HIP(ctx, hipMemsetAsync(ctx->scratch, 0, 4 * sizeof(double), ctx->stream));
-        {
-            // set-up launches are not counted as PCG iterations
-            if (mixed)
-                k_F<float><<<nb, BLOCK, 0, ctx->stream>>>(s, na, ctx->ntype, ctx->phi, ctx->rho,
-                                                          (float*)wbase, P, ctx->scratch);
-            else
-                k_F<double><<<nb, BLOCK, 0, ctx->stream>>>(s, na, ctx->ntype, ctx->phi, ctx->rho,
-                                                           (double*)wbase, P, ctx->scratch);
-        }
+        // set-up launches are not counted as PCG iterations
+        k_F<T, true, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, na, ctx->ntype, ctx->phi, ctx->rho, v.g, v.s, P,
+                                                         ctx->scratch);
+        // F.F (all rows, regular), b.b, and PCG's g.s, g.g
+        k_sum_parts<<<5, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nb, ctx->pin);
         PIC_HIP(ctx, hipGetLastError());
-        PIC_HIP(ctx, hipMemcpyAsync(fr, ctx->scratch, sizeof(fr), hipMemcpyDeviceToHost,
-                                    ctx->stream));
         PIC_HIP(ctx, pic_spin_wait(ctx->stream));
+        for (int q = 0; q < 3; q++) fr[q] = hp[q];
+        const double gg0 = hp[4];
         // target on the inner residual g (g = -F at y = 0)
         double target2;
         if (p->tol_kind == PIC_TOL_REF_RMS)
@@ -775,14 +1016,14 @@ static int solve_pcg(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
         else
             target2 = p->tol * p->tol * (fr[2] > 0 ? fr[2] : 1.0);
         if (!nonlinear && fr[0] <= target2) {
-            conv = true;
+            conv = have_r = true;
             break;
         }
         // relative criterion on the nonlinear problem: the FP64 residual F
         // of the current phi over the regular rows (the Newton iterate is
         // judged by the residual, not by the size of its last step)
         if (nonlinear && p->tol_kind == PIC_TOL_REL && fr[1] <= target2) {
-            conv = true;
+            conv = have_r = true;
             break;
         }
         double inner_target2 = target2;
@@ -794,31 +1035,24 @@ static int solve_pcg(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
             // residual, or below the final tolerance
             inner_target2 = std::max(target2 * 0.25, fr[0] * 1e-8);
         }
-        int its = 0;
-        double gg = 0;
-        if (mixed)
-            rc = pcg_inner<float>(ctx, s, (float*)wbase, P, inner_target2, max_it - total_it, check,
-                                  &its, &gg);
-        else
-            rc = pcg_inner<double>(ctx, s, (double*)wbase, P, inner_target2, max_it - total_it,
-                                   check, &its, &gg);
-        total_it += its;
-        if (rc < 0) return rc;
-        PIC_HIP(ctx, hipMemsetAsync(ctx->scratch, 0, sizeof(double), ctx->stream));
-        {
-            // set-up launches are not counted as PCG iterations
-            if (mixed)
-                k_update_phi<float><<<nb, BLOCK, 0, ctx->stream>>>(
-                    s, ctx->ntype, ctx->phi, (const float*)wbase + nn, ctx->scratch);
-            else
-                k_update_phi<double><<<nb, BLOCK, 0, ctx->stream>>>(
-                    s, ctx->ntype, ctx->phi, (const double*)wbase + nn, ctx->scratch);
+        double yy = 0;
+        if (!(gg0 <= inner_target2)) {  // otherwise y = 0 (a zero right-hand side included)
+            int its = 0;
+            rc = pcg_inner<T, NEU>(ctx, s, v, vec(2), vec(3), ggh, ctx->pin + 8, inner_target2, max_it - total_it,
+                                   check, &its);
+            total_it += its;
+            if (rc < 0) return rc;
+            const bool want_yy = nonlinear && p->tol_kind == PIC_TOL_REF_RMS;
+            k_update_phi<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->phi, v.y,
+                                                           want_yy ? ctx->scratch + PART_F : nullptr);
+            PIC_HIP(ctx, hipGetLastError());
+            if (want_yy) {
+                k_sum_parts<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nb, ctx->pin + 5);
+                PIC_HIP(ctx, hipGetLastError());
+                PIC_HIP(ctx, pic_spin_wait(ctx->stream));
+                yy = hp[5];
+            }
         }
-        PIC_HIP(ctx, hipGetLastError());
-        double yy;
-        PIC_HIP(ctx, hipMemcpyAsync(&yy, ctx->scratch, sizeof(double), hipMemcpyDeviceToHost,
-                                    ctx->stream));
-        PIC_HIP(ctx, pic_spin_wait(ctx->stream));
         if (nonlinear && p->tol_kind == PIC_TOL_REF_RMS) {
             if (std::sqrt(yy / (double)nn) < 1e-3) {  // NR_TOL, PotentialSolver.cpp:180, :229-233
                 conv = true;
@@ -828,23 +1062,32 @@ static int solve_pcg(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
         }
         if (total_it >= max_it) break;
     }
-    SorArgs a;
-    a.omega = 1;
-    a.ieps = 1.0 / EPS0;
-    a.itwos = 1.0 / s.twos;
-    a.phi0 = p->phi0;
-    a.n0 = p->n0;
-    a.inv_te0 = na.inv_te0;
     double r[3];
-    Stencil sphys = make_stencil(g, (p->flags & PIC_SOLVE_AXIS_SWAP) != 0);
-    rc = residual_norms(ctx, sphys, a, r);
-    if (rc) return rc;
+    if (have_r && !NEU) {  // k_F's sums are the residual of the final phi
+        for (int q = 0; q < 3; q++) r[q] = fr[q];
+    } else {
+        SorArgs a;
+        a.omega = 1;
+        a.ieps = 1.0 / EPS0;
+        a.itwos = 1.0 / s.twos;
+        a.phi0 = p->phi0;
+        a.n0 = p->n0;
+        a.inv_te0 = na.inv_te0;
+        rc = residual_norms(ctx, s, a, r);
+        if (rc) return rc;
+    }
     st->converged = conv;
     st->iterations = total_it;
     st->newton_iterations = newton;
     st->ref_l2 = std::sqrt(r[0] / (double)nn);
     st->rel_residual = r[2] > 0 ? std::sqrt(r[1] / r[2]) : std::sqrt(r[1]);
     return conv ? PIC_OK : PIC_NOT_CONVERGED;
+}
+
+static int solve_pcg(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st, bool mixed) {
+    if (has_neumann(ctx))
+        return mixed ? solve_pcg_t<float, true>(ctx, p, st) : solve_pcg_t<double, true>(ctx, p, st);
+    return mixed ? solve_pcg_t<float, false>(ctx, p, st) : solve_pcg_t<double, false>(ctx, p, st);
 }
 
 // ------------------------------------------------------------------------
@@ -1596,12 +1839,12 @@ static int solve_learned(pic_ctx* ctx, const pic_solver_params* p, pic_solver_st
     auto precond = [&](const double* rin, float* zout, const double* qv, double* zq, double* rz) {
         return learned_precond(ctx, s, rin, zout, ftmp, qv, zq, rz);
     };
-    // pinned host copies: [0, 3 S) initial sums, [3 S, 6 S) final FP64
-    // residual sums, then the striped r.r history (S = SSIZE doubles)
-    rc = pic_ensure_pin(ctx, (6 * SSIZE + hslots) * sizeof(double));
+    // pinned host copies: [0, 3 S) initial sums, 3 final FP64 residual sums
+    // at 3 S, the striped r.r history from 4 S (S = SSIZE doubles)
+    rc = pic_ensure_pin(ctx, (4 * SSIZE + hslots) * sizeof(double));
     if (rc) return rc;
     double* hp = ctx->pin;
-    double* hrr = hp + 6 * SSIZE;
+    double* hrr = hp + 4 * SSIZE;
     PIC_HIP(ctx, hipMemsetAsync(sc, 0, 3 * SSIZE * sizeof(double), ctx->stream));
     k_fcg_resid<<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->phi, ctx->rho, 1.0 / EPS0, r, sc);
     PIC_HIP(ctx, hipMemcpyAsync(hp, sc, 3 * SSIZE * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -1661,11 +1904,8 @@ static int solve_learned(pic_ctx* ctx, const pic_solver_params* p, pic_solver_st
                 // check, saving a second wait
                 const bool expect = prev > 0 && it >= prev && it <= prev + 1;
                 if (expect) {
-                    PIC_HIP(ctx, hipMemsetAsync(sc, 0, 3 * SSIZE * sizeof(double), ctx->stream));
-                    k_resid<<<nb, BLOCK, 0, ctx->stream>>>(s, plain_args(s), ctx->ntype, ctx->phi, ctx->rho, sc);
-                    PIC_HIP(ctx, hipGetLastError());
-                    PIC_HIP(ctx, hipMemcpyAsync(hp + 3 * SSIZE, sc, 3 * SSIZE * sizeof(double),
-                                                hipMemcpyDeviceToHost, ctx->stream));
+                    rc = queue_residual(ctx, s, plain_args(s), hp + 3 * SSIZE);
+                    if (rc) return rc;
                 }
                 PIC_HIP(ctx, pic_spin_wait(ctx->stream));
                 if (!have_b) read_initial();
@@ -1689,7 +1929,7 @@ static int solve_learned(pic_ctx* ctx, const pic_solver_params* p, pic_solver_st
     double rn[3];
     if (conv) {
         if (have_final) {
-            for (int q2 = 0; q2 < 3; q2++) rn[q2] = shost(hp + (3 + q2) * SSIZE);
+            for (int q2 = 0; q2 < 3; q2++) rn[q2] = hp[3 * SSIZE + q2];
         } else {
             rc = residual_norms(ctx, s, plain_args(s), rn);
             if (rc) return rc;
@@ -1762,14 +2002,14 @@ static int solve_newton_learned(pic_ctx* ctx, const pic_solver_params* p, pic_so
     na.phi0 = p->phi0;
     na.n0 = p->n0;
     na.inv_te0 = 1.0 / (p->Te0 != 0 ? p->Te0 : 1.0);
-    unsigned nb = stencil_blocks(s.nn), nbr = stencil_blocks_red(s.nn);
+    unsigned nb = stencil_blocks(s.nn), nbr = stencil_blocks_red(s.nn), nbp = part_blocks(s.nn);
     int total_it = 0, newton = 0;
     bool conv = false, stalled = false;
     for (newton = 0; newton < 20; newton++) {  // NR_MAX_IT, PotentialSolver.cpp:179
-        PIC_HIP(ctx, hipMemsetAsync(ctx->scratch, 0, 4 * sizeof(double), ctx->stream));
-        k_F<double><<<nbr, BLOCK, 0, ctx->stream>>>(s, na, ctx->ntype, ctx->phi, ctx->rho, r, P, ctx->scratch);
+        k_F<double, false, false><<<nbp, BLOCK, 0, ctx->stream>>>(s, na, ctx->ntype, ctx->phi, ctx->rho, r, nullptr,
+                                                                  P, ctx->scratch);
+        k_sum_parts<<<3, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nbp, hf);
         PIC_HIP(ctx, hipGetLastError());
-        PIC_HIP(ctx, hipMemcpyAsync(hf, ctx->scratch, 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         PIC_HIP(ctx, pic_spin_wait(ctx->stream));
         const double bb = hf[2] > 0 ? hf[2] : 1.0;
         const double target2 = p->tol_kind == PIC_TOL_REF_RMS ? p->tol * p->tol * (double)nn
@@ -1824,11 +2064,10 @@ static int solve_newton_learned(pic_ctx* ctx, const pic_solver_params* p, pic_so
             stalled = true;
             break;
         }
-        PIC_HIP(ctx, hipMemsetAsync(ctx->scratch, 0, sizeof(double), ctx->stream));
-        k_update_phi<double><<<nbr, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->phi, y, ctx->scratch);
+        k_update_phi<double><<<nbp, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->phi, y, ctx->scratch + PART_F);
+        k_sum_parts<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nbp, hf + 3);
         PIC_HIP(ctx, hipGetLastError());
         double yy;
-        PIC_HIP(ctx, hipMemcpyAsync(hf + 3, ctx->scratch, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         PIC_HIP(ctx, pic_spin_wait(ctx->stream));
         yy = hf[3];
         if (p->tol_kind == PIC_TOL_REF_RMS && std::sqrt(yy / (double)nn) < 1e-3) {  // :229-233

@@ -1,0 +1,82 @@
+"""The field solvers at the sizes where their kernels can go wrong: grids whose
+node count is not a multiple of four, whose i-lines are shorter than a group
+of four nodes, and grids with more groups of four than threads."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pg():
+    import pic_gpu
+
+    return pic_gpu
+
+
+def _rho(shape, seed):
+    rng = np.random.default_rng(seed)
+    return 1e-9 * rng.normal(size=shape[0] * shape[1] * shape[2])
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (5, 4, 3), (3, 3, 30), (7, 6, 5), (33, 17, 9), (103, 101, 103)])
+@pytest.mark.parametrize("method,tol", [("SOLVER_PCG", 1e-10), ("SOLVER_PCG_MIXED", 1e-8)])
+def test_pcg_residual_by_the_oracle(pg, shape, method, tol):
+    L = [1e-2 * (n - 1) for n in shape]
+    c = pg.Context(*shape, [0, 0, 0], L)
+    c.dirichlet_walls()
+    g = O.make_grid(*shape, [0, 0, 0], L)
+    rho = _rho(shape, shape[0])
+    c.set_field(pg.FIELD_RHO, rho)
+    st = c.poisson(getattr(pg, method), tol=tol, tol_kind=pg.TOL_REL, max_it=5000)
+    assert st["converged"], st
+    r2, b2 = O.residual_dirichlet(g, c.get_field(pg.FIELD_PHI), rho)
+    # the device sums the same rows in another order
+    assert r2 / b2 <= 1.001 * tol
+    c.close()
+
+
+@pytest.mark.parametrize("shape", [(5, 6, 7), (18, 11, 13), (15, 13, 9)])
+@pytest.mark.parametrize("method,tol", [("SOLVER_PCG", 1e-10), ("SOLVER_PCG_MIXED", 1e-8)])
+def test_boltzmann_pcg_matches_oracle(pg, shape, method, tol):
+    """Newton-Boltzmann on odd grids against the oracle's tight solve; J's
+    smallest eigenvalue is at least the walls' pi^2 / L^2 sum and the start
+    residual F is b, so a residual of tol leaves phi well within 1e3 tol."""
+    L = [1e-2 * (n - 1) for n in shape]
+    c = pg.Context(*shape, [0, 0, 0], L)
+    c.dirichlet_walls()
+    g = O.make_grid(*shape, [0, 0, 0], L)
+    rho = np.full(O.nn(g), O.QE * 1.5e12)
+    c.set_field(pg.FIELD_RHO, rho)
+    st = c.poisson(getattr(pg, method), tol=tol, tol_kind=pg.TOL_REL, max_it=5000, n0=1e12, Te0=2.0)
+    assert st["converged"], st
+    _, nt = c.node_flags()
+    tight, ok, *_ = O.nrpcg(g, np.zeros(O.nn(g), np.int32), nt, np.zeros(O.nn(g)), rho, 0.0, 1e12, 2.0, 5000, 1e-12,
+                            axis_swap=False)
+    phi = c.get_field(pg.FIELD_PHI)
+    assert np.max(np.abs(phi - tight)) <= 1e3 * tol * np.max(np.abs(tight))
+    c.close()
+
+
+@pytest.mark.parametrize("shape", [(21, 18, 19), (40, 33, 29)])
+@pytest.mark.parametrize("method,tol", [("SOLVER_PCG", 1e-10), ("SOLVER_PCG_MIXED", 1e-8)])
+def test_boltzmann_pcg_with_neumann_sides_matches_oracle(pg, shape, method, tol):
+    """An electrode plane and open sides: the PCG kernels that keep s = M g
+    (M per row type) against the oracle's Newton-PCG on the same rows."""
+    L = [1e-2 * (n - 1) for n in shape]
+    rho = _rho(shape, 1) + 1.5e12 * O.QE
+    c = pg.Context(*shape, [0, 0, 0], L)
+    c.add_rectangle([L[0] / 2, L[1] / 2, 0], [1.1 * L[0], 1.1 * L[1], 0.15 * L[2]], 3.0)
+    phi0 = c.get_field(pg.FIELD_PHI)
+    oid, nt = c.node_flags()
+    c.set_field(pg.FIELD_RHO, rho)
+    st = c.poisson(getattr(pg, method), tol=tol, tol_kind=pg.TOL_REL, max_it=5000, n0=1e12, Te0=2.0)
+    assert st["converged"], st
+    g = O.make_grid(*shape, [0, 0, 0], L)
+    tight, ok, *_ = O.nrpcg(g, oid, nt, phi0, rho, 0.0, 1e12, 2.0, 5000, 1e-11, axis_swap=False)
+    phi = c.get_field(pg.FIELD_PHI)
+    # the electrons' shift P bounds J's smallest eigenvalue from below
+    assert np.max(np.abs(phi - tight)) <= 1e3 * tol * np.max(np.abs(tight))
+    c.close()
