@@ -53,7 +53,7 @@ ALG_BYTES = {
 ALG_BYTES_FCG = 76.0
 KERNEL_NAMES = {
     "push": "k_push<false,2>", "scatter": "k_push_scatter", "deposit": "k_dep_cells + k_dep_nodes",
-    "pcg": "k_pcg1<float> + k_pcg2<float>", "sor": "k_sor_split (one launch per colour)",
+    "pcg": "k_pcg1<float> + k_pcg2<float>", "sor": "k_sor_tile (two sweeps per launch)",
 }
 
 
@@ -873,7 +873,7 @@ def main():
     if dom == "pcg":
         units = ctx.nn
     elif dom == "sor":
-        units = ctx.nn  # one profiled launch = one full red-black sweep
+        units = 2 * ctx.nn  # one profiled launch = two red-black sweeps
     else:
         units = N
     per_unit = ALG_BYTES[dom]

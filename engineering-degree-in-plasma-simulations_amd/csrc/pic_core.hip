@@ -178,7 +178,8 @@ extern "C" void pic_destroy(pic_ctx* ctx) {
     pic_unet_free(ctx);
     (void)hipFree(ctx->phi);
     (void)hipFree(ctx->phi_prev);
-    (void)hipFree(ctx->sor_split);
+    (void)hipFree(ctx->sor_phi);
+    (void)hipFree(ctx->sor_bits);
     (void)hipFree(ctx->rho);
     (void)hipFree(ctx->ef);
     (void)hipFree(ctx->emax);
@@ -191,7 +192,7 @@ extern "C" void pic_destroy(pic_ctx* ctx) {
     if (ctx->pin) (void)hipHostFree(ctx->pin);
     for (auto e : ctx->solve_ev)
         if (e) (void)hipEventDestroy(e);
-    for (auto e : ctx->pcg_ev)
+    for (auto e : ctx->batch_ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& r : ctx->prof.recs) {
         (void)hipEventDestroy(r.a);

@@ -242,8 +242,8 @@ struct pic_ctx {
     // device fields
     double* phi = nullptr;
     double* phi_prev = nullptr;  // previous solution (PIC_SOLVE_EXTRAPOLATE), allocated on demand
-    void* sor_split = nullptr;  // the SOR sweeps' red-black split phi, rho, node types (on demand)
-    size_t sor_split_bytes = 0;
+    double* sor_phi = nullptr;   // the tiled SOR sweeps' second potential (on demand)
+    uint8_t* sor_bits = nullptr; // and their row bits
     bool phi_prev_valid = false;
     double* rho = nullptr;
     float4* ef = nullptr;
@@ -269,7 +269,7 @@ struct pic_ctx {
     double* pin = nullptr;     // pinned host memory for the solvers' convergence reads
     size_t pin_bytes = 0;
     hipEvent_t solve_ev[2] = {nullptr, nullptr};  // pic_poisson's timing events
-    hipEvent_t pcg_ev[2] = {nullptr, nullptr};    // ends of PCG's queued batches
+    hipEvent_t batch_ev[2] = {nullptr, nullptr};  // ends of the solvers' queued batches
 };
 
 // ---- host helpers shared between translation units ----

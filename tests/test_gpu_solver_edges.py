@@ -80,3 +80,36 @@ def test_boltzmann_pcg_with_neumann_sides_matches_oracle(pg, shape, method, tol)
     # the electrons' shift P bounds J's smallest eigenvalue from below
     assert np.max(np.abs(phi - tight)) <= 1e3 * tol * np.max(np.abs(tight))
     c.close()
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (4, 3, 5), (17, 16, 15), (31, 33, 32), (65, 41, 29), (70, 71, 72),
+                                   (128, 30, 90)])
+@pytest.mark.parametrize("sides", ["walls", "neumann"])
+@pytest.mark.parametrize("n0", [0.0, 1e10])
+def test_tiled_sor_sweeps_equal_plain(pg, shape, sides, n0):
+    """The tiled sweeps against one launch per colour (PIC_SOLVE_SOR_PLAIN),
+    bit for bit, after an odd and an even number of sweeps and with a check
+    in between: grids smaller than a tile, with cores that end inside a node
+    pair, and of each tile's size; objects on faces, edges and inside."""
+    L = [1e-2 * (n - 1) for n in shape]
+    rng = np.random.default_rng(shape[0])
+    rho = 1e-9 * rng.normal(size=shape[0] * shape[1] * shape[2])
+    phi0 = 0.1 * rng.normal(size=rho.size)
+    for max_it, check in ((1, 25), (2, 25), (25, 9)):
+        out = []
+        for flags in (0, pg.SOLVE_SOR_PLAIN):
+            c = pg.Context(*shape, [0, 0, 0], L)
+            if sides == "walls":
+                c.dirichlet_walls()
+            else:
+                c.add_rectangle([L[0] / 2, L[1] / 2, 0], [0.7 * L[0], 1.1 * L[1], 0.3 * L[2]], 3.0)
+                c.add_rectangle([0, 0.6 * L[1], 0.7 * L[2]], [0.6 * L[0], 0.3 * L[1], 0.4 * L[2]], -2.0)
+            c.set_field(pg.FIELD_RHO, rho)
+            c.set_field(pg.FIELD_PHI, phi0)
+            st = c.poisson(pg.SOLVER_SOR_RB, tol=1e-300, tol_kind=pg.TOL_REL, max_it=max_it, omega=1.6,
+                           check_every=check, n0=n0, Te0=2.0, flags=flags)
+            assert st["iterations"] == max_it and not st["converged"]
+            out.append((c.get_field(pg.FIELD_PHI), st["rel_residual"]))
+            c.close()
+        assert np.array_equal(out[0][0], out[1][0], equal_nan=True), max_it
+        assert out[0][1] == pytest.approx(out[1][1], rel=1e-11, nan_ok=True)
