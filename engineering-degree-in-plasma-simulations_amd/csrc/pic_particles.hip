@@ -1849,12 +1849,28 @@ static int sort_partitioned(pic_ctx* ctx, Species& s) {
     return PIC_OK;
 }
 
+// sorted parts of fewer particles are sorted whole: both ways take the same
+// time there (300k neutrals: 1.35..1.48 ms for a run with either), with fewer
+// launches; 40M with 18M births 1.6 ms joined, 4.6 ms sorted whole
+constexpr size_t JOIN_MIN = 1u << 20;
+
 extern "C" int pic_sort(pic_ctx* ctx, int sid) {
     int rc = pic_check_sid(ctx, sid);
     if (rc) return rc;
     Species& s = ctx->sp[sid];
     const GridC& g = ctx->g;
     const size_t n = s.n_upper ? s.n_upper : 1;
+    // Only appended since the last whole sort (DSMC births, emissions): the
+    // two parts are joined, which streams them, where a counting sort would
+    // scatter the appended part over the whole array.
+    if (!s.sorted && s.tail_ok && s.n_upper >= s.bulk_n && s.bulk_n >= JOIN_MIN) {
+        rc = pic_sort_tail(ctx, sid);
+        if (rc) return rc;
+        if (s.two_part) return pic_join_tail(ctx, sid);
+        s.sorted = true;  // nothing appended: the sorted part alone
+        s.scrambled = false;
+        return PIC_OK;
+    }
     if (s.scrambled && n >= PART_MIN) {
         rc = sort_partitioned(ctx, s);
         if (rc) return rc;
