@@ -148,7 +148,7 @@ struct Species {
     int cur = 0;
     void* block[2] = {nullptr, nullptr};
     uint32_t* rank = nullptr;    // rank of each particle inside its cell bucket
-    uint32_t* count = nullptr;   // ncells + 1 buckets (last = removed)
+    uint32_t* count = nullptr;   // ncells + 1 buckets (the last, the removed ones', stays 0)
     uint32_t* off = nullptr;     // ncells + 2 exclusive offsets
     uint32_t* d_n = nullptr;     // [0] live count, [1] count the histogram covers, [2] overflow
     size_t n_upper = 0;          // host upper bound of the live count

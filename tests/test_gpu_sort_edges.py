@@ -100,3 +100,38 @@ def test_count_leaves_out_removed_particles(pg):
         c.sort(sid)
         assert c.count(sid) == live
         c.close()
+
+
+@pytest.mark.parametrize("dt", [1e-10, 3e-8, 1e-6])  # none, most and all of them leave the box
+@pytest.mark.parametrize("num", [1, 64, 1000, 130_001])
+def test_removed_particles_take_no_place_in_the_sort(pg, dt, num):
+    n, dx = (9, 10, 11), 1e-2
+    L = dx * (np.array(n) - 1)
+    rng = np.random.default_rng(num)
+    p = np.zeros((num, 7))
+    p[:, :3] = rng.uniform(0.1, 0.9, (num, 3)) * L
+    p[:, 3:6] = rng.normal(0, 1e6, (num, 3))
+    p[:, 6] = np.arange(num) + 1.0
+    out = []
+    for fused in (True, False):
+        c = pg.Context(*n, [0, 0, 0], L)
+        sid = c.species_add(ME, 0.0, 1.0, num)
+        c.upload(sid, p)
+        c.sort(sid)
+        if fused:
+            c.push_sort(sid, dt)
+        else:
+            c.push(sid, dt)
+            c.sort(sid)
+        q = c.download(sid)
+        macro = c.species_field(sid, pg.SFIELD_MACRO_COUNT)
+        assert c.count(sid) == q.size // 7 == int(macro.sum())
+        if q.size:
+            cells = _cells(q, dx, n)
+            assert np.all(np.diff(cells) >= 0)
+            assert np.array_equal(macro, np.bincount(cells, minlength=macro.size))
+        out.append(_rows(q))
+        c.close()
+    assert np.array_equal(out[0], out[1])
+    x = p[:, :3] + dt * p[:, 3:6]
+    assert abs(len(out[0]) - np.sum(np.all((x > 0) & (x < L), axis=1))) <= 2 + num // 10000
