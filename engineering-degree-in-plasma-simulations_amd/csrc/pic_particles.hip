@@ -1435,10 +1435,10 @@ __global__ void __launch_bounds__(BLOCK)
 }
 
 // Variable-weight merge (Species::merge, Species.cpp:987-1145) on the
-// cell-sorted arrays, one workgroup per cell of at least 10 particles
+// cell-sorted arrays, for every cell of at least 10 particles
 // (:1029): the cell's velocity range widened by 0.1% at the maximum
 // (:1043-1057) is split into 15 bins per axis (Species.h:129, :1059-1067);
-// the workgroup sorts (bin, place in the cell) keys in LDS (bitonic), and
+// a wave or a workgroup sorts (bin, place in the cell) keys (bitonic), and
 // one thread per bin of more than two particles sums weight, momentum and
 // per-axis energy in cell order in FP64, and writes the pair
 // v = mean +- sqrt(variance) (a negative variance clamped to 0), half the
@@ -1454,180 +1454,270 @@ struct MergeArgs {
     uint32_t seed, call;
     double rewind;  // (q/m) * 0.5 dt, 0 for neutrals
 };
-__global__ void __launch_bounds__(MERGE_BLOCK)
-    k_merge(GridC g, SpeciesBuf b, const uint32_t* __restrict__ off, const float4* __restrict__ E,
-            MergeArgs a, unsigned long long* __restrict__ stats) {
-    __shared__ uint32_t key[MERGE_MAX];
-    __shared__ double red[6][MERGE_BLOCK / 64];
-    const int c = blockIdx.x;
-    const int tid = threadIdx.x;
-    const uint32_t p0 = off[c], p1 = off[c + 1];
-    const int n = (int)(p1 - p0);
-    if (n < 10) return;
-    if (n > MERGE_MAX) {
-        if (tid == 0) atomicAdd(&stats[2], 1ull);
-        return;
-    }
-    // velocity range of the cell (exact min and max)
-    double mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int q = tid; q < n; q += MERGE_BLOCK)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const double v = (double)b.v[d][p0 + q];
-            mn[d] = fmin(mn[d], v);
-            mx[d] = fmax(mx[d], v);
-        }
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-        for (int o = 32; o > 0; o >>= 1) {
-            mn[d] = fmin(mn[d], __shfl_xor(mn[d], o, 64));
-            mx[d] = fmax(mx[d], __shfl_xor(mx[d], o, 64));
-        }
-    if ((tid & 63) == 0)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            red[d][tid >> 6] = mn[d];
-            red[3 + d][tid >> 6] = mx[d];
-        }
-    __syncthreads();
-    double vmin[3], dv[3];
+constexpr uint32_t MERGE_MASK = (1u << MERGE_IDX_BITS) - 1u;
+
+// the widened velocity range of an axis: its lower end and bin width
+__device__ inline void merge_range(double lo, double hi, double& vmin, double& dv) {
+    if (hi > 0)
+        hi *= 1.001;
+    else
+        hi *= 0.999;
+    vmin = lo;
+    dv = (hi - lo) / (double)MERGE_BINS;
+}
+__device__ inline uint32_t merge_key(const float (&v)[3], const double (&vmin)[3], const double (&dv)[3], uint32_t q) {
+    int bi[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        double lo = red[d][0], hi = red[3 + d][0];
-        for (int w = 1; w < MERGE_BLOCK / 64; w++) {
-            lo = fmin(lo, red[d][w]);
-            hi = fmax(hi, red[3 + d][w]);
-        }
-        if (hi > 0)
-            hi *= 1.001;
-        else
-            hi *= 0.999;
-        vmin[d] = lo;
-        dv[d] = (hi - lo) / (double)MERGE_BINS;
+        const double x = ((double)v[d] - vmin[d]) / dv[d];
+        int t = x == x ? (x < (double)MERGE_BINS ? (int)x : MERGE_BINS - 1) : 0;
+        bi[d] = t < 0 ? 0 : t;
     }
-    // keys: bin << 13 | place; padded to a power of two
-    int npad = 16;
-    while (npad < n) npad <<= 1;
-    for (int q = tid; q < npad; q += MERGE_BLOCK) {
-        uint32_t k = 0xFFFFFFFFu;
-        if (q < n) {
-            int bi[3];
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const double x = ((double)b.v[d][p0 + q] - vmin[d]) / dv[d];
-                int t = x == x ? (x < (double)MERGE_BINS ? (int)x : MERGE_BINS - 1) : 0;
-                bi[d] = t < 0 ? 0 : t;
-            }
-            const uint32_t bin = (uint32_t)((bi[0] * MERGE_BINS + bi[1]) * MERGE_BINS + bi[2]);
-            k = (bin << MERGE_IDX_BITS) | (uint32_t)q;
-        }
-        key[q] = k;
-    }
-    __syncthreads();
-    for (int k = 2; k <= npad; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = tid; i < npad; i += MERGE_BLOCK) {
-                const int ixj = i ^ j;
-                if (ixj > i) {
-                    const uint32_t x = key[i], y = key[ixj];
-                    if ((x > y) == ((i & k) == 0)) {
-                        key[i] = y;
-                        key[ixj] = x;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    constexpr uint32_t MASK = (1u << MERGE_IDX_BITS) - 1u;
-    unsigned long long nbins = 0, nin = 0;
-    for (int s0 = tid; s0 < n; s0 += MERGE_BLOCK) {
-        const uint32_t bin = key[s0] >> MERGE_IDX_BITS;
-        if (s0 > 0 && (key[s0 - 1] >> MERGE_IDX_BITS) == bin) continue;  // not a bin's first
-        int e = s0 + 1;
-        while (e < n && (key[e] >> MERGE_IDX_BITS) == bin) e++;
-        const int len = e - s0;
-        if (len <= 2) continue;
-        nbins++;
-        nin += (unsigned long long)len;
-        double tw = 0, tm[3] = {0, 0, 0}, te[3] = {0, 0, 0};
-        for (int q = s0; q < e; q++) {
-            const uint32_t idx = p0 + (key[q] & MASK);
-            const double w = (double)b.w[idx];
-            tw += w;
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const double v = (double)b.v[d][idx];
-                tm[d] += v * w;
-                te[d] += (v * v) * w;
-            }
-        }
-        const double wh = tw * 0.5, inv = 1.0 / tw;
-        double va[3], vb[3];
+    const uint32_t bin = (uint32_t)((bi[0] * MERGE_BINS + bi[1]) * MERGE_BINS + bi[2]);
+    return (bin << MERGE_IDX_BITS) | q;
+}
+// one bin's members key[s0 .. s0 + len) of the cell's particles from p0 on
+__device__ inline void merge_bin(const GridC& g, const SpeciesBuf& b, const float4* __restrict__ E, const MergeArgs& a,
+                                 int c, uint32_t p0, const uint32_t* key, int s0, int len) {
+    const int e = s0 + len;
+    const uint32_t bin = key[s0] >> MERGE_IDX_BITS;
+    double tw = 0, tm[3] = {0, 0, 0}, te[3] = {0, 0, 0};
+    for (int q = s0; q < e; q++) {
+        const uint32_t idx = p0 + (key[q] & MERGE_MASK);
+        const double w = (double)b.w[idx];
+        tw += w;
 #pragma unroll
         for (int d = 0; d < 3; d++) {
-            tm[d] *= inv;
-            te[d] *= inv;
-            te[d] -= tm[d] * tm[d];
-            if (te[d] < 0) te[d] = 0;
-            const double sq = sqrt(te[d]);
-            va[d] = tm[d] + sq;
-            vb[d] = tm[d] - sq;
-        }
-        Draws dr;
-        dr.init((uint32_t)c, bin, a.seed, a.call, TAG_MERGE);
-        int slot = 0;
-        const int ia = (int)(dr(slot++) * (double)len);
-        int ib = (int)(dr(slot++) * (double)len);
-        while (ib == ia) ib = (int)(dr(slot++) * (double)len);
-        const uint32_t xa = p0 + (key[s0 + ia] & MASK), xb = p0 + (key[s0 + ib] & MASK);
-        const uint32_t ca = b.cell[xa], cb = b.cell[xb];
-        float fa[3], fb[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            fa[d] = b.f[d][xa];
-            fb[d] = b.f[d][xb];
-        }
-        if (a.rewind != 0.0) {
-            int i, j, k;
-            unpack_cell(ca, i, j, k);
-            const float3 ea = gather_e(g, E, i, j, k, fa[0], fa[1], fa[2]);
-            unpack_cell(cb, i, j, k);
-            const float3 eb = gather_e(g, E, i, j, k, fb[0], fb[1], fb[2]);
-            va[0] -= (double)ea.x * a.rewind;
-            va[1] -= (double)ea.y * a.rewind;
-            va[2] -= (double)ea.z * a.rewind;
-            vb[0] -= (double)eb.x * a.rewind;
-            vb[1] -= (double)eb.y * a.rewind;
-            vb[2] -= (double)eb.z * a.rewind;
-        }
-        const uint32_t da = p0 + (key[s0] & MASK), db = p0 + (key[s0 + 1] & MASK);
-        b.cell[da] = ca;
-        b.cell[db] = cb;
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            b.f[d][da] = fa[d];
-            b.f[d][db] = fb[d];
-            b.v[d][da] = (float)va[d];
-            b.v[d][db] = (float)vb[d];
-        }
-        b.w[da] = (float)wh;
-        b.w[db] = (float)wh;
-        for (int q = s0 + 2; q < e; q++) {
-            const uint32_t idx = p0 + (key[q] & MASK);
-            b.cell[idx] = DEAD;
-            b.w[idx] = 0.0f;
+            const double v = (double)b.v[d][idx];
+            tm[d] += v * w;
+            te[d] += (v * v) * w;
         }
     }
+    const double wh = tw * 0.5, inv = 1.0 / tw;
+    double va[3], vb[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        tm[d] *= inv;
+        te[d] *= inv;
+        te[d] -= tm[d] * tm[d];
+        if (te[d] < 0) te[d] = 0;
+        const double sq = sqrt(te[d]);
+        va[d] = tm[d] + sq;
+        vb[d] = tm[d] - sq;
+    }
+    Draws dr;
+    dr.init((uint32_t)c, bin, a.seed, a.call, TAG_MERGE);
+    int slot = 0;
+    const int ia = (int)(dr(slot++) * (double)len);
+    int ib = (int)(dr(slot++) * (double)len);
+    while (ib == ia) ib = (int)(dr(slot++) * (double)len);
+    const uint32_t xa = p0 + (key[s0 + ia] & MERGE_MASK), xb = p0 + (key[s0 + ib] & MERGE_MASK);
+    const uint32_t ca = b.cell[xa], cb = b.cell[xb];
+    float fa[3], fb[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        fa[d] = b.f[d][xa];
+        fb[d] = b.f[d][xb];
+    }
+    if (a.rewind != 0.0) {
+        int i, j, k;
+        unpack_cell(ca, i, j, k);
+        const float3 ea = gather_e(g, E, i, j, k, fa[0], fa[1], fa[2]);
+        unpack_cell(cb, i, j, k);
+        const float3 eb = gather_e(g, E, i, j, k, fb[0], fb[1], fb[2]);
+        va[0] -= (double)ea.x * a.rewind;
+        va[1] -= (double)ea.y * a.rewind;
+        va[2] -= (double)ea.z * a.rewind;
+        vb[0] -= (double)eb.x * a.rewind;
+        vb[1] -= (double)eb.y * a.rewind;
+        vb[2] -= (double)eb.z * a.rewind;
+    }
+    const uint32_t da = p0 + (key[s0] & MERGE_MASK), db = p0 + (key[s0 + 1] & MERGE_MASK);
+    b.cell[da] = ca;
+    b.cell[db] = cb;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        b.f[d][da] = fa[d];
+        b.f[d][db] = fb[d];
+        b.v[d][da] = (float)va[d];
+        b.v[d][db] = (float)vb[d];
+    }
+    b.w[da] = (float)wh;
+    b.w[db] = (float)wh;
+    for (int q = s0 + 2; q < e; q++) {
+        const uint32_t idx = p0 + (key[q] & MERGE_MASK);
+        b.cell[idx] = DEAD;
+        b.w[idx] = 0.0f;
+    }
+}
+// a workgroup's merged bins and their members added to the counters
+__device__ inline void merge_stats(unsigned long long nbins, unsigned long long nin, unsigned long long* stats) {
     for (int o = 32; o > 0; o >>= 1) {
         nbins += __shfl_xor(nbins, o, 64);
         nin += __shfl_xor(nin, o, 64);
     }
-    if ((tid & 63) == 0 && nbins) {
+    if ((threadIdx.x & 63) == 0 && nbins) {
         atomicAdd(&stats[0], nbins);
         atomicAdd(&stats[1], nin);
     }
 }
 
+// Cells of up to 64 particles, a wave each: keys sorted across the wave's
+// lanes, no LDS but for the sorted keys.  The waves walk the cells and add
+// their counts once at the end.  (A workgroup per cell with its 32 KB of keys,
+// and two atomics per wave on the same two words, took 1.5 ms for 131k cells of
+// about 15 particles.)
+constexpr int MERGE_SMALL = 64;
+__global__ void __launch_bounds__(MERGE_BLOCK)
+    k_merge_small(GridC g, SpeciesBuf b, const uint32_t* __restrict__ off, const float4* __restrict__ E, MergeArgs a,
+                  unsigned long long* __restrict__ stats) {
+    constexpr int WAVES = MERGE_BLOCK / 64;
+    __shared__ uint32_t keys[WAVES][MERGE_SMALL];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t* key = keys[wave];
+    unsigned long long nbins = 0, nin = 0;
+    for (int cb = blockIdx.x * WAVES; cb < g.ncells; cb += gridDim.x * WAVES) {
+        const int c = cb + wave;
+        uint32_t p0 = 0;
+        int n = 0;
+        if (c < g.ncells) {
+            p0 = off[c];
+            n = (int)(off[c + 1] - p0);
+        }
+        if (n < 10 || n > MERGE_SMALL) n = 0;
+        float v[3] = {0.f, 0.f, 0.f}, mn[3], mx[3];
+        const bool in = lane < n;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            if (in) v[d] = b.v[d][p0 + lane];
+            mn[d] = in ? v[d] : INFINITY;
+            mx[d] = in ? v[d] : -INFINITY;
+            for (int o = 32; o > 0; o >>= 1) {
+                mn[d] = fminf(mn[d], __shfl_xor(mn[d], o, 64));
+                mx[d] = fmaxf(mx[d], __shfl_xor(mx[d], o, 64));
+            }
+        }
+        uint32_t k = 0xFFFFFFFFu;
+        if (in) {
+            double vmin[3], dv[3];
+#pragma unroll
+            for (int d = 0; d < 3; d++) merge_range((double)mn[d], (double)mx[d], vmin[d], dv[d]);
+            k = merge_key(v, vmin, dv, (uint32_t)lane);
+        }
+#pragma unroll
+        for (int s = 2; s <= 64; s <<= 1)
+#pragma unroll
+            for (int j = s >> 1; j > 0; j >>= 1) {
+                const uint32_t o = __shfl_xor(k, j, 64);
+                const bool up = (lane & s) == 0, low = (lane & j) == 0;
+                k = (up == low) ? min(k, o) : max(k, o);
+            }
+        const uint32_t bin = k >> MERGE_IDX_BITS;
+        const uint32_t prev = __shfl_up(bin, 1, 64);
+        const bool head = in && (lane == 0 || prev != bin);
+        const unsigned long long heads = __ballot(head);
+        const unsigned long long above = lane == 63 ? 0ull : heads >> (lane + 1);
+        const int len = (above ? lane + __ffsll(above) : n) - lane;  // (head lanes)
+        key[lane] = k;
+        __syncthreads();
+        if (head && len > 2) {
+            nbins++;
+            nin += (unsigned long long)len;
+            merge_bin(g, b, E, a, c, p0, key, lane, len);
+        }
+        __syncthreads();
+    }
+    merge_stats(nbins, nin, stats);
+}
+
+// larger cells, a workgroup each
+__global__ void __launch_bounds__(MERGE_BLOCK)
+    k_merge(GridC g, SpeciesBuf b, const uint32_t* __restrict__ off, const float4* __restrict__ E,
+            MergeArgs a, unsigned long long* __restrict__ stats) {
+    __shared__ uint32_t key[MERGE_MAX];
+    __shared__ float red[6][MERGE_BLOCK / 64];
+    const int tid = threadIdx.x;
+    unsigned long long nbins = 0, nin = 0;
+    for (int c = blockIdx.x; c < g.ncells; c += gridDim.x) {
+        const uint32_t p0 = off[c], p1 = off[c + 1];
+        const int n = (int)(p1 - p0);
+        if (n <= MERGE_SMALL) continue;  // (the whole workgroup)
+        if (n > MERGE_MAX) {
+            if (tid == 0) atomicAdd(&stats[2], 1ull);
+            continue;
+        }
+        // velocity range of the cell (exact min and max)
+        float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+        for (int q = tid; q < n; q += MERGE_BLOCK)
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const float v = b.v[d][p0 + q];
+                mn[d] = fminf(mn[d], v);
+                mx[d] = fmaxf(mx[d], v);
+            }
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            for (int o = 32; o > 0; o >>= 1) {
+                mn[d] = fminf(mn[d], __shfl_xor(mn[d], o, 64));
+                mx[d] = fmaxf(mx[d], __shfl_xor(mx[d], o, 64));
+            }
+        __syncthreads();  // the previous cell's keys and range are consumed
+        if ((tid & 63) == 0)
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                red[d][tid >> 6] = mn[d];
+                red[3 + d][tid >> 6] = mx[d];
+            }
+        __syncthreads();
+        double vmin[3], dv[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            float lo = red[d][0], hi = red[3 + d][0];
+            for (int w = 1; w < MERGE_BLOCK / 64; w++) {
+                lo = fminf(lo, red[d][w]);
+                hi = fmaxf(hi, red[3 + d][w]);
+            }
+            merge_range((double)lo, (double)hi, vmin[d], dv[d]);
+        }
+        // keys: bin << 13 | place; padded to a power of two
+        int npad = 128;
+        while (npad < n) npad <<= 1;
+        for (int q = tid; q < npad; q += MERGE_BLOCK) {
+            uint32_t k = 0xFFFFFFFFu;
+            if (q < n) {
+                const float v[3] = {b.v[0][p0 + q], b.v[1][p0 + q], b.v[2][p0 + q]};
+                k = merge_key(v, vmin, dv, (uint32_t)q);
+            }
+            key[q] = k;
+        }
+        __syncthreads();
+        for (int k = 2; k <= npad; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int i = tid; i < npad; i += MERGE_BLOCK) {
+                    const int ixj = i ^ j;
+                    if (ixj > i) {
+                        const uint32_t x = key[i], y = key[ixj];
+                        if ((x > y) == ((i & k) == 0)) {
+                            key[i] = y;
+                            key[ixj] = x;
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+        for (int s0 = tid; s0 < n; s0 += MERGE_BLOCK) {
+            const uint32_t bin = key[s0] >> MERGE_IDX_BITS;
+            if (s0 > 0 && (key[s0 - 1] >> MERGE_IDX_BITS) == bin) continue;  // not a bin's first
+            int e = s0 + 1;
+            while (e < n && (key[e] >> MERGE_IDX_BITS) == bin) e++;
+            if (e - s0 <= 2) continue;
+            nbins++;
+            nin += (unsigned long long)(e - s0);
+            merge_bin(g, b, E, a, c, p0, key, s0, e - s0);
+        }
+    }
+    merge_stats(nbins, nin, stats);
+}
 }  // namespace
 
 // ------------------------------------------------------------------------
@@ -2179,7 +2269,10 @@ extern "C" int pic_merge(pic_ctx* ctx, int sid, uint32_t seed, pic_merge_stats* 
     a.seed = seed;
     a.call = s.merge_calls++;
     a.rewind = s.charge != 0.0 ? s.charge / s.mass * (0.5 * ctx->dt) : 0.0;
-    k_merge<<<(unsigned)g.ncells, MERGE_BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], s.off, ctx->ef, a, d);
+    k_merge_small<<<std::min<unsigned>(grid_for((size_t)g.ncells, MERGE_BLOCK / 64), 2048), MERGE_BLOCK, 0,
+                    ctx->stream>>>(g, s.buf[s.cur], s.off, ctx->ef, a, d);
+    k_merge<<<std::min<unsigned>((unsigned)g.ncells, 1024), MERGE_BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], s.off,
+                                                                                         ctx->ef, a, d);
     PIC_HIP(ctx, hipGetLastError());
     s.sorted = false;  // removed members leave at the compaction below
     s.hist_valid = false;
