@@ -275,6 +275,7 @@ extern "C" int pic_dsmc_apply(pic_ctx* ctx, int id, double dt, uint32_t seed, ui
     a.one = D.s1 == D.s2;
     PIC_HIP(ctx, hipMemsetAsync(D.d_part, 0, (size_t)NSTRIPE * SSTRIDE * sizeof(unsigned long long),
                                 ctx->stream));
+    A.safe_ok = B.safe_ok = false;
     {
         PicProfScope ps(ctx, PIC_K_MCC);
         k_dsmc<<<grid_for((size_t)g.ncells, BLOCK), BLOCK, 0, ctx->stream>>>(g, a, A.buf[A.cur], A.off,
@@ -366,6 +367,7 @@ extern "C" int pic_source_sample(pic_ctx* ctx, int id, uint32_t seed, size_t* n_
     a.seed = seed;
     a.call = call;
     a.w = (float)sp.mpw0;
+    sp.safe_ok = false;
     {
         PicProfScope ps(ctx, PIC_K_LOAD);
         k_source<<<grid_for((size_t)num_macro, 256), 256, 0, ctx->stream>>>(g, sp.buf[sp.cur], ctx->ef, a, base,

@@ -403,8 +403,14 @@ extern "C" int pic_species_add(pic_ctx* ctx, double mass, double charge, double 
         }
         s.buf[b].w = (float*)(base + 7 * stride);
     }
-    // ranks; pic_push_sort keeps 64 run bases per group of 64 particles here
-    if (e == hipSuccess) e = hipMalloc(&s.rank, (c + 63) / 64 * 64 * 4);
+    // ranks (pic_push_sort keeps 64 run bases per group of 64 particles here),
+    // pic_push_sort's flags and their bound in one block
+    const size_t rank_bytes = (c + 63) / 64 * 64 * 4, safe_bytes = (c + 255) / 256 * 256;
+    if (e == hipSuccess) e = hipMalloc(&s.rank, rank_bytes + safe_bytes + 4 * sizeof(float));
+    if (e == hipSuccess) {
+        s.safe = reinterpret_cast<uint8_t*>(s.rank) + rank_bytes;
+        s.safe_kick = reinterpret_cast<float*>(s.safe + safe_bytes);
+    }
     if (e == hipSuccess) e = hipMalloc(&s.count, ((size_t)g.ncells + 2) * 4);
     if (e == hipSuccess) e = hipMalloc(&s.off, ((size_t)g.ncells + 2) * 4);
     if (e == hipSuccess) e = hipMalloc(&s.d_n, 4 * sizeof(uint32_t));
@@ -522,6 +528,7 @@ extern "C" int pic_particles_upload(pic_ctx* ctx, int sid, const double* aos7, s
     PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     s.n_upper = n;
     s.hist_valid = false;
+    s.safe_ok = false;
     s.sorted = false;
     s.two_part = false;
     s.tail_ok = false;

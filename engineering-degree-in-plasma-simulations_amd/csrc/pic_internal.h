@@ -170,6 +170,15 @@ struct Species {
     // particles in random order (a load or an upload): the next sort
     // partitions them by coarse bucket first
     bool scrambled = false;
+    // pic_push_sort's flags for the next one: a byte per particle, 1 for
+    // those that cannot leave their cell under kicks of at most safe_kick and
+    // drifts of at most safe_dtx cells per m/s.  They describe the arrays as
+    // that call left them: every call that moves, reorders, adds or changes
+    // particles clears safe_ok.
+    uint8_t* safe = nullptr;     // (in rank's block)
+    float* safe_kick = nullptr;  // device, 3 floats
+    bool safe_ok = false;
+    float safe_dtx[3] = {0.f, 0.f, 0.f};
     double* den = nullptr;       // number density
     double* mom = nullptr;       // n, nvx, nvy, nvz, nuu, nvv, nww (7 * nn)
     uint32_t seq = 0;            // loader stream id

@@ -588,6 +588,7 @@ extern "C" int pic_mcc_apply(pic_ctx* ctx, int id, double dt, uint32_t seed, uin
     if (!ctx || id < 0 || id >= (int)ctx->mcc.size()) return PIC_ERR_ARG;
     Mcc& m = ctx->mcc[id];
     Species &N = ctx->sp[m.sn], &I = ctx->sp[m.si], &E = ctx->sp[m.se];
+    N.safe_ok = I.safe_ok = E.safe_ok = false;
     int rc = 0;
     // the neutrals (they move once per many steps): the births appended
     // since their last whole sort are indexed by cell, and joined with the

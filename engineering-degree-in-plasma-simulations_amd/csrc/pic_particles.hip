@@ -416,12 +416,23 @@ __device__ inline uint32_t cell_key(const GridC& g, uint32_t c) {
 // of all its particles (cell word, offsets, velocities: no load waits on the
 // cell word) before it waits for any, so twice the bytes are in flight.
 constexpr int PUSH_ILP = 2;
-// the histogram pass of pic_push_sort (4 per thread measured slower)
+// the histogram pass of pic_push_sort (200M ions: 1 per thread 833 us, 2 609, 4
+// 606, 8 715; 20M electrons: 176, 158, 161, 182)
 constexpr int PUSH_SORT_ILP = 2;
+//
+// safe (histogram pass; may be null): a byte per particle, set by the
+// k_push_scatter that ordered them, for those that cannot leave their cell
+// under a kick of safe_kick.  While the largest kick is within that, such a
+// particle's key is its cell word: nothing else of it is read (5 bytes
+// instead of 28).  20M particles at 128^3, without and with: ions, which hardly
+// move, 134 and 60 us (then the runs' atomics bound it), electrons, a few per
+// cent of which may leave, 170 and 158; writing the byte costs
+// k_push_scatter 10 of 289 us.  200M ions at 256^3: 1245 and 609 us.
 template <bool WRITE, int ILP, bool SURF>
 __global__ void __launch_bounds__(BLOCK)
     k_push(GridC g, SpeciesBuf b, const float4* __restrict__ E, PushArgs a,
-           uint32_t* __restrict__ d_n, uint32_t* __restrict__ count, uint32_t* __restrict__ rank) {
+           uint32_t* __restrict__ d_n, uint32_t* __restrict__ count, uint32_t* __restrict__ rank,
+           const uint8_t* __restrict__ safe, const float* __restrict__ safe_kick) {
     const size_t p0 = xcd_wg() * (BLOCK * ILP) + threadIdx.x;
     uint32_t n = d_n[0];
     uint32_t covered = gridDim.x * BLOCK * ILP;
@@ -435,12 +446,23 @@ __global__ void __launch_bounds__(BLOCK)
     if (bound && a.kick)
 #pragma unroll
         for (int d = 0; d < 3; d++) kick[d] = fabsf(a.qmdt) * a.emax[d];
+    const bool use_safe = bound && safe != nullptr && kick[0] <= safe_kick[0] && kick[1] <= safe_kick[1] &&
+                          kick[2] <= safe_kick[2];  // (the whole grid; false for NaN)
+    uint8_t stay[ILP];
 #pragma unroll
     for (int q = 0; q < ILP; q++) {
         const size_t p = p0 + (size_t)q * BLOCK;
         c[q] = DEAD;
+        stay[q] = 0;
         if (p < n) {
             c[q] = b.cell[p];
+            if (use_safe) stay[q] = safe[p];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < ILP; q++) {
+        const size_t p = p0 + (size_t)q * BLOCK;
+        if (p < n && !stay[q]) {
 #pragma unroll
             for (int d = 0; d < 3; d++) {
                 f[q][d] = b.f[d][p];
@@ -456,7 +478,7 @@ __global__ void __launch_bounds__(BLOCK)
         if (valid) {
             key = (uint32_t)g.ncells;
             if (c[q] != DEAD) {
-                const uint32_t nc = (bound && stays_in_cell(f[q], v[q], kick, a.dtx))
+                const uint32_t nc = (stay[q] || (bound && stays_in_cell(f[q], v[q], kick, a.dtx)))
                                         ? c[q]
                                         : advance<SURF>(g, E, a, c[q], f[q], v[q], b, p);
                 key = cell_key(g, nc);
@@ -1003,8 +1025,17 @@ template <bool SURF, int ILP>
 __global__ void __launch_bounds__(BLOCK)
     k_push_scatter(GridC g, SpeciesBuf src, SpeciesBuf dst, const float4* __restrict__ E, PushArgs a,
                    const uint32_t* __restrict__ bases, const uint32_t* __restrict__ off,
-                   const uint32_t* __restrict__ d_n, uint32_t cap) {
+                   const uint32_t* __restrict__ d_n, uint32_t cap, uint8_t* __restrict__ safe,
+                   float* __restrict__ safe_kick) {
     const size_t p0 = xcd_wg() * (BLOCK * ILP) + threadIdx.x;
+    // the next push's flags, for a field that at most doubles (see k_push)
+    float kick2[3] = {0.f, 0.f, 0.f};
+    if (!SURF && safe) {
+        if (a.kick)
+#pragma unroll
+            for (int d = 0; d < 3; d++) kick2[d] = 2.f * fabsf(a.qmdt) * a.emax[d];
+        if (p0 < 3) safe_kick[p0] = p0 == 0 ? kick2[0] : p0 == 1 ? kick2[1] : kick2[2];
+    }
     const uint32_t n = d_n[1];
     uint32_t c[ILP];
     float f[ILP][3], v[ILP][3], w[ILP];
@@ -1051,6 +1082,7 @@ __global__ void __launch_bounds__(BLOCK)
             dst.v[d][dst_i] = v[q][d];
         }
         dst.w[dst_i] = w[q];
+        if (!SURF && safe) safe[dst_i] = stays_in_cell(f[q], v[q], kick2, a.dtx) ? 1 : 0;
     }
 }
 
@@ -1754,6 +1786,7 @@ static PushArgs push_args(pic_ctx* ctx, Species& s, double dt) {
 static int after_emission(pic_ctx* ctx, const Species& s, const PushArgs& a) {
     if (a.s.mode != PIC_SURF_RECYCLE) return PIC_OK;
     Species& t = ctx->sp[s.surf_target];
+    t.safe_ok = false;
     uint32_t hn[4];
     PIC_HIP(ctx, hipMemcpyAsync(hn, t.d_n, sizeof(hn), hipMemcpyDeviceToHost, ctx->stream));
     PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1799,6 +1832,7 @@ extern "C" int pic_push(pic_ctx* ctx, int sid, double dt) {
     const GridC& g = ctx->g;
     PushArgs a = push_args(ctx, s, dt);
     a.s.emit = 1;
+    s.safe_ok = false;
     PIC_HIP(ctx, hipMemsetAsync(s.count, 0, ((size_t)g.ncells + 1) * 4, ctx->stream));
     {
         PicProfScope ps(ctx, PIC_K_PUSH);
@@ -1806,10 +1840,10 @@ extern "C" int pic_push(pic_ctx* ctx, int sid, double dt) {
         const unsigned nb = xcd_blocks1(n, BLOCK * PUSH_ILP);
         if (a.s.mode == PIC_SURF_ABSORB)
             k_push<true, PUSH_ILP, false><<<nb, BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], ctx->ef, a, s.d_n,
-                                                                         s.count, s.rank);
+                                                                         s.count, s.rank, nullptr, nullptr);
         else
             k_push<true, PUSH_ILP, true><<<nb, BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], ctx->ef, a, s.d_n,
-                                                                        s.count, s.rank);
+                                                                        s.count, s.rank, nullptr, nullptr);
     }
     PIC_HIP(ctx, hipGetLastError());
     s.hist_valid = true;
@@ -1953,6 +1987,7 @@ extern "C" int pic_sort(pic_ctx* ctx, int sid) {
     Species& s = ctx->sp[sid];
     const GridC& g = ctx->g;
     const size_t n = s.n_upper ? s.n_upper : 1;
+    s.safe_ok = false;
     // Only appended since the last whole sort (DSMC births, emissions): the
     // two parts are joined, which streams them, where a counting sort would
     // scatter the appended part over the whole array.
@@ -2050,6 +2085,7 @@ int pic_join_tail(pic_ctx* ctx, int sid) {
     Species& s = ctx->sp[sid];
     const GridC& g = ctx->g;
     if (!s.two_part) return pic_fail(ctx, PIC_ERR_STATE, "no indexed appended part to join");
+    s.safe_ok = false;
     const size_t nb = s.bulk_n, nt = s.n_upper - s.bulk_n;
     {
         PicProfScope ps(ctx, PIC_K_SCATTER);
@@ -2091,16 +2127,23 @@ extern "C" int pic_push_sort(pic_ctx* ctx, int sid, double dt) {
     }
     PushArgs a = push_args(ctx, s, dt);  // emission in the second pass only
     const size_t n = s.n_upper ? s.n_upper : 1;
+    // the flags of the last pic_push_sort, if nothing has touched the
+    // particles since and the drift per velocity is no larger; the kick's
+    // bound is checked on the device
+    const bool flags = a.emax != nullptr && a.s.mode == PIC_SURF_ABSORB;  // this push leaves flags
+    bool safe = flags && s.safe_ok;
+    for (int d = 0; d < 3; d++) safe = safe && fabsf(a.dtx[d]) <= s.safe_dtx[d];
+    s.safe_ok = false;
     PIC_HIP(ctx, hipMemsetAsync(s.count, 0, ((size_t)g.ncells + 1) * 4, ctx->stream));
     {
         PicProfScope ps(ctx, PIC_K_PUSH);
         const unsigned nb = xcd_blocks1(n, BLOCK * PUSH_SORT_ILP);
         if (a.s.mode == PIC_SURF_ABSORB)
-            k_push<false, PUSH_SORT_ILP, false><<<nb, BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], ctx->ef, a,
-                                                                               s.d_n, s.count, s.rank);
+            k_push<false, PUSH_SORT_ILP, false><<<nb, BLOCK, 0, ctx->stream>>>(
+                g, s.buf[s.cur], ctx->ef, a, s.d_n, s.count, s.rank, safe ? s.safe : nullptr, s.safe_kick);
         else
-            k_push<false, PUSH_SORT_ILP, true><<<nb, BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], ctx->ef, a,
-                                                                              s.d_n, s.count, s.rank);
+            k_push<false, PUSH_SORT_ILP, true><<<nb, BLOCK, 0, ctx->stream>>>(
+                g, s.buf[s.cur], ctx->ef, a, s.d_n, s.count, s.rank, nullptr, nullptr);
     }
     scan_counts(ctx, s, s.off, true);
     a.s.emit = 1;
@@ -2109,12 +2152,16 @@ extern "C" int pic_push_sort(pic_ctx* ctx, int sid, double dt) {
         const unsigned nb2 = xcd_blocks1(n, BLOCK * PUSH_SCATTER_ILP);
         if (a.s.mode == PIC_SURF_ABSORB)
             k_push_scatter<false, PUSH_SCATTER_ILP><<<nb2, BLOCK, 0, ctx->stream>>>(
-                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap);
+                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap,
+                flags ? s.safe : nullptr, s.safe_kick);
         else
             k_push_scatter<true, 1><<<xcd_blocks1(n, BLOCK), BLOCK, 0, ctx->stream>>>(
-                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap);
+                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap, nullptr,
+                nullptr);
     }
     PIC_HIP(ctx, hipGetLastError());
+    s.safe_ok = flags;
+    for (int d = 0; d < 3; d++) s.safe_dtx[d] = fabsf(a.dtx[d]);
     s.cur ^= 1;
     s.sorted = true;
     s.scrambled = false;
@@ -2244,6 +2291,7 @@ extern "C" int pic_load_box_thermal(pic_ctx* ctx, int sid, const double centre[3
     s.n_upper = base + num_macro;
     s.hist_valid = false;
     s.sorted = false;
+    s.safe_ok = false;
     s.two_part = false;
     s.tail_ok = false;
     s.scrambled = true;  // uniform positions in thread order
@@ -2260,6 +2308,7 @@ extern "C" int pic_merge(pic_ctx* ctx, int sid, uint32_t seed, pic_merge_stats* 
         rc = pic_sort(ctx, sid);
         if (rc) return rc;
     }
+    s.safe_ok = false;
     const size_t n_before = s.n_upper;
     rc = pic_ensure_pin(ctx, 64);
     if (rc) return rc;

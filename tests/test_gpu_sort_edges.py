@@ -135,3 +135,81 @@ def test_removed_particles_take_no_place_in_the_sort(pg, dt, num):
     assert np.array_equal(out[0], out[1])
     x = p[:, :3] + dt * p[:, 3:6]
     assert abs(len(out[0]) - np.sum(np.all((x > 0) & (x < L), axis=1))) <= 2 + num // 10000
+
+
+def _charged(pg, num, mass, charge, seed):
+    n, dx = (9, 10, 11), 1e-2
+    L = dx * (np.array(n) - 1)
+    rng = np.random.default_rng(seed)
+    c = pg.Context(*n, [0, 0, 0], L)
+    c.dirichlet_walls()
+    c.set_dt(1e-10)
+    p = np.zeros((num, 7))
+    p[:, :3] = rng.uniform(0.05, 0.95, (num, 3)) * L
+    p[:, 3:6] = rng.normal(0, np.sqrt(1.6e-19 * 2.0 / mass), (num, 3))
+    p[:, 6] = np.arange(num) + 1.0
+    sid = c.species_add(mass, charge, 1.0, num + 5000)
+    c.upload(sid, p)
+    c.sort(sid)
+    ef = rng.normal(0, 100.0, 3 * c.nn)
+    return c, sid, ef
+
+
+@pytest.mark.parametrize("mass,charge", [(ME, -QE), (16 * AMU, QE), (32 * AMU, 0.0)])
+@pytest.mark.parametrize("num", [65, 20_001])
+def test_push_sort_chain_equals_push_then_sort(pg, mass, charge, num):
+    """Several pic_push_sort in a row, whose histogram pass uses the flags the
+    one before left, against pic_push + pic_sort: larger and smaller steps,
+    a field that grows within and beyond the flags' bound, and every call
+    that changes the particles in between."""
+    chains = [_charged(pg, num, mass, charge, 7) for _ in range(2)]
+    field = [1.0, 1.5, 2.9, 2.9, 40.0, 40.0, 1.0, 1.0, 1.0, 1.0, 1.0]
+    steps = [1e-10, 1e-10, 1e-10, 3e-10, 1e-10, 1e-10, 1e-9, 1e-10, 1e-10, 1e-10, 1e-10]
+    for k, (amp, dt) in enumerate(zip(field, steps)):
+        rows = []
+        for fused, (c, sid, ef) in zip((True, False), chains):
+            if amp != (field[k - 1] if k else None):
+                c.set_field(pg.FIELD_EF, amp * ef)
+            if k == 7:  # other particles
+                q = c.download(sid).reshape(-1, 7)
+                q = q[np.argsort(q[:, 6])]
+                q[:, 3:6] *= -3.0
+                c.upload(sid, q)
+                c.sort(sid)
+            if k == 9:  # moved by another call
+                c.push(sid, 5e-10)
+                c.sort(sid)
+            if fused:
+                c.push_sort(sid, dt)
+            else:
+                c.push(sid, dt)
+                c.sort(sid)
+            r = c.download(sid)
+            macro = c.species_field(sid, pg.SFIELD_MACRO_COUNT)
+            cells = _cells(r, 1e-2, (9, 10, 11))
+            assert np.all(np.diff(cells) >= 0), k
+            assert np.array_equal(macro, np.bincount(cells, minlength=macro.size)), k
+            rows.append(_rows(r))
+        assert np.array_equal(rows[0], rows[1]), k
+    for c, _, _ in chains:
+        c.close()
+
+
+def test_push_sort_flags_after_collisions_and_sources(pg):
+    """DSMC_MEX changes velocities in place and a source appends: the next
+    pic_push_sort sorts by where the particles really go."""
+    c, sid, ef = _charged(pg, 30_000, 32 * AMU, 0.0, 3)
+    did = c.dsmc_create(sid)
+    src = c.source_create(sid, 0, 4e3, 5e9, 300.0)
+    for step in range(6):
+        c.push_sort(sid, 5e-7)  # about a tenth of a cell
+        r = c.download(sid)
+        cells = _cells(r, 1e-2, (9, 10, 11))
+        assert np.all(np.diff(cells) >= 0), step
+        macro = c.species_field(sid, pg.SFIELD_MACRO_COUNT)
+        assert np.array_equal(macro, np.bincount(cells, minlength=macro.size)), step
+        if step % 2:
+            assert c.dsmc_apply(did, 1e7, 5, step)["collisions"] > 1000
+        else:
+            assert c.source_sample(src, seed=step) > 0
+    c.close()
