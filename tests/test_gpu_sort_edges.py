@@ -213,3 +213,23 @@ def test_push_sort_flags_after_collisions_and_sources(pg):
         else:
             assert c.source_sample(src, seed=step) > 0
     c.close()
+
+
+@pytest.mark.parametrize("num", [0, 1, (1 << 20) - 1, 1 << 20, (1 << 20) + 3])
+def test_upload_in_pieces(pg, num):
+    """uploads of no, one, and just below and above one staging piece"""
+    n, dx = (9, 10, 11), 1e-2
+    L = dx * (np.array(n) - 1)
+    rng = np.random.default_rng(2)
+    p = np.zeros((num, 7))
+    p[:, :3] = rng.uniform(0.01, 0.99, (num, 3)) * L
+    p[:, 3:6] = rng.normal(0, 1e3, (num, 3)).astype(np.float32)
+    p[:, 6] = np.arange(num) + 1.0
+    c = pg.Context(*n, [0, 0, 0], L)
+    sid = c.species_add(ME, -QE, 1.0, max(num, 1))
+    c.upload(sid, p)
+    q = c.download(sid).reshape(-1, 7)
+    assert np.array_equal(q[:, 3:], p[:, 3:])
+    # the offset in the cell is stored in FP32
+    assert num == 0 or np.max(np.abs(q[:, :3] - p[:, :3])) <= 1e-7 * dx
+    c.close()
