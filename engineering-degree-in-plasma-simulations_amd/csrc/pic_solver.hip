@@ -473,10 +473,12 @@ __global__ void __launch_bounds__(BLOCK)
 // 18.8 with 1280, 16.1 with 1024, 16.3 with 512)
 constexpr int PART_MAX = 1024;
 // ctx->scratch offsets of the partials: three residual sums, then PCG's g.s,
-// g.g and d.z; the stop flag and the g.s ring follow
+// g.g and d.z (a second set of these for k_cg, which reads one and writes the
+// other); the stop flag and the rings of g.s and alpha follow
 constexpr int PART_F = 16384, PART_GS = PART_F + 3 * PART_MAX, PART_GG = PART_GS + PART_MAX,
-              PART_DZ = PART_GG + PART_MAX, PCG_FLAG = PART_DZ + PART_MAX, PCG_GS = PCG_FLAG + 8;
-static_assert(PCG_GS + 4 <= (int)SCRATCH_DOUBLES, "scratch layout");
+              PART_DZ = PART_GG + PART_MAX, PART_SET = 3 * PART_MAX, PCG_FLAG = PART_GS + 2 * PART_SET,
+              PCG_GS = PCG_FLAG + 8, PCG_AL = PCG_GS + 4;
+static_assert(PCG_AL + 4 <= (int)SCRATCH_DOUBLES, "scratch layout");
 __device__ inline double sum_parts(const double* __restrict__ part, int n) {
     __shared__ double red[BLOCK / 64];
     double v = 0;
@@ -891,13 +893,141 @@ __global__ void __launch_bounds__(BLOCK)
     }
 }
 
+// The same iteration in one kernel (Chronopoulos and Gear's arrangement of CG:
+// J. Comput. Appl. Math. 25, 1989), for grids without Neumann faces that a
+// launch's latency bounds.  With u = M g, w = J u and the sums gamma = g.u,
+// delta = w.u of the last kernel,
+//   beta = gamma / gamma_old,  alpha = gamma / (delta - beta gamma / alpha_old)
+//   d = -u + beta d,  z = -w + beta z (= J d),  y += alpha d,  g += alpha z
+// and then the new w and sums.  The new w needs the new g of the neighbours,
+// which every thread makes again from the old g, w and z around its group;
+// those three are therefore written to a second set of vectors.  t = -1: w and
+// delta of the start.
+template <typename T>
+struct CgVec {
+    T *y, *d, *g[2], *w[2], *z[2];
+    const double* P;  // may be null
+};
+template <typename T>
+__global__ void __launch_bounds__(BLOCK)
+    k_cg(Stencil s, const uint8_t* __restrict__ nt, CgVec<T> v, double* __restrict__ scratch,
+         double* __restrict__ ggh, int t) {
+    if (scratch[PCG_FLAG] != 0.0) return;  // (the whole grid)
+    const int from = t < 0 ? 0 : t & 1, to = t < 0 ? 0 : (t + 1) & 1;
+    const double* __restrict__ pin = scratch + from * PART_SET;
+    double* __restrict__ pout = scratch + to * PART_SET;
+    const T* __restrict__ gi = v.g[from];
+    const T* __restrict__ wi = v.w[from];
+    const T* __restrict__ zi = v.z[from];
+    const T mreg = (T)(1.0 / diagA(NT_REG, s));  // M of a regular row; g vanishes on the others
+    long long end;
+    long long m = chunk_begin(s.nn / 4, end) + threadIdx.x;
+    Ring4<T> g{}, w{}, z{};
+    Q4<T> d4{}, y4{};
+    uint32_t t4 = 0;
+    auto load = [&]() {
+        const unsigned u0 = 4u * (unsigned)m;
+        t4 = load_types4(nt, u0);
+        load_ring4(gi, u0, s, g);
+        if (t >= 0) load_ring4(wi, u0, s, w);
+        if (t > 0) {
+            load_ring4(zi, u0, s, z);
+            d4 = load4(v.d + u0);
+            y4 = load4(v.y + u0);
+        }
+    };
+    if (m < end) load();
+    double al = 0.0, be = 0.0, gamma = 0.0;
+    if (t >= 0) {
+        gamma = sum_parts(pin + PART_GS, gridDim.x);
+        double den = sum_parts(pin + PART_DZ, gridDim.x);
+        if (t > 0) {
+            const double go = scratch[PCG_GS + ((t - 1) & 3)], ao = scratch[PCG_AL + ((t - 1) & 3)];
+            be = go != 0.0 ? gamma / go : 0.0;
+            if (ao != 0.0) den -= be * gamma / ao;
+        }
+        al = den != 0.0 ? gamma / den : 0.0;
+    }
+    const T alpha = (T)al, beta = (T)be;
+    double gs = 0, gg = 0, dz = 0;
+    while (m < end) {
+        const unsigned u0 = 4u * (unsigned)m;
+        T zn[4], gn[4], wn[4], dn[4], yn[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            zn[q] = -w.c.a[q] + beta * z.c.a[q];
+            dn[q] = -(mreg * g.c.a[q]) + beta * d4.a[q];
+            yn[q] = y4.a[q] + alpha * dn[q];
+        }
+        // the new g around the group, then u = M g in its place
+        auto next = [&](T& gv, T wv, T zv) { gv = mreg * (gv + alpha * (-wv + beta * zv)); };
+        T gc[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            gc[q] = g.c.a[q] + alpha * zn[q];
+            g.c.a[q] = mreg * gc[q];
+            next(g.ym.a[q], w.ym.a[q], z.ym.a[q]);
+            next(g.yp.a[q], w.yp.a[q], z.yp.a[q]);
+            next(g.zm.a[q], w.zm.a[q], z.zm.a[q]);
+            next(g.zp.a[q], w.zp.a[q], z.zp.a[q]);
+        }
+        next(g.l, w.l, z.l);
+        next(g.r, w.r, z.r);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const T u = g.c.a[q];
+            T ju = type_at(t4, q) == NT_REG ? ring_A(g, q, s) : u;
+            if (v.P) ju -= (T)v.P[u0 + q] * u;
+            wn[q] = ju;
+            gn[q] = gc[q];
+            gs += (double)gn[q] * (double)u;
+            gg += (double)gn[q] * (double)gn[q];
+            dz += (double)ju * (double)u;
+        }
+        store4(v.w[to] + u0, wn);
+        if (t >= 0) {
+            store4(v.g[to] + u0, gn);
+            store4(v.z[to] + u0, zn);
+            store4(v.d + u0, dn);
+            store4(v.y + u0, yn);
+        }
+        m += BLOCK;
+        if (m < end) load();
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group: all zero
+        const long long u = (s.nn & ~3ll) + threadIdx.x;
+        v.w[to][u] = 0;
+        if (t >= 0) {
+            v.g[to][u] = 0;
+            v.z[to][u] = 0;
+            v.y[u] = 0;
+        }
+    }
+    const double a = block_sum(gs), b = block_sum(gg), c = block_sum(dz);
+    if (threadIdx.x == 0) {
+        if (t >= 0) {
+            pout[PART_GS + blockIdx.x] = a;
+            pout[PART_GG + blockIdx.x] = b;
+        }
+        pout[PART_DZ + blockIdx.x] = c;
+    }
+    if (blockIdx.x == 0 && t >= 0) {
+        const double g0 = sum_parts(pin + PART_GG, gridDim.x);
+        if (threadIdx.x == 0) {
+            scratch[PCG_GS + (t & 3)] = gamma;
+            scratch[PCG_AL + (t & 3)] = al;
+            ggh[t] = g0;
+        }
+    }
+}
+
 // The end of a batch of iterations (t0, t1]: g.g of each to the host (pinned
 // memory), and the stop flag when one is within the target.
 __global__ void __launch_bounds__(BLOCK)
-    k_pcg_check(double* __restrict__ scratch, const double* __restrict__ ggh, int nb, int t0, int t1,
-                double target2, double* host) {
+    k_pcg_check(double* __restrict__ scratch, const double* __restrict__ gg1, const double* __restrict__ ggh, int nb,
+                int t0, int t1, double target2, double* host) {
     if (scratch[PCG_FLAG] != 0.0) return;
-    const double gg = sum_parts(scratch + PART_GG, nb);
+    const double gg = sum_parts(gg1, nb);  // of iteration t1
     __shared__ int hit;
     if (threadIdx.x == 0) hit = 0;
     __syncthreads();
@@ -1205,9 +1335,10 @@ static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
 // stop flag), so y is the one of the batch that converged.  hp: 2 * check
 // doubles of pinned memory; ggh: max_it + 1 doubles on the device.
 template <typename T, bool NEU>
-static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, T* d1, double* ggh, double* hp,
-                     double target2, int max_it, int check, int* iters) {
+static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, T* d1, const CgVec<T>* cg, double* ggh,
+                     double* hp, double target2, int max_it, int check, int* iters) {
     const unsigned nb = part_blocks(s.nn);
+    if (cg) k_cg<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, *cg, ctx->scratch, ggh, -1);
     for (auto& e : ctx->batch_ev)
         if (!e) PIC_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // profiled runs wait for every batch, so that no returned-at-once
@@ -1219,14 +1350,19 @@ static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, 
     for (;;) {
         while (t < max_it && queued - done < ahead) {
             const int q = queued & 1, t0 = t, upto = std::min(max_it, t + check);
-            for (; t < upto; t++) {  // one profiled "launch" = one PCG iteration (2 kernels)
+            for (; t < upto; t++) {  // one profiled "launch" = one PCG iteration (1 or 2 kernels)
                 PicProfScope ps(ctx, PIC_K_PCG);
+                if (cg) {
+                    k_cg<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, *cg, ctx->scratch, ggh, t);
+                    continue;
+                }
                 k_pcg1<T, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v, dold, dnew, ctx->scratch, ggh, t);
                 k_pcg2<T, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v, dnew, ctx->scratch, t);
                 std::swap(dold, dnew);
             }
-            k_pcg_check<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch, ggh, (int)nb, t0, t, target2,
-                                                      hp + (size_t)q * check);
+            k_pcg_check<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch,
+                                                      ctx->scratch + (cg ? (t & 1) * PART_SET : 0) + PART_GG, ggh,
+                                                      (int)nb, t0, t, target2, hp + (size_t)q * check);
             PIC_HIP(ctx, hipGetLastError());
             PIC_HIP(ctx, hipEventRecord(ctx->batch_ev[q], ctx->stream));
             beg[q] = t0;
@@ -1251,6 +1387,14 @@ static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, 
     }
 }
 
+// Nodes up to which an iteration is one kernel (k_cg): one launch's latency
+// against three stencil operands instead of one.  Cold solves, two kernels and
+// one: FP32-inner 33^3 1.61 and 1.24 ms, 64^3 3.06 and 2.26, a run on 97 x 65 x 49
+// 16.3 and 14.4, 100^3 6.5 and 7.5; FP64 33^3 1.37 and 1.13, 50^3 1.84 and 1.60, 70^3
+// 3.44 and 3.28, 90^3 5.3 and 6.4.
+template <typename T>
+constexpr size_t CG_ONE_MAX = sizeof(T) == sizeof(float) ? (size_t)1 << 19 : (size_t)3 << 17;
+
 // Newton + PCG (PotentialSolver.cpp:178-241).  The linear case (n0 == 0)
 // needs a single Newton step; each Newton step restarts PCG from y = 0.
 template <typename T, bool NEU>
@@ -1265,7 +1409,8 @@ static int solve_pcg_t(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stat
     // y, g, d0, d1, z (s), P, the g.g history; each vector on a 256-byte line
     const size_t vs = (nn * sizeof(T) + 255) & ~(size_t)255;
     const size_t ps = nonlinear ? (nn * sizeof(double) + 255) & ~(size_t)255 : 0;
-    const int nvec = NEU ? 6 : 5;
+    const bool one = !NEU && nn <= CG_ONE_MAX<T>;  // one kernel per iteration (k_cg)
+    const int nvec = NEU ? 6 : one ? 8 : 5;
     int rc = pic_ensure_work(ctx, nvec * vs + ps + ((size_t)max_it + 2) * sizeof(double));
     if (rc) return rc;
     rc = pic_ensure_pin(ctx, (8 + 2 * (size_t)check) * sizeof(double));
@@ -1280,6 +1425,8 @@ static int solve_pcg_t(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stat
     v.z = vec(4);
     v.s = NEU ? vec(5) : nullptr;
     v.P = P;
+    // k_cg's vectors: g's first is k_F's g
+    const CgVec<T> cg{vec(0), vec(2), {vec(1), vec(3)}, {vec(4), vec(5)}, {vec(6), vec(7)}, P};
     volatile double* hp = ctx->pin;  // [0, 5) sums of k_F, [5] y.y, [8, ...) g.g of the batches
     NewtonArgs na;
     na.ieps = 1.0 / EPS0;
@@ -1330,8 +1477,8 @@ static int solve_pcg_t(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stat
         double yy = 0;
         if (!(gg0 <= inner_target2)) {  // otherwise y = 0 (a zero right-hand side included)
             int its = 0;
-            rc = pcg_inner<T, NEU>(ctx, s, v, vec(2), vec(3), ggh, ctx->pin + 8, inner_target2, max_it - total_it,
-                                   check, &its);
+            rc = pcg_inner<T, NEU>(ctx, s, v, vec(2), vec(3), one ? &cg : nullptr, ggh, ctx->pin + 8, inner_target2,
+                                   max_it - total_it, check, &its);
             total_it += its;
             if (rc < 0) return rc;
             const bool want_yy = nonlinear && p->tol_kind == PIC_TOL_REF_RMS;
