@@ -525,8 +525,29 @@ __global__ void __launch_bounds__(BLOCK)
 }
 
 // ---- exclusive scan of count[0..M) -> off[0..M], M = ncells + 1 ----
-constexpr int SCAN_ITEMS = 16;
-constexpr int SCAN_TILE = BLOCK * SCAN_ITEMS;
+// A workgroup scans a tile as SCAN_ROWS rows of four items per thread, so that
+// consecutive lanes read and write consecutive 16 bytes.  2M cells: reduce 4.7
+// us and down 5.4; 6.7 and 14.0 with 16 consecutive items per thread, whose
+// loads and stores took 64-byte strides.
+constexpr int SCAN_ROWS = 4;
+constexpr int SCAN_ROW = BLOCK * 4;
+constexpr int SCAN_TILE = SCAN_ROW * SCAN_ROWS;
+struct Scan4 {
+    uint32_t a[4];
+};
+__device__ inline Scan4 scan_load(const uint32_t* __restrict__ in, size_t i, size_t M) {
+    typedef uint32_t V __attribute__((ext_vector_type(4), aligned(4)));
+    Scan4 r{{0u, 0u, 0u, 0u}};
+    if (i + 4 <= M) {
+        const V v = *reinterpret_cast<const V*>(in + i);
+        r = Scan4{{v[0], v[1], v[2], v[3]}};
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (i + q < M) r.a[q] = in[i + q];
+    }
+    return r;
+}
 
 __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* total) {
     __shared__ uint32_t wsum[BLOCK / 64];
@@ -552,11 +573,13 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* total) {
 
 __global__ void __launch_bounds__(BLOCK) k_scan_reduce(const uint32_t* __restrict__ in, int M,
                                                        uint32_t* __restrict__ bsum) {
-    size_t base = (size_t)blockIdx.x * SCAN_TILE + (size_t)threadIdx.x * SCAN_ITEMS;
+    const size_t base = (size_t)blockIdx.x * SCAN_TILE + (size_t)threadIdx.x * 4;
     uint32_t s = 0;
 #pragma unroll
-    for (int q = 0; q < SCAN_ITEMS; q++)
-        if (base + q < (size_t)M) s += in[base + q];
+    for (int r = 0; r < SCAN_ROWS; r++) {
+        const Scan4 v = scan_load(in, base + (size_t)r * SCAN_ROW, (size_t)M);
+        s += (v.a[0] + v.a[1]) + (v.a[2] + v.a[3]);
+    }
     uint32_t tot;
     block_exclusive_scan(s, &tot);
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
@@ -581,27 +604,37 @@ __global__ void __launch_bounds__(BLOCK) k_scan_top(uint32_t* __restrict__ bsum,
 __global__ void __launch_bounds__(BLOCK)
     k_scan_down(const uint32_t* __restrict__ in, int M, const uint32_t* __restrict__ bsum,
                 uint32_t* __restrict__ out, int ncells, uint32_t* __restrict__ d_n) {
-    size_t base = (size_t)blockIdx.x * SCAN_TILE + (size_t)threadIdx.x * SCAN_ITEMS;
-    uint32_t v[SCAN_ITEMS];
-    uint32_t s = 0;
+    typedef uint32_t V __attribute__((ext_vector_type(4), aligned(4)));
+    const size_t base = (size_t)blockIdx.x * SCAN_TILE + (size_t)threadIdx.x * 4;
+    Scan4 v[SCAN_ROWS];
 #pragma unroll
-    for (int q = 0; q < SCAN_ITEMS; q++) {
-        v[q] = (base + q < (size_t)M) ? in[base + q] : 0u;
-        s += v[q];
-    }
-    uint32_t ex = block_exclusive_scan(s, nullptr) + bsum[blockIdx.x];
+    for (int r = 0; r < SCAN_ROWS; r++) v[r] = scan_load(in, base + (size_t)r * SCAN_ROW, (size_t)M);
+    uint32_t carry = bsum[blockIdx.x];
 #pragma unroll
-    for (int q = 0; q < SCAN_ITEMS; q++) {
-        size_t idx = base + q;
-        if (idx < (size_t)M) {
-            out[idx] = ex;
+    for (int r = 0; r < SCAN_ROWS; r++) {
+        uint32_t total;
+        uint32_t ex = carry + block_exclusive_scan((v[r].a[0] + v[r].a[1]) + (v[r].a[2] + v[r].a[3]), &total);
+        carry += total;
+        const size_t i = base + (size_t)r * SCAN_ROW;
+        uint32_t o[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            o[q] = ex;
+            const size_t idx = i + q;
             if (idx == (size_t)ncells && d_n) {  // particles alive after compaction
                 d_n[0] = ex;
                 d_n[3] = ex;  // all of them sorted: the sorted part of a two-part species
             }
-            if (idx == (size_t)M - 1) out[M] = ex + v[q];
+            ex += v[r].a[q];
+            if (idx == (size_t)M - 1) out[M] = ex;
         }
-        ex += v[q];
+        if (i + 4 <= (size_t)M) {
+            *reinterpret_cast<V*>(out + i) = V{o[0], o[1], o[2], o[3]};
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (i + q < (size_t)M) out[i + q] = o[q];
+        }
     }
 }
 

@@ -233,3 +233,28 @@ def test_upload_in_pieces(pg, num):
     # the offset in the cell is stored in FP32
     assert num == 0 or np.max(np.abs(q[:, :3] - p[:, :3])) <= 1e-7 * dx
     c.close()
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (5, 5, 64), (33, 33, 5), (33, 33, 6), (17, 65, 67), (50, 100, 201)])
+def test_cell_offsets_at_scan_tile_edges(pg, shape):
+    """cell counts below, at and above a scan row (1024) and tile (4096), and
+    more tiles than one workgroup has threads"""
+    dx = 1e-2
+    L = dx * (np.array(shape) - 1)
+    ncells = int(np.prod(np.array(shape) - 1))
+    rng = np.random.default_rng(ncells)
+    num = 20_000
+    p = np.zeros((num, 7))
+    p[:, :3] = rng.uniform(0.001, 0.999, (num, 3)) * L
+    p[:, 6] = np.arange(num) + 1.0
+    c = pg.Context(*shape, [0, 0, 0], L)
+    sid = c.species_add(ME, 0.0, 1.0, num)
+    c.upload(sid, p)
+    for sort in (c.sort, lambda s: c.push_sort(s, 1e-12)):
+        sort(sid)
+        q = c.download(sid)
+        assert np.array_equal(np.sort(q.reshape(-1, 7)[:, 6]), p[:, 6])
+        cells = _cells(q, dx, shape)
+        assert np.all(np.diff(cells) >= 0)
+        assert np.array_equal(c.species_field(sid, pg.SFIELD_MACRO_COUNT), np.bincount(cells, minlength=ncells))
+    c.close()
