@@ -1115,9 +1115,9 @@ constexpr int WX = 8, WY = 4, WZ = 4;  // voxels of a tile
 // sum it is exactly (24 bits of significand in three times 8), padded to 16;
 // k_wgrad_sum3 adds the three.  An infinity is one part, so that it stays one in
 // the sums.  In FP32 vector arithmetic the two layers took 253 and 123 us at 64^3
-// voxels and a training step of two samples 4.45 ms, here 3.95 ms.  Error of their
-// gradients against 64 bits from the same operands, at 32^3 and 64^3 voxels:
-// input 2.2e-7 to 3.5e-7 before, 3.7e-8 to 4.6e-8 here; output 3.3e-7 to 5.0e-7
+// voxels and a training step of two samples 4.45 ms; here 47 and 42 us and 3.9 ms.
+// Error of their gradients against 64 bits from the same operands, at 32^3 and
+// 64^3 voxels: input 2.2e-7 to 3.5e-7 before, 3.7e-8 to 4.6e-8 here; output 3.3e-7 to 5.0e-7
 // before, 0.9e-7 to 1.8e-7 here.
 __device__ inline void split3(float x, uint32_t (&h)[3]) {
 #pragma unroll
