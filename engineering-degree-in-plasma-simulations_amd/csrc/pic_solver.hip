@@ -1283,8 +1283,8 @@ static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
         while (it < p->max_it && queued - done < ahead) {
             const int q = queued & 1;
             // sweep numbers 0, check, 2 check, ... are checked, and the last
-            int upto = it == 0 ? 1 : it + check;
-            if (upto > p->max_it) upto = p->max_it;
+            // (check may be as large as INT_MAX: only the first sweep and the last)
+            const int upto = it == 0 ? 1 : check < p->max_it - it ? it + check : p->max_it;
             while (it < upto) {
                 PicProfScope ps(ctx, PIC_K_SOR);
                 const int n = std::min(2, upto - it);
@@ -1349,7 +1349,7 @@ static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, 
     T *dold = d0, *dnew = d1;
     for (;;) {
         while (t < max_it && queued - done < ahead) {
-            const int q = queued & 1, t0 = t, upto = std::min(max_it, t + check);
+            const int q = queued & 1, t0 = t, upto = check < max_it - t ? t + check : max_it;
             for (; t < upto; t++) {  // one profiled "launch" = one PCG iteration (1 or 2 kernels)
                 PicProfScope ps(ctx, PIC_K_PCG);
                 if (cg) {

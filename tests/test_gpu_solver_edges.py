@@ -113,3 +113,24 @@ def test_tiled_sor_sweeps_equal_plain(pg, shape, sides, n0):
             c.close()
         assert np.array_equal(out[0][0], out[1][0], equal_nan=True), max_it
         assert out[0][1] == pytest.approx(out[1][1], rel=1e-11, nan_ok=True)
+
+
+@pytest.mark.parametrize("check", [2**31 - 1, 2**31 - 7, 31])
+@pytest.mark.parametrize("flags", ["SOLVE_SOR_PLAIN", None])
+def test_sor_check_interval_beyond_the_sweeps(pg, check, flags):
+    """A check interval larger than max_it, up to INT_MAX (only the first sweep
+    and the last are checked): all max_it sweeps are made, and the sweep
+    count does not overflow."""
+    shape = (17, 12, 9)
+    L = [1e-2 * (n - 1) for n in shape]
+    out = []
+    for chk in (check, 1):
+        c = pg.Context(*shape, [0, 0, 0], L)
+        c.dirichlet_walls()
+        c.set_field(pg.FIELD_RHO, _rho(shape, 2))
+        st = c.poisson(pg.SOLVER_SOR_RB, tol=1e-300, tol_kind=pg.TOL_REL, max_it=31, omega=1.5, check_every=chk,
+                       flags=getattr(pg, flags) if flags else 0)
+        assert st["iterations"] == 31 and not st["converged"]
+        out.append(c.get_field(pg.FIELD_PHI))
+        c.close()
+    assert np.array_equal(out[0], out[1])
