@@ -1250,11 +1250,21 @@ static void sor_sweeps(pic_ctx* ctx, const Stencil& s, const SorArgs& a, bool ne
         launch_sor_tile<16, 32, 16>(ctx, s, a, neu, in, out, sweeps, own);
 }
 
+// Launches (PCG: iterations) that the host queues behind a check before it
+// waits for it: enough to keep the device busy while the host sees the check's
+// event, and few, because those behind a check that ends the solve are waited
+// for although they return at once (2 us each).  32^3 nodes, SOR from the solution,
+// a check every 25 and every 1000 sweeps: 44 us with 4; 75 and 2225 with the whole
+// interval queued; 47 and 69 with none.  The cold solve 0.38 ms with 2 and with 4, 0.40
+// with the whole interval; 128^3 FP64 PCG 12.6 ms with any.
+constexpr int RUN_AHEAD = 4;
+
 // Red-black SOR (PotentialSolver.cpp:69-166) on tiles.  The residual is
 // checked after the first sweep and then every `check` sweeps (:124); the
-// host queues the sweeps up to the next check before it waits for the last
-// one, and once a check is met the launches behind it return at once (the
-// stop flag), so the potential is the one that was checked.
+// host queues the first RUN_AHEAD launches of the sweeps up to the next check
+// before it waits for the last one, and once a check is met the launches
+// behind it return at once (the stop flag), so the potential is the one that
+// was checked.
 static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st) {
     if (p->flags & PIC_SOLVE_SOR_PLAIN) return solve_sor_plain(ctx, p, st);
     const GridC& g = ctx->g;
@@ -1279,19 +1289,33 @@ static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
     int at[2], par[2], queued = 0, done = 0; // batches queued and waited for; their last sweep and buffer
     bool conv = false;
     int last = 0;
-    for (;;) {
-        while (it < p->max_it && queued - done < ahead) {
+    auto wait_oldest = [&]() {  // for the oldest queued batch; conv: it met the criterion
+        last = done & 1;
+        const hipError_t e = pic_spin_event(ctx->batch_ev[last]);
+        if (e != hipSuccess) return pic_hip_check(ctx, e, "SOR check");
+        done++;
+        conv = hp[4 * last + 3] != 0.0;
+        return (int)PIC_OK;
+    };
+    while (!conv) {
+        while (!conv && it < p->max_it && queued - done < ahead) {
             const int q = queued & 1;
             // sweep numbers 0, check, 2 check, ... are checked, and the last
             // (check may be as large as INT_MAX: only the first sweep and the last)
             const int upto = it == 0 ? 1 : check < p->max_it - it ? it + check : p->max_it;
-            while (it < upto) {
+            for (int m = 0; it < upto; m++) {
+                if (m == RUN_AHEAD && queued > done) {
+                    rc = wait_oldest();
+                    if (rc) return rc;
+                    if (conv) break;
+                }
                 PicProfScope ps(ctx, PIC_K_SOR);
                 const int n = std::min(2, upto - it);
                 sor_sweeps(ctx, s, a, neu, buf[launches & 1], buf[(launches & 1) ^ 1], n, it > 0);
                 launches++;
                 it += n;
             }
+            if (conv) break;
             double* cur = buf[launches & 1];
             if (neu)
                 k_neumann_all<<<stencil_blocks(s.nn), BLOCK, 0, ctx->stream>>>(s, ctx->ntype, cur,
@@ -1307,14 +1331,9 @@ static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
             par[q] = launches & 1;
             queued++;
         }
-        if (done == queued) break;
-        last = done & 1;
-        PIC_HIP(ctx, pic_spin_event(ctx->batch_ev[last]));
-        done++;
-        if (hp[4 * last + 3] != 0.0) {
-            conv = true;
-            break;
-        }
+        if (conv || done == queued) break;
+        rc = wait_oldest();
+        if (rc) return rc;
     }
     if (par[last]) std::swap(ctx->phi, ctx->sor_phi);
     double r[3];
@@ -1329,11 +1348,12 @@ static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
 
 // The iterations of PCG on J y = F after k_F's set-up (vectors of type T, g.g
 // = gg0 > target2); stops at the end of the first batch of `check` iterations
-// in which g.g reached target2, or at max_it.  The host queues one batch
-// ahead of the one it waits for, so the device never idles during a check;
-// once a batch has converged the kernels of the next return at once (the
-// stop flag), so y is the one of the batch that converged.  hp: 2 * check
-// doubles of pinned memory; ggh: max_it + 1 doubles on the device.
+// in which g.g reached target2, or at max_it.  The host queues the first
+// RUN_AHEAD iterations of the next batch before it waits for one, so the
+// device never idles during a check; once a batch has converged the kernels
+// behind it return at once (the stop flag), so y is the one of the batch that
+// converged.  hp: 2 * check doubles of pinned memory; ggh: max_it + 1 doubles
+// on the device.
 template <typename T, bool NEU>
 static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, T* d1, const CgVec<T>* cg, double* ggh,
                      double* hp, double target2, int max_it, int check, int* iters) {
@@ -1347,10 +1367,31 @@ static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, 
     int t = 0;                        // iterations queued
     int beg[2], end[2], queued = 0, done = 0;  // batches queued and waited for
     T *dold = d0, *dnew = d1;
+    bool conv = false;
+    auto wait_oldest = [&]() {  // for the oldest queued batch; conv: it reached target2
+        const int q = done & 1;
+        const hipError_t e = pic_spin_event(ctx->batch_ev[q]);
+        if (e != hipSuccess) return pic_hip_check(ctx, e, "PCG check");
+        done++;
+        const volatile double* h = hp + (size_t)q * check;
+        for (int m = 0; m < end[q] - beg[q]; m++) {
+            if (!(h[m] == h[m])) return pic_fail(ctx, PIC_ERR_NUMERIC, "PCG produced NaN");
+            if (h[m] <= target2) {
+                *iters = end[q];
+                conv = true;
+                break;
+            }
+        }
+        return (int)PIC_OK;
+    };
     for (;;) {
         while (t < max_it && queued - done < ahead) {
             const int q = queued & 1, t0 = t, upto = check < max_it - t ? t + check : max_it;
             for (; t < upto; t++) {  // one profiled "launch" = one PCG iteration (1 or 2 kernels)
+                if (t - t0 == RUN_AHEAD && queued > done) {
+                    const int rc = wait_oldest();
+                    if (rc || conv) return rc;
+                }
                 PicProfScope ps(ctx, PIC_K_PCG);
                 if (cg) {
                     k_cg<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, *cg, ctx->scratch, ggh, t);
@@ -1373,17 +1414,8 @@ static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, 
             *iters = t;
             return PIC_NOT_CONVERGED;
         }
-        const int q = done & 1;
-        PIC_HIP(ctx, pic_spin_event(ctx->batch_ev[q]));
-        done++;
-        const volatile double* h = hp + (size_t)q * check;
-        for (int e = 0; e < end[q] - beg[q]; e++) {
-            if (!(h[e] == h[e])) return pic_fail(ctx, PIC_ERR_NUMERIC, "PCG produced NaN");
-            if (h[e] <= target2) {
-                *iters = end[q];
-                return PIC_OK;
-            }
-        }
+        const int rc = wait_oldest();
+        if (rc || conv) return rc;
     }
 }
 
