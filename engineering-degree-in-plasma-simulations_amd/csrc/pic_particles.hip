@@ -1868,11 +1868,11 @@ static int after_emission(pic_ctx* ctx, const Species& s, const PushArgs& a) {
     PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (hn[0] > t.cap) hn[0] = (uint32_t)t.cap;
     t.bulk_n = hn[3];  // the emissions were appended behind the last whole sort's particles
-    if ((size_t)hn[0] != t.n_upper) {
-        t.n_upper = hn[0];
-        t.sorted = false;
-        t.hist_valid = false;
-    }
+    // whether anything was appended is read from the counts on the device:
+    // the host's n_upper is not lowered when particles leave in a push
+    if (hn[0] != hn[3]) t.sorted = false;      // beyond the last whole sort
+    if (hn[0] != hn[1]) t.hist_valid = false;  // beyond the histogram
+    t.n_upper = hn[0];
     if (hn[2]) {
         uint32_t z = 0;
         PIC_HIP(ctx, hipMemcpyAsync(t.d_n + 2, &z, sizeof(z), hipMemcpyHostToDevice, ctx->stream));

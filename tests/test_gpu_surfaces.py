@@ -181,3 +181,44 @@ def test_reflection_steps_are_keyed_by_push_count(pg, golden):
                                    stable=True)
     with pytest.raises(AssertionError):
         _match(r2x, c.download(a), g, allow=3)
+
+
+@pytest.mark.parametrize("state", ["sorted", "histogram"])
+def test_as_many_emitted_as_had_left(pg, state):
+    """A target that lost particles in its own push and then receives exactly
+    as many emitted ones: its count is what it was, and the emitted ones are
+    nevertheless in the next density, macro count and sort."""
+    n, dx, left = 11, 0.01, 37
+    L = dx * (n - 1)
+    c = pg.Context(n, n, n, [0, 0, 0], [L, L, L])
+    c.add_rectangle([L / 2, L / 2, L / 2], [1.2 * L, 1.2 * L, dx], 0.0)
+    c.set_dt(1e-6)
+    rng = np.random.default_rng(5)
+
+    def parts(num, z, v, w):
+        p = np.zeros((num, 7))
+        p[:, :2] = rng.uniform(0.2 * L, 0.8 * L, (num, 2))
+        p[:, 2] = z
+        p[:, 3:6] = v
+        p[:, 6] = w
+        return p
+
+    sn = c.species_add(16 * O.AMU, 0.0, 2.0, 3000)
+    si = c.species_add(16 * O.AMU, 0.0, 2.0, 100)
+    c.upload(sn, np.concatenate([parts(1000 - left, 0.2 * L, 0.0, 2.0), parts(left, 0.1 * L, [2e5, 0, 0], 2.0)]))
+    c.upload(si, parts(left, 0.42 * L, [0, 0, 8e3], 2.0))  # each emits int(1 + U) = 1
+    c.set_surface(si, pg.SURF_RECYCLE, sn, seed=3)
+    c.sort(sn)
+    c.sort(si)
+    c.push_sort(sn, 1e-6)
+    if state == "histogram":
+        c.push(sn, 1e-12)
+    c.push(si, 1e-6)
+    c.deposit(sn)
+    den = c.species_field(sn, pg.SFIELD_DEN) * c.get_field(pg.FIELD_NODE_VOL)
+    assert abs(den.sum() - 2.0 * 1000) < 1e-2
+    assert c.species_field(sn, pg.SFIELD_MACRO_COUNT).sum() == 1000
+    assert c.count(sn) == 1000 and c.count(si) == 0
+    q = c.download(sn).reshape(-1, 7)
+    assert np.sum(np.abs(q[:, 2] - 0.45 * L) < 1e-6) == left  # on the plate's lower face
+    c.close()
