@@ -2057,6 +2057,31 @@ static int sort_partitioned(pic_ctx* ctx, Species& s) {
 // launches; a run of 50M with collisions 16.1 ms joined, 19.1 sorted whole
 constexpr size_t JOIN_MIN = 1u << 20;
 
+// an index of the appended particles up to t_end that the next one extends
+static bool tail_indexed(const Species& s) {
+    return s.two_part && s.t_end >= s.bulk_n && s.t_end <= s.n_upper;
+}
+// memory for the index of the particles appended since (pic_sort_tail); kept
+// with the species
+static hipError_t tail_room(const GridC& g, Species& s) {
+    const bool more = tail_indexed(s);
+    if (s.n_upper == (more ? s.t_end : s.bulk_n)) return hipSuccess;  // none
+    const size_t words = ((size_t)g.ncells + 2) * 4, iw = (s.cap + 63) / 64 * 64 * 4;
+    hipError_t e = hipSuccess;
+    auto get = [&](uint32_t*& p, size_t bytes) {
+        if (!p && e == hipSuccess) e = hipMalloc(&p, bytes);
+    };
+    get(s.toff, words);
+    get(s.tidx, iw);
+    if (more) {
+        get(s.boff, words);
+        get(s.toff_n, words);
+        get(s.tidx_n, iw);
+    }
+    if (e != hipSuccess) (void)hipGetLastError();  // not the next launch's error
+    return e;
+}
+
 extern "C" int pic_sort(pic_ctx* ctx, int sid) {
     int rc = pic_check_sid(ctx, sid);
     if (rc) return rc;
@@ -2066,8 +2091,10 @@ extern "C" int pic_sort(pic_ctx* ctx, int sid) {
     s.safe_ok = false;
     // Only appended since the last whole sort (DSMC births, emissions): the
     // two parts are joined, which streams them, where a counting sort would
-    // scatter the appended part over the whole array.
-    if (!s.sorted && s.tail_ok && s.n_upper >= s.bulk_n && s.bulk_n >= JOIN_MIN) {
+    // scatter the appended part over the whole array.  Without memory for the
+    // index (4 bytes per particle of the capacity) it is sorted whole.
+    if (!s.sorted && s.tail_ok && s.n_upper >= s.bulk_n && s.bulk_n >= JOIN_MIN &&
+        tail_room(g, s) == hipSuccess) {
         rc = pic_sort_tail(ctx, sid);
         if (rc) return rc;
         if (s.two_part) return pic_join_tail(ctx, sid);
@@ -2113,15 +2140,13 @@ int pic_sort_tail(pic_ctx* ctx, int sid) {
     const GridC& g = ctx->g;
     const size_t n = s.n_upper;
     if (n < s.bulk_n) return pic_fail(ctx, PIC_ERR_STATE, "appended part before the sorted part");
-    const bool more = s.two_part && s.t_end >= s.bulk_n && s.t_end <= n;
+    const bool more = tail_indexed(s);
     const size_t start = more ? s.t_end : s.bulk_n;
     if (n == start) {  // nothing appended since (e.g. only ionizing collisions)
         if (!more) s.two_part = false;  // the sorted part alone
         return PIC_OK;
     }
-    const size_t words = ((size_t)g.ncells + 2) * 4, iw = (s.cap + 63) / 64 * 64 * 4;
-    if (!s.toff) PIC_HIP(ctx, hipMalloc(&s.toff, words));
-    if (!s.tidx) PIC_HIP(ctx, hipMalloc(&s.tidx, iw));
+    PIC_HIP(ctx, tail_room(g, s));
     PIC_HIP(ctx, hipMemsetAsync(s.count, 0, ((size_t)g.ncells + 1) * 4, ctx->stream));
     const size_t cnt = n - start;
     {
@@ -2135,9 +2160,6 @@ int pic_sort_tail(pic_ctx* ctx, int sid) {
         k_tail_index<<<grid_for(cnt, BLOCK), BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur].cell, s.rank, s.toff,
                                                                      s.d_n, (uint32_t)start, s.tidx);
     } else {
-        if (!s.boff) PIC_HIP(ctx, hipMalloc(&s.boff, words));
-        if (!s.toff_n) PIC_HIP(ctx, hipMalloc(&s.toff_n, words));
-        if (!s.tidx_n) PIC_HIP(ctx, hipMalloc(&s.tidx_n, iw));
         scan_counts(ctx, s, s.boff, false);
         PicProfScope ps(ctx, PIC_K_SCATTER);
         k_tail_merge<<<grid_for((size_t)g.ncells + 2, BLOCK), BLOCK, 0, ctx->stream>>>(

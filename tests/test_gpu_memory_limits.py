@@ -1,0 +1,89 @@
+"""Calls that work faster with memory they can do without, on a GPU that has
+none left: they take their other path and give the same result.  One block
+takes the GPU's free memory but for a rest that the call's buffer does not
+fit in."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ME, QE, AMU, KB = 9.10938215e-31, 1.602176565e-19, 1.660538921e-27, 1.380648e-23
+MB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def pg():
+    import pic_gpu
+
+    return pic_gpu
+
+
+class _Hog:
+    """all of the GPU's free memory but `rest` bytes, through the HIP runtime
+    that the library is linked with"""
+
+    def __init__(self, ctx, rest):
+        self.hip, self.rest = ctx.L, rest  # (its dependencies' names are found through it)
+        self.block = C.c_void_p()
+
+    def __enter__(self):
+        free, total = C.c_size_t(), C.c_size_t()
+        assert self.hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        assert free.value > self.rest
+        assert self.hip.hipMalloc(C.byref(self.block), C.c_size_t(free.value - self.rest)) == 0
+        return self
+
+    def __exit__(self, *a):
+        assert self.hip.hipFree(self.block) == 0
+
+
+def _cells(p, dx, n):
+    c = np.floor(p.reshape(-1, 7)[:, :3] / dx + 1e-9).astype(np.int64)
+    return (c[:, 2] * (n[1] - 1) + c[:, 1]) * (n[0] - 1) + c[:, 0]
+
+
+def _rows(p):
+    p = np.asarray(p).reshape(-1, 7)
+    return p[np.lexsort(p.T)]
+
+
+def test_sort_without_memory_for_the_index(pg, sigma_table_path):
+    """Births behind 1.2M sorted neutrals: pic_sort joins them through an
+    index of 4 bytes per particle of the capacity (1.2 GB here); without room
+    for it the species is sorted whole."""
+    n, dx = (20, 18, 33), 1e-4
+    L = dx * (np.array(n) - 1)
+    box, n_neu, n_ele, cap = 0.98 * L, 1_200_000, 60_000, 300_000_000
+    vol = float(np.prod(box))
+    n_gas = 10.0 / (KB * 300.0)
+    w_n = n_gas * vol / n_neu
+    c = pg.Context(*n, [0, 0, 0], L)
+    c.set_dt(1e-9)
+    sn = c.species_add(32 * AMU, 0.0, w_n, cap)
+    si = c.species_add(32 * AMU, QE, w_n / 1000, n_ele + 200000)
+    se = c.species_add(ME, -QE, w_n / 1000, n_ele + 200000)
+    c.load_box_thermal(sn, 0.5 * L, box, n_gas, 300.0, seed=3, mode=0)
+    c.load_box_thermal(se, 0.5 * L, box, n_ele * w_n / 1000 / vol, 10.0 * 11604.52, seed=4, mode=0)
+    t = np.loadtxt(sigma_table_path)
+    m_red = 32 * AMU * ME / (32 * AMU + ME)
+    wsv = w_n * float(np.max(t[:, 1] * np.sqrt(2.0 * t[:, 0] * QE / m_red)))
+    mid = c.mcc_create(sn, si, se, 12.07 * QE, t[:, 0], t[:, 1], wsv_max_init=wsv)
+    assert c.mcc_apply(mid, 1e-9, 5, 0)["collisions"] > 0
+    num = c.count(sn)
+    assert num > n_neu  # births behind the sorted part
+    with _Hog(c, 600 * MB):
+        c.sort(sn)
+        after = c.download(sn)
+        macro = c.species_field(sn, pg.SFIELD_MACRO_COUNT)
+    cells = _cells(after, dx, n)
+    assert c.count(sn) == num == after.size // 7
+    assert np.all(np.diff(cells) >= 0)
+    assert np.array_equal(macro, np.bincount(cells, minlength=macro.size))
+    # with the memory back, the next births are joined again
+    assert c.mcc_apply(mid, 1e-9, 5, 1)["collisions"] > 0
+    before = c.download(sn)
+    c.sort(sn)
+    assert np.array_equal(_rows(before), _rows(c.download(sn)))
+    c.close()
