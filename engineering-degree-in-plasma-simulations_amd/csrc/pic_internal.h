@@ -175,7 +175,7 @@ struct Species {
     // drifts of at most safe_dtx cells per m/s.  They describe the arrays as
     // that call left them: every call that moves, reorders, adds or changes
     // particles clears safe_ok.
-    uint8_t* safe = nullptr;     // (in rank's block)
+    uint8_t* safe = nullptr;     // null: no memory for them
     float* safe_kick = nullptr;  // device, 3 floats
     bool safe_ok = false;
     float safe_dtx[3] = {0.f, 0.f, 0.f};

@@ -2228,7 +2228,8 @@ extern "C" int pic_push_sort(pic_ctx* ctx, int sid, double dt) {
     // the flags of the last pic_push_sort, if nothing has touched the
     // particles since and the drift per velocity is no larger; the kick's
     // bound is checked on the device
-    const bool flags = a.emax != nullptr && a.s.mode == PIC_SURF_ABSORB;  // this push leaves flags
+    // (this push leaves flags)
+    const bool flags = a.emax != nullptr && a.s.mode == PIC_SURF_ABSORB && s.safe != nullptr;
     bool safe = flags && s.safe_ok;
     for (int d = 0; d < 3; d++) safe = safe && fabsf(a.dtx[d]) <= s.safe_dtx[d];
     s.safe_ok = false;

@@ -1,6 +1,6 @@
 """Calls that work faster with memory they can do without, on a GPU that has
-none left: they take their other path and give the same result.  One block
-takes the GPU's free memory but for a rest that the call's buffer does not
+none left: they take their other path and give the same result.  Blocks
+take the GPU's free memory but for a rest that the call's buffer does not
 fit in."""
 import ctypes as C
 
@@ -25,18 +25,33 @@ class _Hog:
     that the library is linked with"""
 
     def __init__(self, ctx, rest):
-        self.hip, self.rest = ctx.L, rest  # (its dependencies' names are found through it)
-        self.block = C.c_void_p()
+        self.hip, self.rest, self.blocks = ctx.L, rest, []  # (its dependencies' names are found through it)
+
+    def _take(self, size):
+        p = C.c_void_p()
+        if self.hip.hipMalloc(C.byref(p), C.c_size_t(size)):
+            self.hip.hipGetLastError()
+            return None
+        return p
 
     def __enter__(self):
         free, total = C.c_size_t(), C.c_size_t()
         assert self.hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
-        assert free.value > self.rest
-        assert self.hip.hipMalloc(C.byref(self.block), C.c_size_t(free.value - self.rest)) == 0
+        kept = self._take(self.rest)
+        assert kept
+        size = free.value - self.rest
+        while size >= 4 * MB:
+            p = self._take(size)
+            if p:
+                self.blocks.append(p)
+            else:
+                size //= 2
+        assert self.hip.hipFree(kept) == 0
         return self
 
     def __exit__(self, *a):
-        assert self.hip.hipFree(self.block) == 0
+        for p in self.blocks:
+            assert self.hip.hipFree(p) == 0
 
 
 def _cells(p, dx, n):
@@ -51,11 +66,11 @@ def _rows(p):
 
 def test_sort_without_memory_for_the_index(pg, sigma_table_path):
     """Births behind 1.2M sorted neutrals: pic_sort joins them through an
-    index of 4 bytes per particle of the capacity (1.2 GB here); without room
+    index of 4 bytes per particle of the capacity (240 MB here); without room
     for it the species is sorted whole."""
     n, dx = (20, 18, 33), 1e-4
     L = dx * (np.array(n) - 1)
-    box, n_neu, n_ele, cap = 0.98 * L, 1_200_000, 60_000, 300_000_000
+    box, n_neu, n_ele, cap = 0.98 * L, 1_200_000, 60_000, 60_000_000
     vol = float(np.prod(box))
     n_gas = 10.0 / (KB * 300.0)
     w_n = n_gas * vol / n_neu
@@ -73,7 +88,7 @@ def test_sort_without_memory_for_the_index(pg, sigma_table_path):
     assert c.mcc_apply(mid, 1e-9, 5, 0)["collisions"] > 0
     num = c.count(sn)
     assert num > n_neu  # births behind the sorted part
-    with _Hog(c, 600 * MB):
+    with _Hog(c, 128 * MB):
         c.sort(sn)
         after = c.download(sn)
         macro = c.species_field(sn, pg.SFIELD_MACRO_COUNT)
@@ -87,3 +102,35 @@ def test_sort_without_memory_for_the_index(pg, sigma_table_path):
     c.sort(sn)
     assert np.array_equal(_rows(before), _rows(c.download(sn)))
     c.close()
+
+
+def test_species_without_memory_for_the_flags(pg):
+    """pic_push_sort keeps a byte per particle of the capacity (60 MB here)
+    for its next call; a species that there is no room for them for is
+    added all the same and pushed like any other."""
+    n, dx, num = (9, 10, 11), 1e-2, 20_001
+    L = dx * (np.array(n) - 1)
+    rng = np.random.default_rng(7)
+    p = np.zeros((num, 7))
+    p[:, :3] = rng.uniform(0.05, 0.95, (num, 3)) * L
+    p[:, 3:6] = rng.normal(0, 4e3, (num, 3))
+    p[:, 6] = np.arange(num) + 1.0
+    cap = 60_000_000
+    out = []
+    for full in (True, False):
+        c = pg.Context(*n, [0, 0, 0], L)
+        if full:
+            with _Hog(c, int(68.5 * cap)):
+                sid = c.species_add(16 * AMU, QE, 1.0, cap)
+        else:
+            sid = c.species_add(16 * AMU, QE, 1.0, num)
+        c.set_field(pg.FIELD_EF, np.random.default_rng(1).normal(0, 100.0, 3 * c.nn))
+        c.upload(sid, p)
+        c.sort(sid)
+        for _ in range(5):
+            c.push_sort(sid, 2e-8)
+        q = c.download(sid)
+        assert np.all(np.diff(_cells(q, dx, n)) >= 0)
+        out.append(_rows(q))
+        c.close()
+    assert np.array_equal(out[0], out[1])
