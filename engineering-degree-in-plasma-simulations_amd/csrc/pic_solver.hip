@@ -1264,7 +1264,8 @@ constexpr int RUN_AHEAD = 4;
 // host queues the first RUN_AHEAD launches of the sweeps up to the next check
 // before it waits for the last one, and once a check is met the launches
 // behind it return at once (the stop flag), so the potential is the one that
-// was checked.
+// was checked.  Without memory for the second potential and the row bits the
+// sweeps are made in place.
 static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st) {
     if (p->flags & PIC_SOLVE_SOR_PLAIN) return solve_sor_plain(ctx, p, st);
     const GridC& g = ctx->g;
@@ -1273,8 +1274,11 @@ static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats*
     SorArgs a = sor_args(p, s);
     const bool neu = has_neumann(ctx);
     const int check = p->check_every > 0 ? p->check_every : 25;
-    if (!ctx->sor_phi) PIC_HIP(ctx, hipMalloc(&ctx->sor_phi, nn * sizeof(double)));
-    if (!ctx->sor_bits) PIC_HIP(ctx, hipMalloc(&ctx->sor_bits, nn));
+    if ((!ctx->sor_phi && hipMalloc(&ctx->sor_phi, nn * sizeof(double)) != hipSuccess) ||
+        (!ctx->sor_bits && hipMalloc(&ctx->sor_bits, nn) != hipSuccess)) {
+        (void)hipGetLastError();
+        return solve_sor_plain(ctx, p, st);  // in place
+    }
     int rc = pic_ensure_pin(ctx, 8 * sizeof(double));
     if (rc) return rc;
     for (auto& e : ctx->batch_ev)

@@ -134,3 +134,27 @@ def test_species_without_memory_for_the_flags(pg):
         out.append(_rows(q))
         c.close()
     assert np.array_equal(out[0], out[1])
+
+
+def test_sor_without_memory_for_the_second_potential(pg):
+    """The tiled sweeps go from one potential to another (49 MB here); without
+    room for it they are made in place, with the same values."""
+    shape = (190, 180, 180)
+    L = [1e-2 * (n - 1) for n in shape]
+    rng = np.random.default_rng(2)
+    rho = 1e-9 * rng.normal(size=shape[0] * shape[1] * shape[2])
+    out = []
+    for full in (True, False):
+        c = pg.Context(*shape, [0, 0, 0], L)
+        c.add_rectangle([L[0] / 2, L[1] / 2, 0], [1.1 * L[0], 1.1 * L[1], 0.2 * L[2]], 3.0)  # open sides
+        c.set_field(pg.FIELD_RHO, rho)
+        kw = dict(method=pg.SOLVER_SOR_RB, tol=1e-300, tol_kind=pg.TOL_REL, max_it=21, omega=1.7, check_every=8)
+        if full:
+            with _Hog(c, 24 * MB):
+                st = c.poisson(**kw)
+        else:
+            st = c.poisson(**kw)
+        assert st["iterations"] == 21 and not st["converged"]
+        out.append(c.get_field(pg.FIELD_PHI))
+        c.close()
+    assert np.array_equal(out[0], out[1])
