@@ -423,10 +423,10 @@ extern "C" int pic_species_add(pic_ctx* ctx, double mass, double charge, double 
         (void)hipFree(s.den);
         return pic_hip_check(ctx, e, "species allocation");
     }
-    // pic_push_sort's flags and their bound; a species does without where
-    // there is no memory for them
+    // pic_push_sort's flags, their bound and counts; a species does without
+    // where there is no memory for them
     const size_t safe_bytes = (c + 255) / 256 * 256;
-    if (hipMalloc(&s.safe, safe_bytes + 4 * sizeof(float)) == hipSuccess)
+    if (hipMalloc(&s.safe, safe_bytes + 8 * sizeof(float)) == hipSuccess)
         s.safe_kick = reinterpret_cast<float*>(s.safe + safe_bytes);
     else
         (void)hipGetLastError();

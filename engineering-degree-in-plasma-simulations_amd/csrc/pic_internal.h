@@ -176,7 +176,8 @@ struct Species {
     // that call left them: every call that moves, reorders, adds or changes
     // particles clears safe_ok.
     uint8_t* safe = nullptr;     // null: no memory for them
-    float* safe_kick = nullptr;  // device, 3 floats
+    float* safe_kick = nullptr;  // device, 3 floats (-1: no flags left), then two pairs of counts by turns
+    uint32_t safe_calls = 0;
     bool safe_ok = false;
     float safe_dtx[3] = {0.f, 0.f, 0.f};
     double* den = nullptr;       // number density

@@ -102,6 +102,25 @@ struct PushArgs {
     SurfArgs s;
 };
 
+// pic_push_sort's flags for the next one (see k_push and Species).  Leaving
+// them costs k_push_scatter about 3%.  They are of use only to a
+// pic_push_sort that follows with the particles unchanged, and only if nearly
+// all particles have one, since loads are saved line by line.  So a call
+// leaves flags (or kick = -1, which no kick is within) if it is itself such a
+// call (`allow`) and the call before found at most one particle in SAFE_RARE
+// without; every call counts those of every 64th workgroup.  20M particles at
+// 128^3, us per call in a run of calls with flags always, never and by this rule:
+// ions, which hardly move, 373, 433, 374; electrons of which 3% may leave 509,
+// 512, 510; with steps 10 and 50 times as long 749, 727, 727 and 1042, 1006, 1007.
+struct SafeArgs {
+    uint8_t* flags;  // null: none
+    float* kick;     // the kick that they hold for, 3 floats
+    const uint32_t* prev;  // counted by the call before: particles that may leave, particles
+    uint32_t* next;        // counted by this call
+    int allow;
+};
+constexpr uint32_t SAFE_RARE = 32;
+
 // A particle whose drift cannot take it out of its cell, whatever E it
 // gathers: for every axis |f' - f| <= (|v| + |qm dt| max|E|) dt/dx (with
 // margins for the FP32 rounding of the kick, the interpolation and the
@@ -424,16 +443,14 @@ constexpr int PUSH_SORT_ILP = 2;
 // k_push_scatter that ordered them, for those that cannot leave their cell
 // under a kick of safe_kick.  While the largest kick is within that, such a
 // particle's key is its cell word: nothing else of it is read (5 bytes
-// instead of 28).  20M particles at 128^3, without and with: ions, which hardly
-// move, 134 and 60 us (then the runs' atomics bound it), electrons, a few per
-// cent of which may leave, 170 and 158; writing the byte costs
-// k_push_scatter 10 of 289 us.  200M ions at 256^3: 1245 and 609 us.
+// instead of 28).  The flags are left where they pay (SafeArgs).
 template <bool WRITE, int ILP, bool SURF>
 __global__ void __launch_bounds__(BLOCK)
     k_push(GridC g, SpeciesBuf b, const float4* __restrict__ E, PushArgs a,
            uint32_t* __restrict__ d_n, uint32_t* __restrict__ count, uint32_t* __restrict__ rank,
-           const uint8_t* __restrict__ safe, const float* __restrict__ safe_kick) {
+           const uint8_t* __restrict__ safe, SafeArgs sa) {
     const size_t p0 = xcd_wg() * (BLOCK * ILP) + threadIdx.x;
+    if (!WRITE && !SURF && sa.flags && p0 < 2) sa.next[p0] = 0;  // for the k_push_scatter that follows
     uint32_t n = d_n[0];
     uint32_t covered = gridDim.x * BLOCK * ILP;
     if (n > covered) n = covered;
@@ -446,8 +463,8 @@ __global__ void __launch_bounds__(BLOCK)
     if (bound && a.kick)
 #pragma unroll
         for (int d = 0; d < 3; d++) kick[d] = fabsf(a.qmdt) * a.emax[d];
-    const bool use_safe = bound && safe != nullptr && kick[0] <= safe_kick[0] && kick[1] <= safe_kick[1] &&
-                          kick[2] <= safe_kick[2];  // (the whole grid; false for NaN)
+    const bool use_safe = bound && safe != nullptr && kick[0] <= sa.kick[0] && kick[1] <= sa.kick[1] &&
+                          kick[2] <= sa.kick[2];  // (the whole grid; false for NaN)
     uint8_t stay[ILP];
 #pragma unroll
     for (int q = 0; q < ILP; q++) {
@@ -1058,16 +1075,18 @@ template <bool SURF, int ILP>
 __global__ void __launch_bounds__(BLOCK)
     k_push_scatter(GridC g, SpeciesBuf src, SpeciesBuf dst, const float4* __restrict__ E, PushArgs a,
                    const uint32_t* __restrict__ bases, const uint32_t* __restrict__ off,
-                   const uint32_t* __restrict__ d_n, uint32_t cap, uint8_t* __restrict__ safe,
-                   float* __restrict__ safe_kick) {
-    const size_t p0 = xcd_wg() * (BLOCK * ILP) + threadIdx.x;
-    // the next push's flags, for a field that at most doubles (see k_push)
+                   const uint32_t* __restrict__ d_n, uint32_t cap, SafeArgs sa) {
+    const size_t wg = xcd_wg(), p0 = wg * (BLOCK * ILP) + threadIdx.x;
+    // the next push's flags, for a field that at most doubles
+    const bool count = !SURF && sa.flags != nullptr && (wg & 63) == 0;                               // (the workgroup)
+    const bool leave = !SURF && sa.flags != nullptr && sa.allow && sa.prev[0] * SAFE_RARE <= sa.prev[1];  // (the grid)
     float kick2[3] = {0.f, 0.f, 0.f};
-    if (!SURF && safe) {
+    uint32_t may_leave = 0, counted = 0;
+    if (count || leave) {
         if (a.kick)
 #pragma unroll
             for (int d = 0; d < 3; d++) kick2[d] = 2.f * fabsf(a.qmdt) * a.emax[d];
-        if (p0 < 3) safe_kick[p0] = p0 == 0 ? kick2[0] : p0 == 1 ? kick2[1] : kick2[2];
+        if (p0 < 3) sa.kick[p0] = !leave ? -1.f : p0 == 0 ? kick2[0] : p0 == 1 ? kick2[1] : kick2[2];
     }
     const uint32_t n = d_n[1];
     uint32_t c[ILP];
@@ -1115,7 +1134,22 @@ __global__ void __launch_bounds__(BLOCK)
             dst.v[d][dst_i] = v[q][d];
         }
         dst.w[dst_i] = w[q];
-        if (!SURF && safe) safe[dst_i] = stays_in_cell(f[q], v[q], kick2, a.dtx) ? 1 : 0;
+        if (count || leave) {
+            const bool stay = stays_in_cell(f[q], v[q], kick2, a.dtx);
+            if (leave) sa.flags[dst_i] = stay ? 1 : 0;
+            may_leave += stay ? 0 : 1;
+            counted++;
+        }
+    }
+    if (count) {
+        for (int o = 32; o > 0; o >>= 1) {
+            may_leave += __shfl_xor(may_leave, o, 64);
+            counted += __shfl_xor(counted, o, 64);
+        }
+        if ((threadIdx.x & 63) == 0) {
+            atomicAdd(&sa.next[0], may_leave);
+            atomicAdd(&sa.next[1], counted);
+        }
     }
 }
 
@@ -1916,10 +1950,10 @@ extern "C" int pic_push(pic_ctx* ctx, int sid, double dt) {
         const unsigned nb = xcd_blocks1(n, BLOCK * PUSH_ILP);
         if (a.s.mode == PIC_SURF_ABSORB)
             k_push<true, PUSH_ILP, false><<<nb, BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], ctx->ef, a, s.d_n,
-                                                                         s.count, s.rank, nullptr, nullptr);
+                                                                         s.count, s.rank, nullptr, SafeArgs{});
         else
             k_push<true, PUSH_ILP, true><<<nb, BLOCK, 0, ctx->stream>>>(g, s.buf[s.cur], ctx->ef, a, s.d_n,
-                                                                        s.count, s.rank, nullptr, nullptr);
+                                                                        s.count, s.rank, nullptr, SafeArgs{});
     }
     PIC_HIP(ctx, hipGetLastError());
     s.hist_valid = true;
@@ -2228,9 +2262,14 @@ extern "C" int pic_push_sort(pic_ctx* ctx, int sid, double dt) {
     // the flags of the last pic_push_sort, if nothing has touched the
     // particles since and the drift per velocity is no larger; the kick's
     // bound is checked on the device
-    // (this push leaves flags)
     const bool flags = a.emax != nullptr && a.s.mode == PIC_SURF_ABSORB && s.safe != nullptr;
     bool safe = flags && s.safe_ok;
+    SafeArgs sa{};
+    if (flags) {
+        uint32_t* stat = reinterpret_cast<uint32_t*>(s.safe_kick + 4);
+        sa = SafeArgs{s.safe, s.safe_kick, stat + 2 * (s.safe_calls & 1), stat + 2 * (~s.safe_calls & 1), s.safe_ok};
+        s.safe_calls++;
+    }
     for (int d = 0; d < 3; d++) safe = safe && fabsf(a.dtx[d]) <= s.safe_dtx[d];
     s.safe_ok = false;
     PIC_HIP(ctx, hipMemsetAsync(s.count, 0, ((size_t)g.ncells + 1) * 4, ctx->stream));
@@ -2239,10 +2278,10 @@ extern "C" int pic_push_sort(pic_ctx* ctx, int sid, double dt) {
         const unsigned nb = xcd_blocks1(n, BLOCK * PUSH_SORT_ILP);
         if (a.s.mode == PIC_SURF_ABSORB)
             k_push<false, PUSH_SORT_ILP, false><<<nb, BLOCK, 0, ctx->stream>>>(
-                g, s.buf[s.cur], ctx->ef, a, s.d_n, s.count, s.rank, safe ? s.safe : nullptr, s.safe_kick);
+                g, s.buf[s.cur], ctx->ef, a, s.d_n, s.count, s.rank, safe ? s.safe : nullptr, sa);
         else
             k_push<false, PUSH_SORT_ILP, true><<<nb, BLOCK, 0, ctx->stream>>>(
-                g, s.buf[s.cur], ctx->ef, a, s.d_n, s.count, s.rank, nullptr, nullptr);
+                g, s.buf[s.cur], ctx->ef, a, s.d_n, s.count, s.rank, nullptr, SafeArgs{});
     }
     scan_counts(ctx, s, s.off, true);
     a.s.emit = 1;
@@ -2251,12 +2290,10 @@ extern "C" int pic_push_sort(pic_ctx* ctx, int sid, double dt) {
         const unsigned nb2 = xcd_blocks1(n, BLOCK * PUSH_SCATTER_ILP);
         if (a.s.mode == PIC_SURF_ABSORB)
             k_push_scatter<false, PUSH_SCATTER_ILP><<<nb2, BLOCK, 0, ctx->stream>>>(
-                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap,
-                flags ? s.safe : nullptr, s.safe_kick);
+                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap, sa);
         else
             k_push_scatter<true, 1><<<xcd_blocks1(n, BLOCK), BLOCK, 0, ctx->stream>>>(
-                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap, nullptr,
-                nullptr);
+                g, s.buf[s.cur], s.buf[s.cur ^ 1], ctx->ef, a, s.rank, s.off, s.d_n, (uint32_t)s.cap, sa);
     }
     PIC_HIP(ctx, hipGetLastError());
     s.safe_ok = flags;

@@ -215,6 +215,72 @@ def test_push_sort_flags_after_collisions_and_sources(pg):
     c.close()
 
 
+def _in_cell_order(pg, c, sid, dx, n):
+    r = c.download(sid)
+    cells = _cells(r, dx, n)
+    assert np.all(np.diff(cells) >= 0)
+    macro = c.species_field(sid, pg.SFIELD_MACRO_COUNT)
+    assert np.array_equal(macro, np.bincount(cells, minlength=macro.size))
+    return r.size // 7
+
+
+def test_push_sort_flags_after_merges(pg):
+    """Three pic_push_sort in a row (the second leaves flags, of 99% of the
+    particles, and the third uses them), then a merge, which moves particles
+    to other members' places and velocities: the next ones sort by where the
+    particles really go."""
+    n, dx = (9, 10, 11), 1e-2
+    c, sid, _ = _charged(pg, 200_000, 16 * AMU, QE, 5)
+    left = 200_000
+    for step in range(4):
+        for _ in range(3):
+            c.push_sort(sid, 1e-9)  # 0.03% of a cell
+            left = _in_cell_order(pg, c, sid, dx, n)
+        st = c.merge(sid, seed=step)
+        assert st["removed"] > 1000 or step
+        assert _in_cell_order(pg, c, sid, dx, n) == left - st["removed"]
+        c.push_sort(sid, 1e-9)
+        _in_cell_order(pg, c, sid, dx, n)
+    c.close()
+
+
+def test_push_sort_flags_after_mcc_steps(pg, sigma_table_path):
+    """The same with MC_MEX steps in a box without objects: the collisions turn
+    electrons and neutrals and append others."""
+    c, sn, si, se, mid, dx, n = _gas(pg, sigma_table_path, 1e-9, 300_000, 60_000)
+    for step in range(4):
+        for sid, dt in ((se, 2e-13), (sn, 5e-10), (si, 5e-10)):
+            for _ in range(3):
+                c.push_sort(sid, dt)
+                _in_cell_order(pg, c, sid, dx, n)
+        st = c.mcc_apply(mid, 1e-9, 5, step)
+        assert st["collisions"] > 1000 and st["ionizations"] > 0
+    c.close()
+
+
+def test_push_sort_rule_for_flags_in_a_changing_run(pg):
+    """Steps that change between those that nearly no particle leaves its cell
+    in and those that most do, so that flags are left, left out and left
+    again, against pic_push + pic_sort."""
+    chains = [_charged(pg, 60_001, 16 * AMU, QE, 11) for _ in range(2)]
+    for _, (c, sid, ef) in zip(range(2), chains):
+        c.set_field(pg.FIELD_EF, ef)
+    for k, dt in enumerate([1e-10] * 4 + [2e-6] * 3 + [1e-10] * 4 + [2e-6, 1e-10, 1e-10, 1e-10]):
+        rows = []
+        for fused, (c, sid, _) in zip((True, False), chains):
+            if fused:
+                c.push_sort(sid, dt)
+            else:
+                c.push(sid, dt)
+                c.sort(sid)
+            _in_cell_order(pg, c, sid, 1e-2, (9, 10, 11))
+            rows.append(_rows(c.download(sid)))
+        assert np.array_equal(rows[0], rows[1]), k
+    assert len(rows[0]) > 100
+    for c, _, _ in chains:
+        c.close()
+
+
 @pytest.mark.parametrize("num", [0, 1, (1 << 20) - 1, 1 << 20, (1 << 20) + 3])
 def test_upload_in_pieces(pg, num):
     """uploads of no, one, and just below and above one staging piece"""
