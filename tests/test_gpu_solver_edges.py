@@ -154,3 +154,42 @@ def test_long_check_interval_costs_nothing_after_convergence(pg):
         best[check] = min(best.get(check, 1.0), st["seconds"])
     assert best[4000] < 2 * best[25] + 2e-4, best
     c.close()
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (3, 9, 5), (12, 3, 4), (5, 4, 3), (17, 11, 13)])
+@pytest.mark.parametrize("objects", [0, 1, 3])
+def test_row_types_of_open_boxes(pg, shape, objects):
+    """The operator's row of every node (Dirichlet in objects and on flagged
+    nodes; a Neumann face copies its neighbour along the first axis it is an end
+    of; regular inside): a face node's value after one sweep is that of the node
+    its row names, for boxes with open sides and objects on faces and edges."""
+    L = np.array([1e-2 * (n - 1) for n in shape])
+    c = pg.Context(*shape, [0, 0, 0], L)
+    rng = np.random.default_rng(sum(shape) + objects)
+    for q in range(objects):
+        c.add_rectangle([L, 0 * L, 0.5 * L][q], 0.6 * L, float(q + 1))
+    rho = 1e-9 * rng.normal(size=int(np.prod(shape)))
+    c.set_field(pg.FIELD_RHO, rho)
+    oid, _ = c.node_flags()
+    phi0 = c.get_field(pg.FIELD_PHI)
+    phi0[oid == 0] = rng.normal(size=int(np.sum(oid == 0)))
+    c.set_field(pg.FIELD_PHI, phi0)
+    c.poisson(pg.SOLVER_SOR_RB, tol=1e-300, tol_kind=pg.TOL_REL, max_it=1, omega=1.3)
+    phi = c.get_field(pg.FIELD_PHI).reshape(shape[::-1])
+    oid = oid.reshape(shape[::-1])
+    old = phi0.reshape(shape[::-1])
+    n = shape[::-1]  # index order k, j, i
+    for k in range(n[0]):
+        for j in range(n[1]):
+            for i in range(n[2]):
+                at = [k, j, i]
+                if oid[k, j, i] > 0:
+                    assert phi[k, j, i] == old[k, j, i]
+                    continue
+                axis = next((d for d in (2, 1, 0) if at[d] in (0, n[d] - 1)), None)
+                if axis is not None:
+                    at[axis] += 1 if at[axis] == 0 else -1
+                    assert phi[k, j, i] == phi[tuple(at)], (k, j, i)
+                else:
+                    assert phi[k, j, i] != old[k, j, i]
+    c.close()
