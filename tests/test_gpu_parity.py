@@ -390,10 +390,10 @@ def test_sor_dirichlet_matches_oracle(pg, golden):
 
 @pytest.mark.parametrize("shape,n0", [((67, 45, 37), 0.0), ((130, 33, 29), 1e10)])
 def test_split_sor_sweeps_equal_plain(pg, shape, n0):
-    """The sweeps on the red-black split layout (default without Neumann
-    faces) against the natural layout's (PIC_SOLVE_SOR_PLAIN): the same
-    potential bit for bit after 37 sweeps, on grids of odd and even ni, with
-    two objects and, in the second case, the Boltzmann term."""
+    """The default sweeps (on tiles, two per launch) against one launch per
+    colour (PIC_SOLVE_SOR_PLAIN): the same potential bit for bit after 37
+    sweeps, on grids of odd and even ni, with two objects and, in the second
+    case, the Boltzmann term."""
     ni, nj, nk = shape
     L = [1e-2 * (ni - 1), 1e-2 * (nj - 1), 1e-2 * (nk - 1)]
     rng = np.random.default_rng(ni)
@@ -414,7 +414,7 @@ def test_split_sor_sweeps_equal_plain(pg, shape, n0):
         c.close()
     assert np.all(np.isfinite(out[0][0]))
     assert np.array_equal(out[0][0], out[1][0])
-    # the residual's striped sums add in no fixed order
+    # the residual's partial sums are added in another order
     assert out[0][1] == pytest.approx(out[1][1], rel=1e-12)
 
 

@@ -82,15 +82,36 @@ def test_boltzmann_pcg_with_neumann_sides_matches_oracle(pg, shape, method, tol)
     c.close()
 
 
-@pytest.mark.parametrize("shape", [(3, 3, 3), (4, 3, 5), (17, 16, 15), (31, 33, 32), (65, 41, 29), (70, 71, 72),
-                                   (128, 30, 90)])
-@pytest.mark.parametrize("sides", ["walls", "neumann"])
+SMALL, LINES, SQUARE = (32, 16, 12), (64, 16, 16), (32, 32, 16)  # nodes of the SOR tiles
+
+
+def _sor_tile(shape, neumann):
+    """the tile that the sweeps of a grid are made on (the solver's rule)"""
+    def tiles(t):  # cores of t - 8 nodes, and four more at the ends
+        return np.prod([next(m for m in range(1, 999) if (m - 1) * (e - 8) + e >= n) for n, e in zip(shape, t)])
+
+    if tiles(SMALL) <= 400:
+        return SMALL
+    return LINES if neumann or tiles(LINES) < tiles(SQUARE) else SQUARE
+
+
+@pytest.mark.parametrize("shape,tile,sides", [
+    ((3, 3, 3), SMALL, "walls"), ((3, 3, 3), SMALL, "neumann"), ((4, 3, 5), SMALL, "walls"), ((4, 3, 5), SMALL, "neumann"),
+    ((17, 16, 15), SMALL, "walls"), ((17, 16, 15), SMALL, "neumann"), ((31, 33, 32), SMALL, "walls"),
+    ((31, 33, 32), SMALL, "neumann"), ((65, 41, 29), SMALL, "walls"), ((65, 41, 29), SMALL, "neumann"),
+    ((70, 71, 72), SMALL, "walls"), ((70, 71, 72), SMALL, "neumann"), ((128, 30, 90), SMALL, "walls"),
+    ((128, 30, 90), SMALL, "neumann"),
+    ((100, 81, 67), SQUARE, "walls"), ((100, 81, 67), LINES, "neumann"), ((128, 65, 64), SQUARE, "walls"),
+    ((128, 65, 64), LINES, "neumann"), ((33, 130, 140), SQUARE, "walls"), ((33, 130, 140), LINES, "neumann"),
+    ((63, 64, 101), LINES, "walls"), ((63, 64, 101), LINES, "neumann"), ((61, 106, 51), LINES, "walls")])
 @pytest.mark.parametrize("n0", [0.0, 1e10])
-def test_tiled_sor_sweeps_equal_plain(pg, shape, sides, n0):
+def test_tiled_sor_sweeps_equal_plain(pg, shape, tile, sides, n0):
     """The tiled sweeps against one launch per colour (PIC_SOLVE_SOR_PLAIN),
     bit for bit, after an odd and an even number of sweeps and with a check
     in between: grids smaller than a tile, with cores that end inside a node
-    pair, and of each tile's size; objects on faces, edges and inside."""
+    pair, and of several tiles of each of the three kinds, with ragged ends;
+    objects on faces, edges and inside."""
+    assert _sor_tile(shape, sides == "neumann") == tile
     L = [1e-2 * (n - 1) for n in shape]
     rng = np.random.default_rng(shape[0])
     rho = 1e-9 * rng.normal(size=shape[0] * shape[1] * shape[2])
