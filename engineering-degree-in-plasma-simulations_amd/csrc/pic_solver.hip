@@ -1,58 +1,14 @@
-// pic_solver.hip -- field solve of the gfx950 PIC library.
+// pic_solver.hip -- field solve of the gfx950 PIC library: the entry point, the
+// E-field and the learned solver (pic_sor.hip and pic_pcg.hip: the others).
 //
 //   k_efield     E = -grad(phi), FP64 math, FP32 float4 output
 //                (PotentialSolver.cpp:354-408)
-//   k_sor_tile   red-black SOR with the Boltzmann electron term
-//                (PotentialSolver.cpp:69-166; ch2/v1/PotentialSolver.cpp:8-87),
-//                two sweeps per launch on tiles; k_sor: one colour per launch
-//   k_neumann    Neumann face copies (PotentialSolver.cpp:96-107)
-//   k_F          Newton residual F = A phi - b - q n0 e^{(phi-phi0)/Te0}/eps0
-//                and the Jacobian diagonal shift (PotentialSolver.cpp:189-217)
-//   k_pcg1/2     matrix-free Jacobi PCG (PotentialSolver.cpp:243-313), two
-//                fused kernels per iteration, scalars kept on the device
-//
-// The operator rows follow PotentialSolver::buildMatrix
-// (PotentialSolver.cpp:414-471): Dirichlet rows are the identity, Neumann face
-// rows are one-sided (1/dx)(phi_u - phi_nbr), regular rows are the 7-point
-// Laplacian.  Jacobi M = 1/diag(A) of that operator (PotentialSolver.cpp:470).
-//
-// All stencil kernels walk the grid in contiguous chunks per workgroup and
-// map consecutive chunks to the same XCD (workgroups are dealt round-robin
-// over the 8 XCDs), so k-neighbour planes are reused from that XCD's L2.
-#include <algorithm>
-#include <cmath>
-#include <type_traits>
-#include <utility>
+//   k_fcg_*      flexible CG with the learned two-level preconditioner
 #include <vector>
 
-#include "pic_internal.h"
-
-using namespace pic;
+#include "pic_stencil.h"
 
 namespace {
-
-constexpr int BLOCK = 256;
-constexpr int NXCD = 8;
-
-struct Stencil {
-    double cx, cy, cz, twos;  // +-1, +-ni, +-ni*nj coefficients; 2(sum 1/dx^2)
-    double itwos;             // 1 / twos
-    double idx[3];            // 1/dx per axis (Neumann rows)
-    long long sj, sk, nn;
-    int ni, nj, nk;
-};
-
-// gridDim.x is a multiple of NXCD (stencil_blocks), so lb is a bijection
-__device__ inline long long chunk_begin(long long nn, long long& end) {
-    int nb = gridDim.x;
-    int b = blockIdx.x;
-    int per_xcd = nb / NXCD;
-    int lb = (b % NXCD) * per_xcd + b / NXCD;  // logical, XCD-contiguous
-    long long chunk = ((nn + nb - 1) / nb + BLOCK - 1) / BLOCK * BLOCK;
-    long long beg = (long long)lb * chunk;
-    end = beg + chunk < nn ? beg + chunk : nn;
-    return beg;
-}
 
 // Node pairs (2h, 2h+1) of every i-line, XCD-contiguous chunks per
 // workgroup: f(u, second, red) for the pair's first node u, whether the
@@ -74,59 +30,6 @@ __device__ inline void for_pairs(const Stencil& s, F f) {
         unsigned u = row * (unsigned)s.ni + 2 * h;
         f(u, 2 * h + 1 < (unsigned)s.ni, ((j + k) & 1u) == 0);
     }
-}
-
-__device__ inline double block_sum(double v) {
-    __shared__ double red[BLOCK / 64];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double t = 0;
-    if (threadIdx.x == 0)
-        for (int w = 0; w < BLOCK / 64; w++) t += red[w];
-    __syncthreads();
-    return t;  // valid in thread 0
-}
-
-template <typename T>
-__device__ inline T nbr_of(uint8_t t, const T* v, long long u, const Stencil& s) {
-    switch (t) {
-        case NT_NEU_IM: return v[u + 1];
-        case NT_NEU_IP: return v[u - 1];
-        case NT_NEU_JM: return v[u + s.sj];
-        case NT_NEU_JP: return v[u - s.sj];
-        case NT_NEU_KM: return v[u + s.sk];
-        default: return v[u - s.sk];
-    }
-}
-__device__ inline double neu_coef(uint8_t t, const Stencil& s) {
-    return t <= NT_NEU_IP ? s.idx[0] : (t <= NT_NEU_JP ? s.idx[1] : s.idx[2]);
-}
-// diag(A) for the Jacobi preconditioner
-__device__ inline double diagA(uint8_t t, const Stencil& s) {
-    if (t == NT_REG) return -s.twos;
-    if (t == NT_DIR) return 1.0;
-    return neu_coef(t, s);
-}
-
-// (A v)_u for a vector given as a functor of the node index
-template <typename T, typename F>
-__device__ inline T apply_A(uint8_t t, long long u, const Stencil& s, F v) {
-    T vu = v(u);
-    if (t == NT_REG)
-        return (T)s.cz * (v(u - s.sk) + v(u + s.sk)) + (T)s.cy * (v(u - s.sj) + v(u + s.sj)) +
-               (T)s.cx * (v(u - 1) + v(u + 1)) - (T)s.twos * vu;
-    if (t == NT_DIR) return vu;
-    long long o;
-    switch (t) {
-        case NT_NEU_IM: o = 1; break;
-        case NT_NEU_IP: o = -1; break;
-        case NT_NEU_JM: o = s.sj; break;
-        case NT_NEU_JP: o = -s.sj; break;
-        case NT_NEU_KM: o = s.sk; break;
-        default: o = -s.sk; break;
-    }
-    return (T)neu_coef(t, s) * (vu - v(u + o));
 }
 
 // ------------------------------------------------------------------------
@@ -180,918 +83,12 @@ __global__ void __launch_bounds__(BLOCK)
     }
 }
 
-// ------------------------------------------------------------------------
-// red-black SOR
-// ------------------------------------------------------------------------
-struct SorArgs {
-    double omega, ieps, itwos, phi0, n0, inv_te0;
-    int color;
-};
-
-// The SOR update of a regular node from its neighbour sums along each axis
-// (shared by both sweep kernels, rounded the same way: no contraction).
-template <bool BOLTZ>
-__device__ inline double sor_node(const Stencil& s, const SorArgs& a, double p, double rho_u, double sx,
-                                  double sy, double sz) {
-#pragma clang fp contract(off)
-    double q = rho_u;
-    if (BOLTZ) q -= QE * (a.n0 * exp((p - a.phi0) * a.inv_te0));
-    const double nw = (q * a.ieps + sx * s.cx + sy * s.cy + sz * s.cz) * a.itwos;
-    return p + a.omega * (nw - p);
-}
-
-__global__ void __launch_bounds__(BLOCK)
-    k_sor(Stencil s, SorArgs a, const uint8_t* __restrict__ nt, double* __restrict__ phi,
-          const double* __restrict__ rho) {
-    long long half = (s.ni + 1) / 2;
-    long long items = half * s.nj * s.nk;
-    long long end;
-    for (long long m = chunk_begin(items, end) + threadIdx.x; m < end; m += BLOCK) {
-        unsigned row = (unsigned)m / (unsigned)half;
-        int h = (int)((unsigned)m - row * (unsigned)half);
-        unsigned kk = row / (unsigned)s.nj;
-        int j = (int)(row - kk * (unsigned)s.nj), k = (int)kk;
-        int i = 2 * h + ((j + k + a.color) & 1);
-        if (i >= s.ni) continue;
-        long long u = row * s.ni + i;
-        if (nt[u] != NT_REG) continue;
-        const double sx = phi[u - 1] + phi[u + 1], sy = phi[u - s.sj] + phi[u + s.sj], sz = phi[u - s.sk] + phi[u + s.sk];
-        phi[u] = a.n0 != 0.0 ? sor_node<true>(s, a, phi[u], rho[u], sx, sy, sz)
-                             : sor_node<false>(s, a, phi[u], rho[u], sx, sy, sz);
-    }
-}
-
-// ---- tiled sweeps: several half sweeps per launch ----
-// A launch per colour is bound by its launch: a half sweep of a 64 x 64 x 256
-// grid took 6.9 us (4.1 us at 32^3, an empty launch's time).  k_sor_tile
-// therefore keeps a tile of the potential on chip and makes up to SOR_HALO
-// half sweeps on it.  The tile's core is what it writes; around it lie
-// SOR_HALO more nodes in every direction, because half sweep q + 1 of a node
-// needs its neighbours after half sweep q: what a half sweep computes is right
-// for nodes at least q + 1 from the tile's edge, so the core is right after
-// SOR_HALO of them.  Nodes nearer the edge hold values that nothing correct
-// reads.  Where the tile ends at the grid's end there is no halo (face nodes
-// are not updated).  The potential goes from one buffer to another, since
-// neighbouring tiles read each other's cores.
-//
-// A thread owns the node pair (2h, 2h + 1) of one j-line of the tile for all
-// TK planes, in registers with their charge density and row bits; one of the
-// two is red, by the plane's parity.  A wave's j-lines all have the same
-// parity, so which one it is is a constant of the wave and the code has no
-// selection.  A node's neighbours along k and one of those along i are the
-// thread's own; the other three come from LDS, which holds the first and the
-// second nodes as [plane][j][pair] (consecutive lanes read consecutive
-// words).  The update is sor_node on the same operands as k_sor's (a sum of
-// two neighbours does not depend on their order), so every value equals
-// k_sor's bit for bit.
-//
-// Row bits of a node: SOR_REG, and for each neighbour whether it is a Neumann
-// face.  Such a face holds a copy of the node next to it from the end of the
-// previous sweep (k_neumann), which is the value the node still has when its
-// own turn comes, so from the second sweep on (own) the node's value stands
-// in for the face's and no copies are made between sweeps.
-constexpr int SOR_HALO = 4;
-enum : unsigned { SOR_REG = 1, SOR_IM = 2, SOR_IP = 4, SOR_JM = 8, SOR_JP = 16, SOR_KM = 32, SOR_KP = 64 };
-
-__global__ void __launch_bounds__(BLOCK)
-    k_sor_bits(Stencil s, const uint8_t* __restrict__ nt, uint8_t* __restrict__ bits) {
-    long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        unsigned m = 0;
-        if (nt[u] == NT_REG) {  // an interior node
-            auto neu = [&](long long v) { return nt[v] != NT_REG && nt[v] != NT_DIR; };
-            m = SOR_REG | (neu(u - 1) ? SOR_IM : 0) | (neu(u + 1) ? SOR_IP : 0) | (neu(u - s.sj) ? SOR_JM : 0) |
-                (neu(u + s.sj) ? SOR_JP : 0) | (neu(u - s.sk) ? SOR_KM : 0) | (neu(u + s.sk) ? SOR_KP : 0);
-        }
-        bits[u] = (uint8_t)m;
-    }
-}
-
-// One axis of the tiling: a grid of n nodes in m tiles of t nodes
-struct TileAxis {
-    int n, t, m;
-    __host__ __device__ int start(int q) const {  // even, and the last tile reaches the grid's end
-        if (q == 0) return 0;
-        const int b = q * (t - 2 * SOR_HALO), e = (n - t + 1) & ~1;
-        return b < e ? b : e;
-    }
-    __host__ __device__ int core(int q) const {  // the first node tile q writes; core(m) = n
-        return q == 0 ? 0 : (q == m ? n : q * (t - 2 * SOR_HALO) + SOR_HALO);
-    }
-};
-TileAxis tile_axis(int n, int t) {
-    TileAxis a{n, t, 1};
-    while ((a.m - 1) * (t - 2 * SOR_HALO) + t < n) a.m++;
-    return a;
-}
-
-// f(1), ..., f(n) with constant arguments, K = 0 .. n - 1
-template <typename F, int... K>
-__device__ __attribute__((always_inline)) inline void for_planes(F f, std::integer_sequence<int, K...>) {
-    (f(std::integral_constant<int, K + 1>{}), ...);
-}
-
-template <int PI, int TJ, int TK, bool NEU, bool BOLTZ>
-__global__ void __launch_bounds__(PI* TJ)
-    k_sor_tile(Stencil s, SorArgs a, TileAxis ax, TileAxis ay, TileAxis az, const uint8_t* __restrict__ bits,
-               const double* __restrict__ in, double* __restrict__ out, const double* __restrict__ rho, int ns,
-               int own, const double* __restrict__ stop) {
-    constexpr int NT = PI * TJ, LINES = 64 / PI;  // j-lines of a wave
-    static_assert(NT % 128 == 0 && TJ % (2 * LINES) == 0, "waves of one parity");
-    __shared__ double lds[2][TK][NT];  // [first or second node][plane][j, pair]
-    if (*stop != 0.0) return;          // (the whole grid)
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int h = lane % PI;
-    const int jl = (wave & 1) + 2 * (LINES * (wave >> 1) + lane / PI);  // the wave's lines: every second one
-    const int tid = jl * PI + h;
-    const unsigned b = (unsigned)xcd_wg();
-    const int bx = (int)(b % (unsigned)ax.m), by = (int)(b / (unsigned)ax.m % (unsigned)ay.m),
-              bz = (int)(b / (unsigned)(ax.m * ay.m));
-    if (bz >= az.m) return;  // (the whole workgroup)
-    const int i0 = ax.start(bx), j0 = ay.start(by), k0 = az.start(bz);
-    const int i = i0 + 2 * h, j = j0 + jl;
-    const bool in1 = i < s.ni && j < s.nj, in2 = i + 1 < s.ni && j < s.nj;
-    const unsigned ub = ((unsigned)k0 * (unsigned)s.nj + (unsigned)j) * (unsigned)s.ni + (unsigned)i;
-    const unsigned sk = (unsigned)s.sk;
-    // Every load before any use, without branches: clamped addresses (a node
-    // beyond the grid gets some other node's values and no row bits).
-    typedef double D2 __attribute__((ext_vector_type(2), aligned(8)));
-    const unsigned top = (unsigned)s.nn - 2u;
-    D2 P[TK], R[TK];
-    unsigned m[TK];  // row bits: first | second << 8
-#pragma unroll
-    for (int k = 0; k < TK; k++) {
-        const unsigned u = ub + (unsigned)k * sk, v = u < top ? u : top;
-        P[k] = *reinterpret_cast<const D2*>(in + v);
-        R[k] = *reinterpret_cast<const D2*>(rho + v);
-        uint16_t w;
-        __builtin_memcpy(&w, bits + v, 2);
-        m[k] = w;
-    }
-    const unsigned keep = (in1 ? 0xFFu : 0u) | (in2 ? 0xFF00u : 0u);
-#pragma unroll
-    for (int k = 0; k < TK; k++) {
-        if (ub + (unsigned)k * sk == top + 1u) {  // the grid's last node: the second of the clamped pair
-            P[k][0] = P[k][1];
-            m[k] = 0;
-        }
-        m[k] = k0 + k < s.nk ? m[k] & keep : 0u;
-        lds[0][k][tid] = P[k][0];
-        lds[1][k][tid] = P[k][1];
-    }
-    __syncthreads();
-    // LDS places of the neighbours (a place beyond the tile: the thread's own,
-    // read only for nodes whose value nothing correct reads)
-    const int qm = h > 0 ? tid - 1 : tid, qp = h < PI - 1 ? tid + 1 : tid;
-    const int jm = jl > 0 ? tid - PI : tid, jp = jl < TJ - 1 ? tid + PI : tid;
-    const bool jlo = j0 == 0, jhi = j0 + TJ >= s.nj, klo = k0 == 0, khi = k0 + TK >= s.nk;
-    // one node of plane k: the pair's node e
-    auto node = [&](auto kc, auto ec, bool fresh) __attribute__((always_inline)) {
-        constexpr int k = decltype(kc)::value, e = decltype(ec)::value;
-        const double p = P[k][e];
-        double w = P[k][1 - e], wl = P[k - 1][e], wh = P[k + 1][e];
-        double q = lds[1 - e][k][e ? qp : qm], yl = lds[e][k][jm], yh = lds[e][k][jp];
-        const unsigned mb = m[k] >> (8 * e);
-        if (NEU && fresh) {
-            unsigned nb = mb;
-            // (opaque: the bits' comparisons are made here, not kept in
-            // scalar registers for every plane across the half sweeps)
-            asm volatile("" : "+v"(nb));
-            w = (nb & (e ? SOR_IM : SOR_IP)) ? p : w;
-            constexpr unsigned others = (e ? SOR_IP : SOR_IM) | SOR_JM | SOR_JP | SOR_KM | SOR_KP;
-            if (__ballot(nb & others) != 0) {  // tiles at the other faces
-                q = (nb & (e ? SOR_IP : SOR_IM)) ? p : q;
-                yl = (nb & SOR_JM) ? p : yl;
-                yh = (nb & SOR_JP) ? p : yh;
-                wl = (nb & SOR_KM) ? p : wl;
-                wh = (nb & SOR_KP) ? p : wh;
-            }
-        }
-        const double v = sor_node<BOLTZ>(s, a, p, R[k][e], w + q, yl + yh, wl + wh);
-        const double n = (mb & SOR_REG) ? v : p;
-        P[k][e] = n;
-        lds[e][k][tid] = n;
-    };
-    // Half sweep q: the first nodes of the planes of one parity, the second
-    // ones of the other's (first = 1: odd planes' first nodes).  Waves whose
-    // lines are too near the tile's ends to be right skip it.  With Neumann
-    // bits to look at, such planes are left out too; without, all are made,
-    // with no branches, so that their loads and sums overlap (measured both
-    // ways: 96^3 walls 2.76 ms against 3.11 with the branches; the plates' 64 x
-    // 64 x 256 64.4 ms against 61.1 with them).
-    auto half = [&](auto firstc, int q, bool fresh) __attribute__((always_inline)) {
-        constexpr int first = decltype(firstc)::value;
-        if (!((jlo || jl > q) && (jhi || jl < TJ - 1 - q))) return;
-        auto plane = [&](auto kc) __attribute__((always_inline)) {
-            constexpr int k = decltype(kc)::value;
-            constexpr int near = SOR_HALO;  // planes that every half sweep makes
-            if (NEU && k < near && !(klo || k > q)) return;
-            if (NEU && k > TK - 1 - near && !(khi || k < TK - 1 - q)) return;
-            node(kc, std::integral_constant<int, ((k & 1) == first) ? 0 : 1>{}, fresh);
-        };
-        for_planes(plane, std::make_integer_sequence<int, TK - 2>{});
-    };
-    // planes whose first node is red: even ones where j + k0 is even
-    const bool odd = ((j0 + (wave & 1) + k0) & 1) != 0;
-    auto sweeps = [&](auto redc) __attribute__((always_inline)) {
-        constexpr int red = decltype(redc)::value;
-        for (int q = 0; q < ns; q += 2) {
-            const bool fresh = own != 0 || q >= 2;
-            half(std::integral_constant<int, red>{}, q, fresh);
-            __syncthreads();
-            half(std::integral_constant<int, 1 - red>{}, q + 1, fresh);
-            __syncthreads();
-        }
-    };
-    if (odd)
-        sweeps(std::integral_constant<int, 1>{});
-    else
-        sweeps(std::integral_constant<int, 0>{});
-    const int ci = ax.core(bx), ce = ax.core(bx + 1);
-    const bool wj = j >= ay.core(by) && j < ay.core(by + 1);
-    const bool w1 = wj && i >= ci && i < ce, w2 = wj && i + 1 >= ci && i + 1 < ce;
-    const int kc = az.core(bz), ke = az.core(bz + 1);
-    if (w1 && w2) {
-#pragma unroll
-        for (int k = 0; k < TK; k++)
-            if (k0 + k >= kc && k0 + k < ke) *reinterpret_cast<D2*>(out + (ub + (unsigned)k * sk)) = P[k];
-    } else if (w1 || w2) {  // a core that ends inside a pair
-#pragma unroll
-        for (int k = 0; k < TK; k++)
-            if (k0 + k >= kc && k0 + k < ke) out[ub + (unsigned)k * sk + (w1 ? 0u : 1u)] = w1 ? P[k][0] : P[k][1];
-    }
-}
-
-// every Neumann face node from the node its chain of copies ends at (an edge
-// node copies a face node, which copies an interior one): what k_neumann's
-// three phases leave
-__global__ void __launch_bounds__(BLOCK)
-    k_neumann_all(Stencil s, const uint8_t* __restrict__ nt, double* __restrict__ phi,
-                  const double* __restrict__ stop) {
-    if (*stop != 0.0) return;
-    long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        uint8_t t = nt[u];
-        if (t == NT_REG || t == NT_DIR) continue;
-        long long v = u;
-        while (t != NT_REG && t != NT_DIR) {
-            switch (t) {
-                case NT_NEU_IM: v += 1; break;
-                case NT_NEU_IP: v -= 1; break;
-                case NT_NEU_JM: v += s.sj; break;
-                case NT_NEU_JP: v -= s.sj; break;
-                case NT_NEU_KM: v += s.sk; break;
-                default: v -= s.sk; break;
-            }
-            t = nt[v];
-        }
-        phi[u] = phi[v];
-    }
-}
-
-// Neumann copies; phase 0 = k faces, 1 = j faces, 2 = i faces, so edge and
-// corner chains (an i face reads a j face reads a k face) resolve in order.
-__global__ void __launch_bounds__(BLOCK)
-    k_neumann(Stencil s, const uint8_t* __restrict__ nt, double* __restrict__ phi, int phase) {
-    long long u = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    if (u >= s.nn) return;
-    uint8_t t = nt[u];
-    if (t == NT_REG || t == NT_DIR) return;
-    int ph = t <= NT_NEU_IP ? 2 : (t <= NT_NEU_JP ? 1 : 0);
-    if (ph != phase) return;
-    phi[u] = nbr_of<double>(t, phi, u, s);
-}
-
-// Grid-wide sums of the linear solvers: every workgroup stores its partial
-// sum at part[blockIdx.x] (a plain store, nothing to clear and no atomics:
-// 1000 workgroups adding to one FP64 word took longer than the PCG kernels'
-// loads), and every workgroup of the kernel that needs the total adds the
-// partials up itself, while its first loads are in flight.
-// PART_MAX workgroups at most: four per CU, all resident at once at these
-// kernels' 44..107 registers (128^3 FP64 solve of 424 iterations: 20.0 ms with
-// up to 2048 workgroups, whose last ones ran as a second, nearly empty wave,
-// 18.8 with 1280, 16.1 with 1024, 16.3 with 512)
-constexpr int PART_MAX = 1024;
-// ctx->scratch offsets of the partials: three residual sums, then PCG's g.s,
-// g.g and d.z (a second set of these for k_cg, which reads one and writes the
-// other); the stop flag and the rings of g.s and alpha follow
-constexpr int PART_F = 16384, PART_GS = PART_F + 3 * PART_MAX, PART_GG = PART_GS + PART_MAX,
-              PART_DZ = PART_GG + PART_MAX, PART_SET = 3 * PART_MAX, PCG_FLAG = PART_GS + 2 * PART_SET,
-              PCG_GS = PCG_FLAG + 8, PCG_AL = PCG_GS + 4;
-static_assert(PCG_AL + 4 <= (int)SCRATCH_DOUBLES, "scratch layout");
-__device__ inline double sum_parts(const double* __restrict__ part, int n) {
-    __shared__ double red[BLOCK / 64];
-    double v = 0;
-    for (int q = threadIdx.x; q < n; q += BLOCK) v += part[q];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double t = 0;
-#pragma unroll
-    for (int w = 0; w < BLOCK / 64; w++) t += red[w];
-    __syncthreads();
-    return t;  // valid in every thread
-}
-// out[q] = the sum of part[q * PART_MAX ..] (one workgroup per q); out may
-// be pinned host memory
-__global__ void __launch_bounds__(BLOCK) k_sum_parts(const double* __restrict__ part, int n, double* out) {
-    const double t = sum_parts(part + (size_t)blockIdx.x * PART_MAX, n);
-    if (threadIdx.x == 0) out[blockIdx.x] = t;
-}
-
-// The end of a batch of SOR sweeps: the residual's three sums to the host
-// (pinned memory), and the stop flag when the criterion is met; out[3]: met
-__global__ void __launch_bounds__(BLOCK)
-    k_sor_check(double* __restrict__ scratch, int nb, int ref_rms, double nn, double tol, double* out) {
-    if (scratch[PCG_FLAG] != 0.0) return;
-    double r[3];
-#pragma unroll
-    for (int q = 0; q < 3; q++) r[q] = sum_parts(scratch + PART_F + q * PART_MAX, nb);
-    if (threadIdx.x != 0) return;
-    const double crit = ref_rms ? sqrt(r[0] / nn) : (r[2] > 0 ? sqrt(r[1] / r[2]) : sqrt(r[1]));
-    for (int q = 0; q < 3; q++) out[q] = r[q];
-    out[3] = crit < tol ? 1.0 : 0.0;
-    if (crit < tol) scratch[PCG_FLAG] = 1.0;
-}
-__global__ void k_clear_flag(double* __restrict__ scratch) { scratch[PCG_FLAG] = 0.0; }
-
-// Four consecutive nodes u0 .. u0 + 3 (u0 a multiple of 4) per thread, in
-// flat order: a vector's own values in one 16-byte load (two in FP64), the
-// rows on either side likewise (unaligned where a row is not a multiple of 4
-// long), the i-neighbours beyond the group as single words.  Rows need no
-// special care: a group that straddles two i-lines holds face nodes there,
-// and face nodes do not use the 7-point stencil.  Addresses are clamped into
-// the array for the groups on its first and last planes.
-template <typename T>
-struct Q4 {
-    T a[4];
-};
-template <typename T>
-__device__ inline Q4<T> load4(const T* __restrict__ p) {
-    typedef T V __attribute__((ext_vector_type(4), aligned(sizeof(T))));
-    const V v = *reinterpret_cast<const V*>(p);
-    return Q4<T>{{v[0], v[1], v[2], v[3]}};
-}
-template <typename T>
-__device__ inline void store4(T* __restrict__ p, const T (&a)[4]) {
-    typedef T V __attribute__((ext_vector_type(4), aligned(sizeof(T))));
-    *reinterpret_cast<V*>(p) = V{a[0], a[1], a[2], a[3]};
-}
-template <typename T>
-struct Ring4 {
-    Q4<T> c, ym, yp, zm, zp;
-    T l, r;
-};
-template <typename T>
-__device__ inline void load_ring4(const T* __restrict__ v, unsigned u0, const Stencil& s, Ring4<T>& g) {
-    const unsigned n = (unsigned)s.nn, sj = (unsigned)s.sj, sk = (unsigned)s.sk, last = n - 4u;
-    g.c = load4(v + u0);
-    g.ym = load4(v + (u0 >= sj ? u0 - sj : 0u));
-    g.yp = load4(v + (u0 + sj <= last ? u0 + sj : last));
-    g.zm = load4(v + (u0 >= sk ? u0 - sk : 0u));
-    g.zp = load4(v + (u0 + sk <= last ? u0 + sk : last));
-    g.l = v[u0 >= 1u ? u0 - 1u : 0u];
-    g.r = v[u0 + 4u < n ? u0 + 4u : n - 1u];
-}
-// the 7-point operator at the group's node q (apply_A's order)
-template <typename T>
-__device__ inline T ring_A(const Ring4<T>& g, int q, const Stencil& s) {
-    const T xm = q == 0 ? g.l : g.c.a[q == 0 ? 0 : q - 1];
-    const T xp = q == 3 ? g.r : g.c.a[q == 3 ? 3 : q + 1];
-    return (T)s.cz * (g.zm.a[q] + g.zp.a[q]) + (T)s.cy * (g.ym.a[q] + g.yp.a[q]) + (T)s.cx * (xm + xp) -
-           (T)s.twos * g.c.a[q];
-}
-__device__ inline uint32_t load_types4(const uint8_t* __restrict__ nt, unsigned u0) {
-    return *reinterpret_cast<const uint32_t*>(nt + u0);
-}
-__device__ inline uint8_t type_at(uint32_t t4, int q) { return (uint8_t)((t4 >> (8 * q)) & 0xFFu); }
-
-// workgroups of the four-node kernels with partial sums: one group per
-// thread up to PART_MAX workgroups
-unsigned part_blocks(long long nn) {
-    long long b = (nn / 4 + BLOCK - 1) / BLOCK;
-    if (b > PART_MAX) b = PART_MAX;
-    return (unsigned)((b + NXCD - 1) / NXCD * NXCD);
-}
-
-// residual of the (Boltzmann) Poisson problem, three partial sums: sum R^2
-// over all non-Dirichlet rows (reference RMS numerator), sum R^2 over
-// regular rows, sum b^2 over regular rows.
-__global__ void __launch_bounds__(BLOCK)
-    k_resid(Stencil s, SorArgs a, const uint8_t* __restrict__ nt, const double* __restrict__ phi,
-            const double* __restrict__ rho, double* __restrict__ part) {
-    double r_all = 0, r_reg = 0, b_reg = 0;
-    auto regular = [&](double p, double rho_u, double sx, double sy, double sz) {
-        double q = rho_u;
-        if (a.n0 != 0.0) q -= QE * (a.n0 * exp((p - a.phi0) * a.inv_te0));
-        const double R = -p * s.twos + q * a.ieps + sx * s.cx + sy * s.cy + sz * s.cz;
-        const double b = rho_u * a.ieps;
-        r_all += R * R;
-        r_reg += R * R;
-        b_reg += b * b;
-    };
-    auto face = [&](uint8_t t, long long u) {
-        const double R = phi[u] - nbr_of<double>(t, phi, u, s);
-        r_all += R * R;
-    };
-    long long end;
-    for (long long m = chunk_begin(s.nn / 4, end) + threadIdx.x; m < end; m += BLOCK) {
-        const unsigned u0 = 4u * (unsigned)m;
-        const uint32_t t4 = load_types4(nt, u0);
-        Ring4<double> g;
-        load_ring4(phi, u0, s, g);
-        const Q4<double> rh = load4(rho + u0);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint8_t t = type_at(t4, q);
-            if (t == NT_REG)
-                regular(g.c.a[q], rh.a[q], (q == 0 ? g.l : g.c.a[q == 0 ? 0 : q - 1]) +
-                                               (q == 3 ? g.r : g.c.a[q == 3 ? 3 : q + 1]),
-                        g.ym.a[q] + g.yp.a[q], g.zm.a[q] + g.zp.a[q]);
-            else if (t != NT_DIR)
-                face(t, u0 + q);
-        }
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
-        const long long u = (s.nn & ~3ll) + threadIdx.x;
-        if (nt[u] != NT_REG && nt[u] != NT_DIR) face(nt[u], u);
-    }
-    double t0 = block_sum(r_all), t1 = block_sum(r_reg), t2 = block_sum(b_reg);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = t0;
-        part[PART_MAX + blockIdx.x] = t1;
-        part[2 * PART_MAX + blockIdx.x] = t2;
-    }
-}
-
-// ------------------------------------------------------------------------
-// Newton residual and Jacobian shift (PotentialSolver.cpp:189-217)
-//   b_u = 0 (Neumann), phi_u (Dirichlet), -rho_u/eps0 (regular)
-//   F = A phi - b - [regular] q n0 exp((phi-phi0)/Te0)/eps0
-//   P = [regular] q n0/(eps0 Te0) exp((phi-phi0)/Te0)
-// partial sums F.F (all rows), F.F (regular), b.b (regular)
-// START: the set-up of PCG on J y = F from y = 0 instead of F itself: g = -F
-// (TF), its Jacobi-scaled s = M g (NEU), and the partial sums g.s and g.g;
-// the stop flag of the iterations that follow is cleared.
-// ------------------------------------------------------------------------
-struct NewtonArgs {
-    double ieps, phi0, n0, inv_te0;
-};
-
-template <typename TF, bool START, bool NEU>
-__global__ void __launch_bounds__(BLOCK)
-    k_F(Stencil s, NewtonArgs a, const uint8_t* __restrict__ nt, const double* __restrict__ phi,
-        const double* __restrict__ rho, TF* __restrict__ F, TF* __restrict__ sv, double* __restrict__ P,
-        double* __restrict__ scratch) {
-    double f_all = 0, f_reg = 0, b_reg = 0, gs = 0, gg = 0;
-    // one node: its row of F, and what START keeps of it
-    auto row = [&](uint8_t t, double Ap, double pu, double rho_u, double& Pu, TF& Fu, TF& su) {
-        Pu = 0.0;
-        double f;
-        if (t == NT_REG) {
-            const double b = -rho_u * a.ieps;
-            f = Ap - b;
-            if (a.n0 != 0.0) {
-                const double ex = exp((pu - a.phi0) * a.inv_te0);
-                f -= QE * a.n0 * ex * a.ieps;
-                Pu = QE * a.n0 * a.ieps * a.inv_te0 * ex;
-            }
-            f_reg += f * f;
-            b_reg += b * b;
-        } else {
-            f = t == NT_DIR ? 0.0 : Ap;  // a Dirichlet row is phi - phi
-        }
-        f_all += f * f;
-        Fu = START ? -(TF)f : (TF)f;
-        if (START) {
-            su = (TF)(1.0 / diagA(t, s)) * Fu;
-            gs += (double)Fu * (double)su;
-            gg += (double)Fu * (double)Fu;
-        }
-    };
-    long long end;
-    for (long long m = chunk_begin(s.nn / 4, end) + threadIdx.x; m < end; m += BLOCK) {
-        const unsigned u0 = 4u * (unsigned)m;
-        const uint32_t t4 = load_types4(nt, u0);
-        Ring4<double> g;
-        load_ring4(phi, u0, s, g);
-        const Q4<double> rh = load4(rho + u0);
-        TF f4[4], s4[4];
-        double P4[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint8_t t = type_at(t4, q);
-            double Ap = 0.0;
-            if (t == NT_REG)
-                Ap = ring_A(g, q, s);
-            else if (NEU && t != NT_DIR)
-                Ap = apply_A<double>(t, u0 + q, s, [&](long long v) { return phi[v]; });
-            s4[q] = 0;
-            row(t, Ap, g.c.a[q], rh.a[q], P4[q], f4[q], s4[q]);
-        }
-        store4(F + u0, f4);
-        if (START && NEU) store4(sv + u0, s4);
-        if (P) store4(P + u0, P4);
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
-        const long long u = (s.nn & ~3ll) + threadIdx.x;
-        const uint8_t t = nt[u];
-        double Pu;
-        TF Fu, su = 0;
-        row(t, NEU ? apply_A<double>(t, u, s, [&](long long v) { return phi[v]; }) : 0.0, phi[u], rho[u], Pu, Fu, su);
-        F[u] = Fu;
-        if (START && NEU) sv[u] = su;
-        if (P) P[u] = Pu;
-    }
-    double t0 = block_sum(f_all), t1 = block_sum(f_reg), t2 = block_sum(b_reg);
-    if (threadIdx.x == 0) {
-        scratch[PART_F + blockIdx.x] = t0;
-        scratch[PART_F + PART_MAX + blockIdx.x] = t1;
-        scratch[PART_F + 2 * PART_MAX + blockIdx.x] = t2;
-    }
-    if (START) {
-        double t3 = block_sum(gs), t4 = block_sum(gg);
-        if (threadIdx.x == 0) {
-            scratch[PART_GS + blockIdx.x] = t3;
-            scratch[PART_GG + blockIdx.x] = t4;
-            if (blockIdx.x == 0) scratch[PCG_FLAG] = 0.0;
-        }
-    }
-}
-
-// ------------------------------------------------------------------------
-// PCG on J y = F, J = A - diag(P), M = 1/diag(A), two kernels per iteration
-// over groups of four nodes, sums by partials.  Without Neumann faces M is
-// one constant on every row where g is not 0 (Dirichlet rows of F vanish),
-// so s = M g is formed from g where it is read; with them (NEU) s is kept.
-//
-// 128^3 nodes, FP64: k_pcg1 moves 41 B and k_pcg2 48 B per node of
-// cache-resident vectors, about 18 us each (5 TB/s); with one node per load,
-// eight nodes per thread, s stored and atomics on single words they took 27.8
-// and 30.2 us.  97^3 FP32: 5.6 and 5.0 us, close to an empty launch's 4 us,
-// against 14.1 and 13.5 us.
-// ------------------------------------------------------------------------
-template <typename T>
-struct PcgVec {
-    T *y, *g, *s, *z;  // s: NEU only
-    const double* P;   // may be null
-};
-
-// d_new = beta d_old - s (beta = gs[t]/gs[t-1], 0 at t = 0); z = J d_new,
-// by the recurrence J d_new = beta J d_old - J s: the stencil of s alone
-// (one operand's neighbours instead of two), the previous z in place.
-// gg[t] is kept for the host's check.  Returns at once when the stop flag is
-// set (an earlier iteration converged).
-template <typename T, bool NEU>
-__global__ void __launch_bounds__(BLOCK)
-    k_pcg1(Stencil s, const uint8_t* __restrict__ nt, PcgVec<T> v, const T* __restrict__ dold,
-           T* __restrict__ dnew, double* __restrict__ scratch, double* __restrict__ ggh, int t) {
-    if (scratch[PCG_FLAG] != 0.0) return;  // (the whole grid)
-    const T* __restrict__ src = NEU ? v.s : v.g;
-    const T mreg = (T)(1.0 / diagA(NT_REG, s));  // M of a regular row (k_pcg2's s, rounded alike)
-    long long end;
-    long long m = chunk_begin(s.nn / 4, end) + threadIdx.x;
-    Ring4<T> r;
-    Q4<T> d4{}, z4{};
-    uint32_t t4 = 0;
-    auto load = [&]() {
-        const unsigned u0 = 4u * (unsigned)m;
-        t4 = load_types4(nt, u0);
-        load_ring4(src, u0, s, r);
-        if (t > 0) {
-            d4 = load4(dold + u0);
-            z4 = load4(v.z + u0);
-        }
-    };
-    if (m < end) load();
-    const double gs = sum_parts(scratch + PART_GS, gridDim.x);
-    double beta = 0.0;
-    if (t > 0) {
-        const double den = scratch[PCG_GS + ((t - 1) & 3)];
-        beta = den != 0.0 ? gs / den : 0.0;
-    }
-    const T bt = (T)beta;
-    double acc = 0;
-    while (m < end) {
-        const unsigned u0 = 4u * (unsigned)m;
-        if (!NEU) {  // s = M g
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                r.c.a[q] *= mreg;
-                r.ym.a[q] *= mreg;
-                r.yp.a[q] *= mreg;
-                r.zm.a[q] *= mreg;
-                r.zp.a[q] *= mreg;
-            }
-            r.l *= mreg;
-            r.r *= mreg;
-        }
-        T dn[4], zn[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint8_t ty = type_at(t4, q);
-            const T su = r.c.a[q];
-            T js = su;  // a Dirichlet row
-            if (ty == NT_REG)
-                js = ring_A(r, q, s);
-            else if (NEU && ty != NT_DIR)
-                js = apply_A<T>(ty, u0 + q, s, [&](long long w) { return src[w]; });
-            if (v.P) js -= (T)v.P[u0 + q] * su;
-            dn[q] = -su + bt * d4.a[q];
-            zn[q] = -js + bt * z4.a[q];
-            acc += (double)dn[q] * (double)zn[q];
-        }
-        store4(dnew + u0, dn);
-        store4(v.z + u0, zn);
-        m += BLOCK;
-        if (m < end) load();
-    }
-    if (NEU && blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
-        const long long u = (s.nn & ~3ll) + threadIdx.x;
-        const T su = src[u];
-        T js = apply_A<T>(nt[u], u, s, [&](long long w) { return src[w]; });
-        if (v.P) js -= (T)v.P[u] * su;
-        T du = -su, zu = -js;
-        if (t > 0) {
-            du += bt * dold[u];
-            zu += bt * v.z[u];
-        }
-        dnew[u] = du;
-        v.z[u] = zu;
-        acc += (double)du * (double)zu;
-    }
-    const double a = block_sum(acc);
-    if (threadIdx.x == 0) scratch[PART_DZ + blockIdx.x] = a;
-    if (blockIdx.x == 0) {
-        const double gg = sum_parts(scratch + PART_GG, gridDim.x);
-        if (threadIdx.x == 0) {
-            scratch[PCG_GS + (t & 3)] = gs;
-            ggh[t] = gg;
-        }
-    }
-}
-
-// alpha = gs[t]/dz[t]; y += alpha d (y = 0 before t = 0); g += alpha z;
-// s = M g; gs[t+1], gg[t+1]
-template <typename T, bool NEU>
-__global__ void __launch_bounds__(BLOCK)
-    k_pcg2(Stencil s, const uint8_t* __restrict__ nt, PcgVec<T> v, const T* __restrict__ d,
-           double* __restrict__ scratch, int t) {
-    if (scratch[PCG_FLAG] != 0.0) return;  // (the whole grid)
-    const T mreg = (T)(1.0 / diagA(NT_REG, s));
-    long long end;
-    long long m = chunk_begin(s.nn / 4, end) + threadIdx.x;
-    Q4<T> g4, z4, y4{}, d4;
-    uint32_t t4 = 0;
-    auto load = [&]() {
-        const unsigned u0 = 4u * (unsigned)m;
-        g4 = load4(v.g + u0);
-        z4 = load4(v.z + u0);
-        if (t > 0) y4 = load4(v.y + u0);
-        d4 = load4(d + u0);
-        if (NEU) t4 = load_types4(nt, u0);
-    };
-    if (m < end) load();
-    const double den = sum_parts(scratch + PART_DZ, gridDim.x);
-    const T alpha = (T)(den != 0.0 ? scratch[PCG_GS + (t & 3)] / den : 0.0);
-    double gs = 0, gg = 0;
-    auto sums = [&](T gu, T su) {
-        gs += (double)gu * (double)su;
-        gg += (double)gu * (double)gu;
-    };
-    while (m < end) {
-        const unsigned u0 = 4u * (unsigned)m;
-        T gn[4], yn[4], sn[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            gn[q] = g4.a[q] + alpha * z4.a[q];
-            yn[q] = y4.a[q] + alpha * d4.a[q];
-            sn[q] = (NEU ? (T)(1.0 / diagA(type_at(t4, q), s)) : mreg) * gn[q];
-            sums(gn[q], sn[q]);
-        }
-        store4(v.g + u0, gn);
-        store4(v.y + u0, yn);
-        if (NEU) store4(v.s + u0, sn);
-        m += BLOCK;
-        if (m < end) load();
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group
-        const long long u = (s.nn & ~3ll) + threadIdx.x;
-        if (NEU) {
-            const T gu = v.g[u] + alpha * v.z[u];
-            const T su = (T)(1.0 / diagA(nt[u], s)) * gu;
-            v.y[u] = (t > 0 ? v.y[u] : (T)0) + alpha * d[u];
-            v.g[u] = gu;
-            v.s[u] = su;
-            sums(gu, su);
-        }
-    }
-    const double a = block_sum(gs), b = block_sum(gg);
-    if (threadIdx.x == 0) {
-        scratch[PART_GS + blockIdx.x] = a;
-        scratch[PART_GG + blockIdx.x] = b;
-    }
-}
-
-// The same iteration in one kernel (Chronopoulos and Gear's arrangement of CG:
-// J. Comput. Appl. Math. 25, 1989), for grids without Neumann faces that a
-// launch's latency bounds.  With u = M g, w = J u and the sums gamma = g.u,
-// delta = w.u of the last kernel,
-//   beta = gamma / gamma_old,  alpha = gamma / (delta - beta gamma / alpha_old)
-//   d = -u + beta d,  z = -w + beta z (= J d),  y += alpha d,  g += alpha z
-// and then the new w and sums.  The new w needs the new g of the neighbours,
-// which every thread makes again from the old g, w and z around its group;
-// those three are therefore written to a second set of vectors.  t = -1: w and
-// delta of the start.
-template <typename T>
-struct CgVec {
-    T *y, *d, *g[2], *w[2], *z[2];
-    const double* P;  // may be null
-};
-template <typename T>
-__global__ void __launch_bounds__(BLOCK)
-    k_cg(Stencil s, const uint8_t* __restrict__ nt, CgVec<T> v, double* __restrict__ scratch,
-         double* __restrict__ ggh, int t) {
-    if (scratch[PCG_FLAG] != 0.0) return;  // (the whole grid)
-    const int from = t < 0 ? 0 : t & 1, to = t < 0 ? 0 : (t + 1) & 1;
-    const double* __restrict__ pin = scratch + from * PART_SET;
-    double* __restrict__ pout = scratch + to * PART_SET;
-    const T* __restrict__ gi = v.g[from];
-    const T* __restrict__ wi = v.w[from];
-    const T* __restrict__ zi = v.z[from];
-    const T mreg = (T)(1.0 / diagA(NT_REG, s));  // M of a regular row; g vanishes on the others
-    long long end;
-    long long m = chunk_begin(s.nn / 4, end) + threadIdx.x;
-    Ring4<T> g{}, w{}, z{};
-    Q4<T> d4{}, y4{};
-    uint32_t t4 = 0;
-    auto load = [&]() {
-        const unsigned u0 = 4u * (unsigned)m;
-        t4 = load_types4(nt, u0);
-        load_ring4(gi, u0, s, g);
-        if (t >= 0) load_ring4(wi, u0, s, w);
-        if (t > 0) {
-            load_ring4(zi, u0, s, z);
-            d4 = load4(v.d + u0);
-            y4 = load4(v.y + u0);
-        }
-    };
-    if (m < end) load();
-    double al = 0.0, be = 0.0, gamma = 0.0;
-    if (t >= 0) {
-        gamma = sum_parts(pin + PART_GS, gridDim.x);
-        double den = sum_parts(pin + PART_DZ, gridDim.x);
-        if (t > 0) {
-            const double go = scratch[PCG_GS + ((t - 1) & 3)], ao = scratch[PCG_AL + ((t - 1) & 3)];
-            be = go != 0.0 ? gamma / go : 0.0;
-            if (ao != 0.0) den -= be * gamma / ao;
-        }
-        al = den != 0.0 ? gamma / den : 0.0;
-    }
-    const T alpha = (T)al, beta = (T)be;
-    double gs = 0, gg = 0, dz = 0;
-    while (m < end) {
-        const unsigned u0 = 4u * (unsigned)m;
-        T zn[4], gn[4], wn[4], dn[4], yn[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            zn[q] = -w.c.a[q] + beta * z.c.a[q];
-            dn[q] = -(mreg * g.c.a[q]) + beta * d4.a[q];
-            yn[q] = y4.a[q] + alpha * dn[q];
-        }
-        // the new g around the group, then u = M g in its place
-        auto next = [&](T& gv, T wv, T zv) { gv = mreg * (gv + alpha * (-wv + beta * zv)); };
-        T gc[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            gc[q] = g.c.a[q] + alpha * zn[q];
-            g.c.a[q] = mreg * gc[q];
-            next(g.ym.a[q], w.ym.a[q], z.ym.a[q]);
-            next(g.yp.a[q], w.yp.a[q], z.yp.a[q]);
-            next(g.zm.a[q], w.zm.a[q], z.zm.a[q]);
-            next(g.zp.a[q], w.zp.a[q], z.zp.a[q]);
-        }
-        next(g.l, w.l, z.l);
-        next(g.r, w.r, z.r);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const T u = g.c.a[q];
-            T ju = type_at(t4, q) == NT_REG ? ring_A(g, q, s) : u;
-            if (v.P) ju -= (T)v.P[u0 + q] * u;
-            wn[q] = ju;
-            gn[q] = gc[q];
-            gs += (double)gn[q] * (double)u;
-            gg += (double)gn[q] * (double)gn[q];
-            dz += (double)ju * (double)u;
-        }
-        store4(v.w[to] + u0, wn);
-        if (t >= 0) {
-            store4(v.g[to] + u0, gn);
-            store4(v.z[to] + u0, zn);
-            store4(v.d + u0, dn);
-            store4(v.y + u0, yn);
-        }
-        m += BLOCK;
-        if (m < end) load();
-    }
-    if (blockIdx.x == 0 && threadIdx.x < (unsigned)(s.nn & 3)) {  // corner nodes past the last group: all zero
-        const long long u = (s.nn & ~3ll) + threadIdx.x;
-        v.w[to][u] = 0;
-        if (t >= 0) {
-            v.g[to][u] = 0;
-            v.z[to][u] = 0;
-            v.y[u] = 0;
-        }
-    }
-    const double a = block_sum(gs), b = block_sum(gg), c = block_sum(dz);
-    if (threadIdx.x == 0) {
-        if (t >= 0) {
-            pout[PART_GS + blockIdx.x] = a;
-            pout[PART_GG + blockIdx.x] = b;
-        }
-        pout[PART_DZ + blockIdx.x] = c;
-    }
-    if (blockIdx.x == 0 && t >= 0) {
-        const double g0 = sum_parts(pin + PART_GG, gridDim.x);
-        if (threadIdx.x == 0) {
-            scratch[PCG_GS + (t & 3)] = gamma;
-            scratch[PCG_AL + (t & 3)] = al;
-            ggh[t] = g0;
-        }
-    }
-}
-
-// The end of a batch of iterations (t0, t1]: g.g of each to the host (pinned
-// memory), and the stop flag when one is within the target.
-__global__ void __launch_bounds__(BLOCK)
-    k_pcg_check(double* __restrict__ scratch, const double* __restrict__ gg1, const double* __restrict__ ggh, int nb,
-                int t0, int t1, double target2, double* host) {
-    if (scratch[PCG_FLAG] != 0.0) return;
-    const double gg = sum_parts(gg1, nb);  // of iteration t1
-    __shared__ int hit;
-    if (threadIdx.x == 0) hit = 0;
-    __syncthreads();
-    for (int q = t0 + 1 + threadIdx.x; q <= t1; q += BLOCK) {
-        const double x = q == t1 ? gg : ggh[q];
-        host[q - t0 - 1] = x;
-        if (x <= target2) hit = 1;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && hit) scratch[PCG_FLAG] = 1.0;
-}
-
-// phi -= y on non-Dirichlet rows (PotentialSolver.cpp:225-228); with part,
-// the partial sums of y.y over them
-template <typename T>
-__global__ void __launch_bounds__(BLOCK)
-    k_update_phi(Stencil s, const uint8_t* __restrict__ nt, double* __restrict__ phi,
-                 const T* __restrict__ y, double* __restrict__ part) {
-    double yy = 0;
-    long long end;
-    for (long long u = chunk_begin(s.nn, end) + threadIdx.x; u < end; u += BLOCK) {
-        if (nt[u] == NT_DIR) continue;
-        double yv = (double)y[u];
-        phi[u] -= yv;
-        yy += yv * yv;
-    }
-    if (!part) return;
-    double a = block_sum(yy);
-    if (threadIdx.x == 0) part[blockIdx.x] = a;
-}
-
-Stencil make_stencil(const GridC& g, bool axis_swap) {
-    Stencil s;
-    double d2x = 1.0 / (g.dx[0] * g.dx[0]), d2y = 1.0 / (g.dx[1] * g.dx[1]),
-           d2z = 1.0 / (g.dx[2] * g.dx[2]);
-    s.cx = axis_swap ? d2z : d2x;
-    s.cy = d2y;
-    s.cz = axis_swap ? d2x : d2z;
-    s.twos = 2.0 * (d2x + d2y + d2z);
-    s.itwos = 1.0 / s.twos;
-    for (int d = 0; d < 3; d++) s.idx[d] = 1.0 / g.dx[d];
-    s.sj = g.ni;
-    s.sk = (long long)g.ni * g.nj;
-    s.nn = g.nn;
-    s.ni = g.ni;
-    s.nj = g.nj;
-    s.nk = g.nk;
-    return s;
-}
-
 // kernels ending in a single-address grid-wide sum: fewer, longer workgroups
 // (eight items per thread) keep the per-workgroup atomics few
 unsigned stencil_blocks_red(long long items) {
     long long b = (items + BLOCK * 8 - 1) / (BLOCK * 8);
     if (b > 2048) b = 2048;
     b = (b + NXCD - 1) / NXCD * NXCD;
-    return (unsigned)b;
-}
-
-unsigned stencil_blocks(long long items) {
-    // about two items per thread: enough workgroups in flight to cover HBM latency
-    long long b = (items + BLOCK * 2 - 1) / (BLOCK * 2);
-    if (b > 16384) b = 16384;
-    b = (b + NXCD - 1) / NXCD * NXCD;  // multiple of NXCD, at least NXCD
     return (unsigned)b;
 }
 
@@ -1112,457 +109,6 @@ extern "C" int pic_efield(pic_ctx* ctx) {
     }
     PIC_HIP(ctx, hipGetLastError());
     return PIC_OK;
-}
-
-// any Neumann face node (a face node that is neither an object node nor
-// flagged Dirichlet); the node types are current
-static bool has_neumann(pic_ctx* ctx) {
-    if (pic_ensure_ntype(ctx) != PIC_OK) return true;
-    return ctx->has_neumann;
-}
-
-// queues the residual sums of phi (k_resid's three) into out (pinned memory)
-static int queue_residual(pic_ctx* ctx, const Stencil& st, const SorArgs& a, double* out) {
-    const unsigned nb = part_blocks(st.nn);
-    k_resid<<<nb, BLOCK, 0, ctx->stream>>>(st, a, ctx->ntype, ctx->phi, ctx->rho, ctx->scratch + PART_F);
-    k_sum_parts<<<3, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nb, out);
-    PIC_HIP(ctx, hipGetLastError());
-    return PIC_OK;
-}
-static int residual_norms(pic_ctx* ctx, const Stencil& st, const SorArgs& a, double out[3]) {
-    int rc = pic_ensure_pin(ctx, 3 * sizeof(double));
-    if (!rc) rc = queue_residual(ctx, st, a, ctx->pin);
-    if (rc) return rc;
-    PIC_HIP(ctx, pic_spin_wait(ctx->stream));
-    for (int q = 0; q < 3; q++) out[q] = ctx->pin[q];
-    return PIC_OK;
-}
-
-static double crit_value(const pic_solver_params* p, const double r[3], double nn) {
-    if (p->tol_kind == PIC_TOL_REF_RMS) return std::sqrt(r[0] / nn);
-    return r[2] > 0 ? std::sqrt(r[1] / r[2]) : std::sqrt(r[1]);
-}
-
-static SorArgs sor_args(const pic_solver_params* p, const Stencil& s) {
-    SorArgs a;
-    a.omega = p->omega > 0 ? p->omega : 1.4;
-    a.ieps = 1.0 / EPS0;
-    a.itwos = 1.0 / s.twos;
-    a.phi0 = p->phi0;
-    a.n0 = p->n0;
-    a.inv_te0 = 1.0 / (p->Te0 != 0 ? p->Te0 : 1.0);
-    a.color = 0;
-    return a;
-}
-
-// SOR with one launch per colour on the natural layout, in place
-// (PIC_SOLVE_SOR_PLAIN); the tiled sweeps give the same values.
-static int solve_sor_plain(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st) {
-    const GridC& g = ctx->g;
-    Stencil s = make_stencil(g, false);
-    SorArgs a = sor_args(p, s);
-    bool neu = has_neumann(ctx);
-    int check = p->check_every > 0 ? p->check_every : 25;
-    long long half_items = (long long)((g.ni + 1) / 2) * g.nj * g.nk;
-    double r[3] = {0, 0, 0};
-    int it;
-    bool conv = false, fresh = false;  // fresh: r holds the residual of the current potential
-    double crit = 0;
-    for (it = 0; it < p->max_it; it++) {
-        {
-            PicProfScope ps(ctx, PIC_K_SOR);
-            for (int c = 0; c < 2; c++) {
-                a.color = c;
-                k_sor<<<stencil_blocks(half_items), BLOCK, 0, ctx->stream>>>(s, a, ctx->ntype, ctx->phi, ctx->rho);
-            }
-            if (neu)
-                for (int ph = 0; ph < 3; ph++)
-                    k_neumann<<<grid_for((size_t)g.nn, BLOCK), BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->phi,
-                                                                                        ph);
-        }
-        PIC_HIP(ctx, hipGetLastError());
-        fresh = false;
-        if (it % check == 0) {  // PotentialSolver.cpp:124
-            int rc = residual_norms(ctx, s, a, r);
-            if (rc) return rc;
-            fresh = true;
-            crit = crit_value(p, r, (double)g.nn);
-            if (crit < p->tol) {
-                conv = true;
-                break;
-            }
-        }
-    }
-    if (!fresh) {
-        int rc = residual_norms(ctx, s, a, r);
-        if (rc) return rc;
-    }
-    st->converged = conv;
-    st->iterations = conv ? it + 1 : it;
-    st->newton_iterations = 0;
-    st->ref_l2 = std::sqrt(r[0] / (double)g.nn);
-    st->rel_residual = r[2] > 0 ? std::sqrt(r[1] / r[2]) : std::sqrt(r[1]);
-    return conv ? PIC_OK : PIC_NOT_CONVERGED;
-}
-
-// red-black sweeps on tiles: `sweeps` (1 or 2) from in to out
-template <int PI, int TJ, int TK>
-static void launch_sor_tile(pic_ctx* ctx, const Stencil& s, const SorArgs& a, bool neu, const double* in, double* out,
-                            int sweeps, int own) {
-    const TileAxis ax = tile_axis(s.ni, 2 * PI), ay = tile_axis(s.nj, TJ), az = tile_axis(s.nk, TK);
-    const unsigned nb = ((unsigned)(ax.m * ay.m * az.m) + NXCD - 1) / NXCD * NXCD;
-    const double* stop = ctx->scratch + PCG_FLAG;
-    auto go = [&](auto kernel) {
-        kernel<<<nb, PI * TJ, 0, ctx->stream>>>(s, a, ax, ay, az, ctx->sor_bits, in, out, ctx->rho, 2 * sweeps, own,
-                                                stop);
-    };
-    if (a.n0 != 0.0) {
-        if (neu)
-            go(k_sor_tile<PI, TJ, TK, true, true>);
-        else
-            go(k_sor_tile<PI, TJ, TK, false, true>);
-    } else {
-        if (neu)
-            go(k_sor_tile<PI, TJ, TK, true, false>);
-        else
-            go(k_sor_tile<PI, TJ, TK, false, false>);
-    }
-}
-
-// The tile by the grid.  Small grids: the smallest tile, up to 400 of them
-// (three fit a CU), since a launch then lasts as long as one tile's chain of
-// half sweeps: 64^3 with 294 tiles 1.28 ms against 1.53 and 1.59 with the
-// larger tiles, 96^3 with 968 tiles 3.56 against 2.75.  Larger grids without
-// Neumann faces: 64 x 16 or 32 x 32 nodes of a plane, whichever needs fewer
-// tiles (128^3 6.8 ms with 32 x 32, 8.5 with 64 x 16).  With them 64 x 16: whole
-// lines put the i faces into the threads' own pairs (64 x 64 x 256 plates 61 ms
-// against 98; 97 x 80 x 120 23.5 against 23.8).
-static void sor_sweeps(pic_ctx* ctx, const Stencil& s, const SorArgs& a, bool neu, const double* in, double* out,
-                       int sweeps, int own) {
-    auto tiles = [&](int t, int u, int w) {
-        return (long long)tile_axis(s.ni, t).m * tile_axis(s.nj, u).m * tile_axis(s.nk, w).m;
-    };
-    if (tiles(32, 16, 12) <= 400)
-        launch_sor_tile<16, 16, 12>(ctx, s, a, neu, in, out, sweeps, own);
-    else if (neu || tiles(64, 16, 16) < tiles(32, 32, 16))
-        launch_sor_tile<32, 16, 16>(ctx, s, a, neu, in, out, sweeps, own);
-    else
-        launch_sor_tile<16, 32, 16>(ctx, s, a, neu, in, out, sweeps, own);
-}
-
-// Launches (PCG: iterations) that the host queues behind a check before it
-// waits for it: enough to keep the device busy while the host sees the check's
-// event, and few, because those behind a check that ends the solve are waited
-// for although they return at once (2 us each).  32^3 nodes, SOR from the solution,
-// a check every 25 and every 1000 sweeps: 44 us with 4; 75 and 2225 with the whole
-// interval queued; 47 and 69 with none.  The cold solve 0.38 ms with 2 and with 4, 0.40
-// with the whole interval; 128^3 FP64 PCG 12.6 ms with any.
-constexpr int RUN_AHEAD = 4;
-
-// Red-black SOR (PotentialSolver.cpp:69-166) on tiles.  The residual is
-// checked after the first sweep and then every `check` sweeps (:124); the
-// host queues the first RUN_AHEAD launches of the sweeps up to the next check
-// before it waits for the last one, and once a check is met the launches
-// behind it return at once (the stop flag), so the potential is the one that
-// was checked.  Without memory for the second potential and the row bits the
-// sweeps are made in place.
-static int solve_sor(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st) {
-    if (p->flags & PIC_SOLVE_SOR_PLAIN) return solve_sor_plain(ctx, p, st);
-    const GridC& g = ctx->g;
-    const size_t nn = (size_t)g.nn;
-    Stencil s = make_stencil(g, false);
-    SorArgs a = sor_args(p, s);
-    const bool neu = has_neumann(ctx);
-    const int check = p->check_every > 0 ? p->check_every : 25;
-    if ((!ctx->sor_phi && hipMalloc(&ctx->sor_phi, nn * sizeof(double)) != hipSuccess) ||
-        (!ctx->sor_bits && hipMalloc(&ctx->sor_bits, nn) != hipSuccess)) {
-        (void)hipGetLastError();
-        return solve_sor_plain(ctx, p, st);  // in place
-    }
-    int rc = pic_ensure_pin(ctx, 8 * sizeof(double));
-    if (rc) return rc;
-    for (auto& e : ctx->batch_ev)
-        if (!e) PIC_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    volatile double* hp = ctx->pin;  // two batches of {three sums, criterion met}
-    k_clear_flag<<<1, 1, 0, ctx->stream>>>(ctx->scratch);
-    k_sor_bits<<<stencil_blocks(s.nn), BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->sor_bits);
-    double* buf[2] = {ctx->phi, ctx->sor_phi};
-    const unsigned nbr = part_blocks(s.nn);
-    const int ahead = ctx->prof.on ? 1 : 2;  // profiled runs count no launch that returns at once
-    int it = 0, launches = 0;                // sweeps and launches queued
-    int at[2], par[2], queued = 0, done = 0; // batches queued and waited for; their last sweep and buffer
-    bool conv = false;
-    int last = 0;
-    auto wait_oldest = [&]() {  // for the oldest queued batch; conv: it met the criterion
-        last = done & 1;
-        const hipError_t e = pic_spin_event(ctx->batch_ev[last]);
-        if (e != hipSuccess) return pic_hip_check(ctx, e, "SOR check");
-        done++;
-        conv = hp[4 * last + 3] != 0.0;
-        return (int)PIC_OK;
-    };
-    while (!conv) {
-        while (!conv && it < p->max_it && queued - done < ahead) {
-            const int q = queued & 1;
-            // sweep numbers 0, check, 2 check, ... are checked, and the last
-            // (check may be as large as INT_MAX: only the first sweep and the last)
-            const int upto = it == 0 ? 1 : check < p->max_it - it ? it + check : p->max_it;
-            for (int m = 0; it < upto; m++) {
-                if (m == RUN_AHEAD && queued > done) {
-                    rc = wait_oldest();
-                    if (rc) return rc;
-                    if (conv) break;
-                }
-                PicProfScope ps(ctx, PIC_K_SOR);
-                const int n = std::min(2, upto - it);
-                sor_sweeps(ctx, s, a, neu, buf[launches & 1], buf[(launches & 1) ^ 1], n, it > 0);
-                launches++;
-                it += n;
-            }
-            if (conv) break;
-            double* cur = buf[launches & 1];
-            if (neu)
-                k_neumann_all<<<stencil_blocks(s.nn), BLOCK, 0, ctx->stream>>>(s, ctx->ntype, cur,
-                                                                              ctx->scratch + PCG_FLAG);
-            k_resid<<<nbr, BLOCK, 0, ctx->stream>>>(s, a, ctx->ntype, cur, ctx->rho, ctx->scratch + PART_F);
-            // only sweeps 0, check, 2 check, ... can end the solve
-            const bool can = (it - 1) % check == 0;
-            k_sor_check<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch, (int)nbr, p->tol_kind == PIC_TOL_REF_RMS,
-                                                      (double)nn, can ? p->tol : 0.0, ctx->pin + 4 * q);
-            PIC_HIP(ctx, hipGetLastError());
-            PIC_HIP(ctx, hipEventRecord(ctx->batch_ev[q], ctx->stream));
-            at[q] = it;
-            par[q] = launches & 1;
-            queued++;
-        }
-        if (conv || done == queued) break;
-        rc = wait_oldest();
-        if (rc) return rc;
-    }
-    if (par[last]) std::swap(ctx->phi, ctx->sor_phi);
-    double r[3];
-    for (int q = 0; q < 3; q++) r[q] = hp[4 * last + q];
-    st->converged = conv;
-    st->iterations = at[last];
-    st->newton_iterations = 0;
-    st->ref_l2 = std::sqrt(r[0] / (double)g.nn);
-    st->rel_residual = r[2] > 0 ? std::sqrt(r[1] / r[2]) : std::sqrt(r[1]);
-    return conv ? PIC_OK : PIC_NOT_CONVERGED;
-}
-
-// The iterations of PCG on J y = F after k_F's set-up (vectors of type T, g.g
-// = gg0 > target2); stops at the end of the first batch of `check` iterations
-// in which g.g reached target2, or at max_it.  The host queues the first
-// RUN_AHEAD iterations of the next batch before it waits for one, so the
-// device never idles during a check; once a batch has converged the kernels
-// behind it return at once (the stop flag), so y is the one of the batch that
-// converged.  hp: 2 * check doubles of pinned memory; ggh: max_it + 1 doubles
-// on the device.
-template <typename T, bool NEU>
-static int pcg_inner(pic_ctx* ctx, const Stencil& s, const PcgVec<T>& v, T* d0, T* d1, const CgVec<T>* cg, double* ggh,
-                     double* hp, double target2, int max_it, int check, int* iters) {
-    const unsigned nb = part_blocks(s.nn);
-    if (cg) k_cg<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, *cg, ctx->scratch, ggh, -1);
-    for (auto& e : ctx->batch_ev)
-        if (!e) PIC_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    // profiled runs wait for every batch, so that no returned-at-once
-    // iteration is counted
-    const int ahead = ctx->prof.on ? 1 : 2;
-    int t = 0;                        // iterations queued
-    int beg[2], end[2], queued = 0, done = 0;  // batches queued and waited for
-    T *dold = d0, *dnew = d1;
-    bool conv = false;
-    auto wait_oldest = [&]() {  // for the oldest queued batch; conv: it reached target2
-        const int q = done & 1;
-        const hipError_t e = pic_spin_event(ctx->batch_ev[q]);
-        if (e != hipSuccess) return pic_hip_check(ctx, e, "PCG check");
-        done++;
-        const volatile double* h = hp + (size_t)q * check;
-        for (int m = 0; m < end[q] - beg[q]; m++) {
-            if (!(h[m] == h[m])) return pic_fail(ctx, PIC_ERR_NUMERIC, "PCG produced NaN");
-            if (h[m] <= target2) {
-                *iters = end[q];
-                conv = true;
-                break;
-            }
-        }
-        return (int)PIC_OK;
-    };
-    for (;;) {
-        while (t < max_it && queued - done < ahead) {
-            const int q = queued & 1, t0 = t, upto = check < max_it - t ? t + check : max_it;
-            for (; t < upto; t++) {  // one profiled "launch" = one PCG iteration (1 or 2 kernels)
-                if (t - t0 == RUN_AHEAD && queued > done) {
-                    const int rc = wait_oldest();
-                    if (rc || conv) return rc;
-                }
-                PicProfScope ps(ctx, PIC_K_PCG);
-                if (cg) {
-                    k_cg<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, *cg, ctx->scratch, ggh, t);
-                    continue;
-                }
-                k_pcg1<T, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v, dold, dnew, ctx->scratch, ggh, t);
-                k_pcg2<T, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, v, dnew, ctx->scratch, t);
-                std::swap(dold, dnew);
-            }
-            k_pcg_check<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch,
-                                                      ctx->scratch + (cg ? (t & 1) * PART_SET : 0) + PART_GG, ggh,
-                                                      (int)nb, t0, t, target2, hp + (size_t)q * check);
-            PIC_HIP(ctx, hipGetLastError());
-            PIC_HIP(ctx, hipEventRecord(ctx->batch_ev[q], ctx->stream));
-            beg[q] = t0;
-            end[q] = t;
-            queued++;
-        }
-        if (done == queued) {
-            *iters = t;
-            return PIC_NOT_CONVERGED;
-        }
-        const int rc = wait_oldest();
-        if (rc || conv) return rc;
-    }
-}
-
-// Nodes up to which an iteration is one kernel (k_cg): one launch's latency
-// against three stencil operands instead of one.  Cold solves, two kernels and
-// one: FP32-inner 33^3 1.61 and 1.24 ms, 64^3 3.06 and 2.26, a run on 97 x 65 x 49
-// 16.3 and 14.4, 100^3 6.5 and 7.5; FP64 33^3 1.37 and 1.13, 50^3 1.84 and 1.60, 70^3
-// 3.44 and 3.28, 90^3 5.3 and 6.4.
-template <typename T>
-constexpr size_t CG_ONE_MAX = sizeof(T) == sizeof(float) ? (size_t)1 << 19 : (size_t)3 << 17;
-
-// Newton + PCG (PotentialSolver.cpp:178-241).  The linear case (n0 == 0)
-// needs a single Newton step; each Newton step restarts PCG from y = 0.
-template <typename T, bool NEU>
-static int solve_pcg_t(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st) {
-    const GridC& g = ctx->g;
-    constexpr bool mixed = sizeof(T) == sizeof(float);
-    size_t nn = (size_t)g.nn;
-    Stencil s = make_stencil(g, (p->flags & PIC_SOLVE_AXIS_SWAP) != 0);
-    bool nonlinear = p->n0 != 0.0;
-    int max_it = p->max_it > 0 ? p->max_it : 10000;
-    int check = std::min(p->check_every > 0 ? p->check_every : 8, max_it);
-    // y, g, d0, d1, z (s), P, the g.g history; each vector on a 256-byte line
-    const size_t vs = (nn * sizeof(T) + 255) & ~(size_t)255;
-    const size_t ps = nonlinear ? (nn * sizeof(double) + 255) & ~(size_t)255 : 0;
-    const bool one = !NEU && nn <= CG_ONE_MAX<T>;  // one kernel per iteration (k_cg)
-    const int nvec = NEU ? 6 : one ? 8 : 5;
-    int rc = pic_ensure_work(ctx, nvec * vs + ps + ((size_t)max_it + 2) * sizeof(double));
-    if (rc) return rc;
-    rc = pic_ensure_pin(ctx, (8 + 2 * (size_t)check) * sizeof(double));
-    if (rc) return rc;
-    char* wbase = (char*)ctx->work;
-    auto vec = [&](int q) { return reinterpret_cast<T*>(wbase + q * vs); };
-    double* P = nonlinear ? (double*)(wbase + nvec * vs) : nullptr;
-    double* ggh = (double*)(wbase + nvec * vs + ps);
-    PcgVec<T> v;
-    v.y = vec(0);
-    v.g = vec(1);
-    v.z = vec(4);
-    v.s = NEU ? vec(5) : nullptr;
-    v.P = P;
-    // k_cg's vectors: g's first is k_F's g
-    const CgVec<T> cg{vec(0), vec(2), {vec(1), vec(3)}, {vec(4), vec(5)}, {vec(6), vec(7)}, P};
-    volatile double* hp = ctx->pin;  // [0, 5) sums of k_F, [5] y.y, [8, ...) g.g of the batches
-    NewtonArgs na;
-    na.ieps = 1.0 / EPS0;
-    na.phi0 = p->phi0;
-    na.n0 = p->n0;
-    na.inv_te0 = 1.0 / (p->Te0 != 0 ? p->Te0 : 1.0);
-    const unsigned nb = part_blocks(s.nn);
-    int total_it = 0, newton = 0;
-    bool conv = false, have_r = false;
-    double fr[3];
-    const int newton_max = nonlinear ? 20 : 1000;  // PotentialSolver.cpp:179
-    for (newton = 0; newton < newton_max; newton++) {
-        // set-up launches are not counted as PCG iterations
-        k_F<T, true, NEU><<<nb, BLOCK, 0, ctx->stream>>>(s, na, ctx->ntype, ctx->phi, ctx->rho, v.g, v.s, P,
-                                                         ctx->scratch);
-        // F.F (all rows, regular), b.b, and PCG's g.s, g.g
-        k_sum_parts<<<5, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nb, ctx->pin);
-        PIC_HIP(ctx, hipGetLastError());
-        PIC_HIP(ctx, pic_spin_wait(ctx->stream));
-        for (int q = 0; q < 3; q++) fr[q] = hp[q];
-        const double gg0 = hp[4];
-        // target on the inner residual g (g = -F at y = 0)
-        double target2;
-        if (p->tol_kind == PIC_TOL_REF_RMS)
-            target2 = p->tol * p->tol * (double)nn;
-        else
-            target2 = p->tol * p->tol * (fr[2] > 0 ? fr[2] : 1.0);
-        if (!nonlinear && fr[0] <= target2) {
-            conv = have_r = true;
-            break;
-        }
-        // relative criterion on the nonlinear problem: the FP64 residual F
-        // of the current phi over the regular rows (the Newton iterate is
-        // judged by the residual, not by the size of its last step)
-        if (nonlinear && p->tol_kind == PIC_TOL_REL && fr[1] <= target2) {
-            conv = have_r = true;
-            break;
-        }
-        double inner_target2 = target2;
-        if (mixed) {  // FP32 inner solve: reduce the residual by ~1e-3 per pass
-            double floor2 = fr[0] * 1e-6;
-            inner_target2 = std::max(target2 * 0.25, floor2);
-        } else if (nonlinear && p->tol_kind == PIC_TOL_REL) {
-            // inexact Newton: each linear solve to 1e-4 of the current
-            // residual, or below the final tolerance
-            inner_target2 = std::max(target2 * 0.25, fr[0] * 1e-8);
-        }
-        double yy = 0;
-        if (!(gg0 <= inner_target2)) {  // otherwise y = 0 (a zero right-hand side included)
-            int its = 0;
-            rc = pcg_inner<T, NEU>(ctx, s, v, vec(2), vec(3), one ? &cg : nullptr, ggh, ctx->pin + 8, inner_target2,
-                                   max_it - total_it, check, &its);
-            total_it += its;
-            if (rc < 0) return rc;
-            const bool want_yy = nonlinear && p->tol_kind == PIC_TOL_REF_RMS;
-            k_update_phi<T><<<nb, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->phi, v.y,
-                                                           want_yy ? ctx->scratch + PART_F : nullptr);
-            PIC_HIP(ctx, hipGetLastError());
-            if (want_yy) {
-                k_sum_parts<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nb, ctx->pin + 5);
-                PIC_HIP(ctx, hipGetLastError());
-                PIC_HIP(ctx, pic_spin_wait(ctx->stream));
-                yy = hp[5];
-            }
-        }
-        if (nonlinear && p->tol_kind == PIC_TOL_REF_RMS) {
-            if (std::sqrt(yy / (double)nn) < 1e-3) {  // NR_TOL, PotentialSolver.cpp:180, :229-233
-                conv = true;
-                newton++;
-                break;
-            }
-        }
-        if (total_it >= max_it) break;
-    }
-    double r[3];
-    if (have_r && !NEU) {  // k_F's sums are the residual of the final phi
-        for (int q = 0; q < 3; q++) r[q] = fr[q];
-    } else {
-        SorArgs a;
-        a.omega = 1;
-        a.ieps = 1.0 / EPS0;
-        a.itwos = 1.0 / s.twos;
-        a.phi0 = p->phi0;
-        a.n0 = p->n0;
-        a.inv_te0 = na.inv_te0;
-        rc = residual_norms(ctx, s, a, r);
-        if (rc) return rc;
-    }
-    st->converged = conv;
-    st->iterations = total_it;
-    st->newton_iterations = newton;
-    st->ref_l2 = std::sqrt(r[0] / (double)nn);
-    st->rel_residual = r[2] > 0 ? std::sqrt(r[1] / r[2]) : std::sqrt(r[1]);
-    return conv ? PIC_OK : PIC_NOT_CONVERGED;
-}
-
-static int solve_pcg(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st, bool mixed) {
-    if (has_neumann(ctx))
-        return mixed ? solve_pcg_t<float, true>(ctx, p, st) : solve_pcg_t<double, true>(ctx, p, st);
-    return mixed ? solve_pcg_t<float, false>(ctx, p, st) : solve_pcg_t<double, false>(ctx, p, st);
 }
 
 // ------------------------------------------------------------------------
@@ -2418,7 +964,7 @@ static int solve_learned(pic_ctx* ctx, const pic_solver_params* p, pic_solver_st
         pic_solver_params q2 = *p;
         q2.method = PIC_SOLVER_PCG;
         pic_solver_stats s2;
-        rc = solve_pcg(ctx, &q2, &s2, false);
+        rc = pic_solve_pcg(ctx, &q2, &s2, false);
         *st = s2;
         st->iterations += it;
         return rc;
@@ -2477,14 +1023,12 @@ static int solve_newton_learned(pic_ctx* ctx, const pic_solver_params* p, pic_so
     na.phi0 = p->phi0;
     na.n0 = p->n0;
     na.inv_te0 = 1.0 / (p->Te0 != 0 ? p->Te0 : 1.0);
-    unsigned nb = stencil_blocks(s.nn), nbr = stencil_blocks_red(s.nn), nbp = part_blocks(s.nn);
+    unsigned nb = stencil_blocks(s.nn), nbr = stencil_blocks_red(s.nn);
     int total_it = 0, newton = 0;
     bool conv = false, stalled = false;
     for (newton = 0; newton < 20; newton++) {  // NR_MAX_IT, PotentialSolver.cpp:179
-        k_F<double, false, false><<<nbp, BLOCK, 0, ctx->stream>>>(s, na, ctx->ntype, ctx->phi, ctx->rho, r, nullptr,
-                                                                  P, ctx->scratch);
-        k_sum_parts<<<3, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nbp, hf);
-        PIC_HIP(ctx, hipGetLastError());
+        rc = pic_newton_residual(ctx, s, na, r, P, hf);
+        if (rc) return rc;
         PIC_HIP(ctx, pic_spin_wait(ctx->stream));
         const double bb = hf[2] > 0 ? hf[2] : 1.0;
         const double target2 = p->tol_kind == PIC_TOL_REF_RMS ? p->tol * p->tol * (double)nn
@@ -2539,9 +1083,8 @@ static int solve_newton_learned(pic_ctx* ctx, const pic_solver_params* p, pic_so
             stalled = true;
             break;
         }
-        k_update_phi<double><<<nbp, BLOCK, 0, ctx->stream>>>(s, ctx->ntype, ctx->phi, y, ctx->scratch + PART_F);
-        k_sum_parts<<<1, BLOCK, 0, ctx->stream>>>(ctx->scratch + PART_F, (int)nbp, hf + 3);
-        PIC_HIP(ctx, hipGetLastError());
+        rc = pic_newton_update(ctx, s, y, hf + 3);
+        if (rc) return rc;
         double yy;
         PIC_HIP(ctx, pic_spin_wait(ctx->stream));
         yy = hf[3];
@@ -2555,7 +1098,7 @@ static int solve_newton_learned(pic_ctx* ctx, const pic_solver_params* p, pic_so
         pic_solver_params q2 = *p;
         q2.method = PIC_SOLVER_PCG;
         pic_solver_stats s2;
-        rc = solve_pcg(ctx, &q2, &s2, false);
+        rc = pic_solve_pcg(ctx, &q2, &s2, false);
         *st = s2;
         st->iterations += total_it;
         st->newton_iterations += newton;
@@ -2580,20 +1123,6 @@ static int solve_newton_learned(pic_ctx* ctx, const pic_solver_params* p, pic_so
 }
 
 // plain red-black SOR to a relative tolerance (used to make training pairs)
-int pic_poisson_internal_sor(pic_ctx* ctx, double tol, int max_it, pic_solver_stats* st) {
-    pic_solver_params p{};
-    p.method = PIC_SOLVER_SOR_RB;
-    p.tol_kind = PIC_TOL_REL;
-    p.tol = tol;
-    p.max_it = max_it;
-    int nmax = std::max(ctx->g.ni, std::max(ctx->g.nj, ctx->g.nk));
-    p.omega = 2.0 / (1.0 + std::sin(3.141592653589793 / (nmax - 1)));
-    p.check_every = 25;
-    int rc = pic_ensure_ntype(ctx);
-    if (rc) return rc;
-    return solve_sor(ctx, &p, st);
-}
-
 extern "C" int pic_poisson(pic_ctx* ctx, const pic_solver_params* p, pic_solver_stats* st) {
     if (!ctx || !p) return PIC_ERR_ARG;
     if (!(p->tol > 0) || p->max_it <= 0) return pic_fail(ctx, PIC_ERR_ARG, "bad solver params");
@@ -2620,9 +1149,9 @@ extern "C" int pic_poisson(pic_ctx* ctx, const pic_solver_params* p, pic_solver_
         }
     }
     switch (p->method) {
-        case PIC_SOLVER_SOR_RB: rc = solve_sor(ctx, p, st); break;
-        case PIC_SOLVER_PCG: rc = solve_pcg(ctx, p, st, false); break;
-        case PIC_SOLVER_PCG_MIXED: rc = solve_pcg(ctx, p, st, true); break;
+        case PIC_SOLVER_SOR_RB: rc = pic_solve_sor(ctx, p, st); break;
+        case PIC_SOLVER_PCG: rc = pic_solve_pcg(ctx, p, st, false); break;
+        case PIC_SOLVER_PCG_MIXED: rc = pic_solve_pcg(ctx, p, st, true); break;
         case PIC_SOLVER_LEARNED:
             rc = p->n0 != 0.0 ? solve_newton_learned(ctx, p, st) : solve_learned(ctx, p, st);
             break;
