@@ -46,14 +46,14 @@ ALG_BYTES = {
     "scatter": 64.0,   # push into the sorted position: the 32-byte particle read and written
     "deposit": 16.0,   # x, y, z, w
     "pcg": 44.0,       # FP32 inner PCG: per node and iteration (88 B in FP64)
-    "sor": 24.0,       # FP64 phi r/w + rho read per node and sweep
+    "sor": 25.0,       # per node and launch: FP64 phi read and written, rho and the row bits read
 }
 # the learned solver's flexible-CG vector updates per node and iteration: p, q
 # (FP64) from z (FP32) and the previous p (28 B), then x, r updated from p, q (48 B)
 ALG_BYTES_FCG = 76.0
 KERNEL_NAMES = {
     "push": "k_push<false,2>", "scatter": "k_push_scatter", "deposit": "k_dep_cells + k_dep_nodes",
-    "pcg": "k_pcg1<float> + k_pcg2<float>", "sor": "k_sor_tile (two sweeps per launch)",
+    "pcg": "k_pcg1<float> + k_pcg2<float>", "sor": "k_sor_tile (up to two sweeps per launch)",
 }
 
 
@@ -843,6 +843,7 @@ def main():
     ctx.sync()
     prof = ctx.profile_read()
     ctx.profile(False)
+    prof_iters = sum(solve_iters[args.steps:])  # the profiled steps' solver iterations
     K = args.steps
     n_alive = ctx.count(se) + ctx.count(si)
     value = 2 * N * K / T  # pushes issued (both species, every step)
@@ -870,17 +871,15 @@ def main():
     dom = max(cand, key=lambda k: cand[k][0])
     tot_ms, launches = cand[dom]
     avg_s = tot_ms * 1e-3 / launches
-    if dom == "pcg":
-        units = ctx.nn
-    elif dom == "sor":
-        units = 2 * ctx.nn  # one profiled launch = two red-black sweeps
-    else:
-        units = N
+    units = ctx.nn if dom in ("pcg", "sor") else N
     per_unit = ALG_BYTES[dom]
     if dom == "pcg" and step_solver == "learned":
         per_unit = ALG_BYTES_FCG
     alg = per_unit * units
     achieved = alg / avg_s / 1e9
+    # the nodes that the sweeps went over (a launch makes one sweep where an odd
+    # number is left before a check), which do not bound the traffic
+    swept = prof_iters * ctx.nn / (tot_ms * 1e-3) if dom == "sor" else None
     # the network's forward as a whole against the dense BF16 MFMA peak
     roof_net = None
     if net_meta is not None and prof.get("unet", (0, 0))[1]:
@@ -939,7 +938,8 @@ def main():
                      "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": traffic, "alg_bytes_per_launch": alg,
-                     "avg_launch_ms": avg_s * 1e3},
+                     "avg_launch_ms": avg_s * 1e3,
+                     **({"swept_nodes_per_s": swept} if swept else {})},
         "roofline_network": roof_net,
         "rooflines": rooflines,
         "deposits_per_s": deposits_per_s,
