@@ -42,7 +42,8 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # dense BF16 (MI355X)
 
 # algorithmic bytes per unit of work (per particle, or per node and iteration)
 ALG_BYTES = {
-    "push": 24.0,      # histogram pass of the push: read x, y, z, vx, vy, vz (FP32)
+    "push": 5.0,       # histogram pass of the push: the cell word and the flag (x, y, z and the
+                       # velocity, 24 more, of the particles without one not counted)
     "scatter": 64.0,   # push into the sorted position: the 32-byte particle read and written
     "deposit": 16.0,   # x, y, z, w
     "pcg": 44.0,       # FP32 inner PCG: per node and iteration (88 B in FP64)
