@@ -158,3 +158,21 @@ def test_sor_without_memory_for_the_second_potential(pg):
         out.append(c.get_field(pg.FIELD_PHI))
         c.close()
     assert np.array_equal(out[0], out[1])
+
+
+def test_velocity_moments_without_memory_for_all_of_them(pg):
+    """n v is interleaved on the device in pieces of 25 MB; 24 bytes for every
+    node (80 MB here) are not asked for."""
+    shape = (150, 150, 150)
+    L = 1e-2 * (np.array(shape) - 1)
+    c = pg.Context(*shape, [0, 0, 0], L)
+    sid = c.species_add(ME, 0.0, 1.0, 100)
+    p = np.zeros((100, 7))
+    p[:, :3] = 0.5 * L
+    p[:, 3:7] = [1.0, 2.0, -4.0, 1.0]
+    c.upload(sid, p)
+    c.deposit(sid, pg.DEPOSIT_DENSITY | pg.DEPOSIT_MOMENTS)
+    with _Hog(c, 48 * MB):
+        nv = c.species_field(sid, pg.SFIELD_NVSUM)
+    assert np.allclose(nv.reshape(-1, 3).sum(0), [100.0, 200.0, -400.0], rtol=1e-6)
+    c.close()

@@ -301,6 +301,32 @@ def test_upload_in_pieces(pg, num):
     c.close()
 
 
+@pytest.mark.parametrize("shape", [(3, 3, 3), (64, 128, 128), (64, 128, 129), (129, 131, 127)])
+def test_velocity_moments_in_pieces(pg, shape):
+    """n v of grids of up to one, just over one and over two staging pieces of
+    2^20 nodes: with one velocity of powers of two for all particles it is the
+    density sum times that velocity, bit for bit."""
+    dx = 1e-2
+    L = dx * (np.array(shape) - 1)
+    rng = np.random.default_rng(4)
+    num = 300_000
+    p = np.zeros((num, 7))
+    p[:, :3] = rng.uniform(0.001, 0.999, (num, 3)) * L
+    v = np.array([2.0, -64.0, 0.25])
+    p[:, 3:6] = v
+    p[:, 6] = rng.uniform(0.5, 2.0, num)
+    c = pg.Context(*shape, [0, 0, 0], L)
+    sid = c.species_add(ME, 0.0, 1.0, num)
+    c.upload(sid, p)
+    c.clear_samples(sid)
+    c.deposit(sid, pg.DEPOSIT_DENSITY | pg.DEPOSIT_MOMENTS)
+    n = c.species_field(sid, pg.SFIELD_NSUM)
+    nv = c.species_field(sid, pg.SFIELD_NVSUM).reshape(-1, 3)
+    assert n.sum() > 0.99 * p[:, 6].sum()
+    assert np.array_equal(nv, n[:, None] * v)
+    c.close()
+
+
 @pytest.mark.parametrize("shape", [(3, 3, 3), (5, 5, 64), (33, 33, 5), (33, 33, 6), (17, 65, 67), (50, 100, 201)])
 def test_cell_offsets_at_scan_tile_edges(pg, shape):
     """cell counts below, at and above a scan row (1024) and tile (4096), and
