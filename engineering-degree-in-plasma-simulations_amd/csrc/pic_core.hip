@@ -405,7 +405,7 @@ extern "C" int pic_species_add(pic_ctx* ctx, double mass, double charge, double 
     }
     // ranks; pic_push_sort keeps 64 run bases per group of 64 particles here
     if (e == hipSuccess) e = hipMalloc(&s.rank, (c + 63) / 64 * 64 * 4);
-    if (e == hipSuccess) e = hipMalloc(&s.count, ((size_t)g.ncells + 2) * 4);
+    if (e == hipSuccess) e = hipMalloc(&s.count, count_bytes(g));
     if (e == hipSuccess) e = hipMalloc(&s.off, ((size_t)g.ncells + 2) * 4);
     if (e == hipSuccess) e = hipMalloc(&s.d_n, 4 * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc(&s.den, (size_t)g.nn * sizeof(double));
@@ -422,10 +422,10 @@ extern "C" int pic_species_add(pic_ctx* ctx, double mass, double charge, double 
         (void)hipFree(s.den);
         return pic_hip_check(ctx, e, "species allocation");
     }
-    // pic_push_sort's flags, their bound and counts; a species does without
-    // where there is no memory for them
+    // pic_push_sort's flags and their bound; a species does without where
+    // there is no memory for them
     const size_t safe_bytes = (c + 255) / 256 * 256;
-    if (hipMalloc(&s.safe, safe_bytes + 8 * sizeof(float)) == hipSuccess)
+    if (hipMalloc(&s.safe, safe_bytes + 4 * sizeof(float)) == hipSuccess)
         s.safe_kick = reinterpret_cast<float*>(s.safe + safe_bytes);
     else
         (void)hipGetLastError();
@@ -540,7 +540,7 @@ extern "C" int pic_particles_upload(pic_ctx* ctx, int sid, const double* aos7, s
     PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
     s.n_upper = n;
     s.hist_valid = false;
-    s.safe_ok = false;
+    s.safe_ok = s.safe_left = s.safe_unused = false;
     s.sorted = false;
     s.two_part = false;
     s.tail_ok = false;

@@ -68,6 +68,9 @@ __host__ __device__ inline void unpack_cell(uint32_t c, int& i, int& j, int& k) 
 __host__ __device__ inline int cell_index(const GridC& g, int i, int j, int k) {
     return (k * g.cj + j) * g.ci + i;
 }
+// Species::count: ncells + 3 words, in whole 16 bytes (2M cells: other sizes are
+// cleared 1.2 us slower)
+inline size_t count_bytes(const GridC& g) { return ((size_t)g.ncells + 3 + 3) / 4 * 16; }
 // 1 / node volume (World.cpp:353-367): half volume per boundary axis
 __host__ __device__ inline double inv_node_vol(const GridC& g, int i, int j, int k) {
     double s = g.inv_dx[0] * g.inv_dx[1] * g.inv_dx[2];
@@ -148,7 +151,7 @@ struct Species {
     int cur = 0;
     void* block[2] = {nullptr, nullptr};
     uint32_t* rank = nullptr;    // rank of each particle inside its cell bucket
-    uint32_t* count = nullptr;   // ncells + 1 buckets (the last, the removed ones', stays 0)
+    uint32_t* count = nullptr;   // ncells + 1 buckets (the last, the removed ones', stays 0); then SafeArgs::tally
     uint32_t* off = nullptr;     // ncells + 2 exclusive offsets
     uint32_t* d_n = nullptr;     // [0] live count, [1] count the histogram covers, [2] overflow
     size_t n_upper = 0;          // host upper bound of the live count
@@ -176,9 +179,10 @@ struct Species {
     // that call left them: every call that moves, reorders, adds or changes
     // particles clears safe_ok.
     uint8_t* safe = nullptr;     // null: no memory for them
-    float* safe_kick = nullptr;  // device, 3 floats (-1: no flags left), then two pairs of counts by turns
-    uint32_t safe_calls = 0;
+    float* safe_kick = nullptr;  // device, 3 floats (-1: no flags left)
     bool safe_ok = false;
+    // the last pic_push_sort may have left flags; the last ones went unused
+    bool safe_left = false, safe_unused = false;
     float safe_dtx[3] = {0.f, 0.f, 0.f};
     double* den = nullptr;       // number density
     double* mom = nullptr;       // n, nvx, nvy, nvz, nuu, nvv, nww (7 * nn)

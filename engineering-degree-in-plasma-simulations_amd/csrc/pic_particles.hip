@@ -106,20 +106,24 @@ struct PushArgs {
 // them costs k_push_scatter about 3%.  They are of use only to a
 // pic_push_sort that follows with the particles unchanged, and only if nearly
 // all particles have one, since loads are saved line by line.  So a call
-// leaves flags (or kick = -1, which no kick is within) if it is itself such a
-// call (`allow`) and the call before found at most one particle in SAFE_RARE
-// without; every call counts those of every 64th workgroup.  20M particles at
-// 128^3, us per call in a run of calls with flags always, never and by this rule:
-// ions, which hardly move, 373, 433, 374; electrons of which 3% may leave 509,
-// 512, 510; with steps 10 and 50 times as long 749, 727, 727 and 1042, 1006, 1007.
+// leaves flags (or kick = -1, which no kick is within) unless the species'
+// last ones went unused (`allow`), and if its own histogram pass found at most
+// one particle in SAFE_RARE that may leave its cell among those of up to 32
+// workgroups.  20M particles at 128^3, us per call in a run of calls with
+// flags always, never and by this rule: ions, which hardly move, 374, 434, 376;
+// electrons of which 3% may leave 510, 514, 509; with steps 10 and 50 times as
+// long 750, 728, 721 and 1043, 1007, 1001.
 struct SafeArgs {
-    uint8_t* flags;  // null: none
-    float* kick;     // the kick that they hold for, 3 floats
-    const uint32_t* prev;  // counted by the call before: particles that may leave, particles
-    uint32_t* next;        // counted by this call
+    uint8_t* flags;   // null: none
+    float* kick;      // the kick that they hold for, 3 floats
+    uint32_t* tally;  // particles that may leave | particles << 16 of these; cleared before the histogram pass
+    // the histogram pass's workgroups whose index has none of these bits tally:
+    // 16 to 32 of them (3000 adding to the one word took 8% of a pass over 200M particles)
+    unsigned skip;
     int allow;
 };
 constexpr uint32_t SAFE_RARE = 32;
+static_assert(32 * BLOCK * 2 < 1 << 16, "a tally's halves");  // two particles per thread
 
 // A particle whose drift cannot take it out of its cell, whatever E it
 // gathers: for every axis |f' - f| <= (|v| + |qm dt| max|E|) dt/dx (with
@@ -449,8 +453,7 @@ __global__ void __launch_bounds__(BLOCK)
     k_push(GridC g, SpeciesBuf b, const float4* __restrict__ E, PushArgs a,
            uint32_t* __restrict__ d_n, uint32_t* __restrict__ count, uint32_t* __restrict__ rank,
            const uint8_t* __restrict__ safe, SafeArgs sa) {
-    const size_t p0 = xcd_wg() * (BLOCK * ILP) + threadIdx.x;
-    if (!WRITE && !SURF && sa.flags && p0 < 2) sa.next[p0] = 0;  // for the k_push_scatter that follows
+    const size_t wg = xcd_wg(), p0 = wg * (BLOCK * ILP) + threadIdx.x;
     uint32_t n = d_n[0];
     uint32_t covered = gridDim.x * BLOCK * ILP;
     if (n > covered) n = covered;
@@ -465,6 +468,8 @@ __global__ void __launch_bounds__(BLOCK)
         for (int d = 0; d < 3; d++) kick[d] = fabsf(a.qmdt) * a.emax[d];
     const bool use_safe = bound && safe != nullptr && kick[0] <= sa.kick[0] && kick[1] <= sa.kick[1] &&
                           kick[2] <= sa.kick[2];  // (the whole grid; false for NaN)
+    const bool tally = bound && sa.flags != nullptr && ((unsigned)wg & sa.skip) == 0;  // (the workgroup)
+    uint32_t tallied = 0;
     uint8_t stay[ILP];
 #pragma unroll
     for (int q = 0; q < ILP; q++) {
@@ -495,9 +500,9 @@ __global__ void __launch_bounds__(BLOCK)
         if (valid) {
             key = (uint32_t)g.ncells;
             if (c[q] != DEAD) {
-                const uint32_t nc = (stay[q] || (bound && stays_in_cell(f[q], v[q], kick, a.dtx)))
-                                        ? c[q]
-                                        : advance<SURF>(g, E, a, c[q], f[q], v[q], b, p);
+                const bool in = stay[q] || (bound && stays_in_cell(f[q], v[q], kick, a.dtx));
+                if (tally) tallied += in ? 1u << 16 : (1u << 16) + 1u;
+                const uint32_t nc = in ? c[q] : advance<SURF>(g, E, a, c[q], f[q], v[q], b, p);
                 key = cell_key(g, nc);
                 if (WRITE) {
                     if (nc != c[q]) b.cell[p] = nc;  // most particles stay in their cell
@@ -515,6 +520,10 @@ __global__ void __launch_bounds__(BLOCK)
         } else {
             run_bases(key, valid, (uint32_t)g.ncells, count, rank + (p & ~(size_t)63));  // the group's run bases
         }
+    }
+    if (tally) {
+        for (int o = 32; o > 0; o >>= 1) tallied += __shfl_xor(tallied, o, 64);
+        if ((threadIdx.x & 63) == 0) atomicAdd(sa.tally, tallied);
     }
 }
 
@@ -1076,18 +1085,15 @@ __global__ void __launch_bounds__(BLOCK)
     k_push_scatter(GridC g, SpeciesBuf src, SpeciesBuf dst, const float4* __restrict__ E, PushArgs a,
                    const uint32_t* __restrict__ bases, const uint32_t* __restrict__ off,
                    const uint32_t* __restrict__ d_n, uint32_t cap, SafeArgs sa) {
-    const size_t wg = xcd_wg(), p0 = wg * (BLOCK * ILP) + threadIdx.x;
-    // the next push's flags, for a field that at most doubles
-    const bool count = !SURF && sa.flags != nullptr && (wg & 63) == 0;                               // (the workgroup)
-    const bool leave = !SURF && sa.flags != nullptr && sa.allow && sa.prev[0] * SAFE_RARE <= sa.prev[1];  // (the grid)
+    const size_t p0 = xcd_wg() * (BLOCK * ILP) + threadIdx.x;
+    // the next push's flags, for a field that at most doubles; the tally is
+    // first waited for where they are stored
+    const bool may_flag = !SURF && sa.flags && sa.allow;
+    const uint32_t tally = may_flag ? *sa.tally : 0u;
     float kick2[3] = {0.f, 0.f, 0.f};
-    uint32_t may_leave = 0, counted = 0;
-    if (count || leave) {
-        if (a.kick)
+    if (may_flag && a.kick)
 #pragma unroll
-            for (int d = 0; d < 3; d++) kick2[d] = 2.f * fabsf(a.qmdt) * a.emax[d];
-        if (p0 < 3) sa.kick[p0] = !leave ? -1.f : p0 == 0 ? kick2[0] : p0 == 1 ? kick2[1] : kick2[2];
-    }
+        for (int d = 0; d < 3; d++) kick2[d] = 2.f * fabsf(a.qmdt) * a.emax[d];
     const uint32_t n = d_n[1];
     uint32_t c[ILP];
     float f[ILP][3], v[ILP][3], w[ILP];
@@ -1111,6 +1117,7 @@ __global__ void __launch_bounds__(BLOCK)
             w[q] = src.w[p];
         }
     }
+    const bool leave = may_flag && (tally & 0xFFFFu) * SAFE_RARE <= tally >> 16;  // (the grid)
 #pragma unroll
     for (int q = 0; q < ILP; q++) {
         const size_t p = p0 + (size_t)q * BLOCK;
@@ -1134,23 +1141,9 @@ __global__ void __launch_bounds__(BLOCK)
             dst.v[d][dst_i] = v[q][d];
         }
         dst.w[dst_i] = w[q];
-        if (count || leave) {
-            const bool stay = stays_in_cell(f[q], v[q], kick2, a.dtx);
-            if (leave) sa.flags[dst_i] = stay ? 1 : 0;
-            may_leave += stay ? 0 : 1;
-            counted++;
-        }
+        if (leave) sa.flags[dst_i] = stays_in_cell(f[q], v[q], kick2, a.dtx) ? 1 : 0;
     }
-    if (count) {
-        for (int o = 32; o > 0; o >>= 1) {
-            may_leave += __shfl_xor(may_leave, o, 64);
-            counted += __shfl_xor(counted, o, 64);
-        }
-        if ((threadIdx.x & 63) == 0) {
-            atomicAdd(&sa.next[0], may_leave);
-            atomicAdd(&sa.next[1], counted);
-        }
-    }
+    if (!SURF && sa.flags && p0 < 3) sa.kick[p0] = !leave ? -1.f : p0 == 0 ? kick2[0] : p0 == 1 ? kick2[1] : kick2[2];
 }
 
 // Number density without atomics, in two passes over the sorted particles.
@@ -2275,13 +2268,15 @@ extern "C" int pic_push_sort(pic_ctx* ctx, int sid, double dt) {
     bool safe = flags && s.safe_ok;
     SafeArgs sa{};
     if (flags) {
-        uint32_t* stat = reinterpret_cast<uint32_t*>(s.safe_kick + 4);
-        sa = SafeArgs{s.safe, s.safe_kick, stat + 2 * (s.safe_calls & 1), stat + 2 * (~s.safe_calls & 1), s.safe_ok};
-        s.safe_calls++;
+        s.safe_unused = !s.safe_ok && (s.safe_left || s.safe_unused);
+        s.safe_left = !s.safe_unused;
+        unsigned skip = 1;  // a power of two
+        while (skip * 32 <= xcd_blocks1(n, BLOCK * PUSH_SORT_ILP)) skip *= 2;
+        sa = SafeArgs{s.safe, s.safe_kick, s.count + g.ncells + 2, skip - 1, s.safe_left};
     }
     for (int d = 0; d < 3; d++) safe = safe && fabsf(a.dtx[d]) <= s.safe_dtx[d];
     s.safe_ok = false;
-    PIC_HIP(ctx, hipMemsetAsync(s.count, 0, ((size_t)g.ncells + 1) * 4, ctx->stream));
+    PIC_HIP(ctx, hipMemsetAsync(s.count, 0, count_bytes(g), ctx->stream));  // and the tally
     {
         PicProfScope ps(ctx, PIC_K_PUSH);
         const unsigned nb = xcd_blocks1(n, BLOCK * PUSH_SORT_ILP);
@@ -2436,7 +2431,7 @@ extern "C" int pic_load_box_thermal(pic_ctx* ctx, int sid, const double centre[3
     s.n_upper = base + num_macro;
     s.hist_valid = false;
     s.sorted = false;
-    s.safe_ok = false;
+    s.safe_ok = s.safe_left = s.safe_unused = false;
     s.two_part = false;
     s.tail_ok = false;
     s.scrambled = true;  // uniform positions in thread order
