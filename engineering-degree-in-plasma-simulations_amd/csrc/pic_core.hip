@@ -157,7 +157,6 @@ extern "C" void pic_destroy(pic_ctx* ctx) {
     for (auto& s : ctx->sp) {
         for (int b = 0; b < 2; b++) (void)hipFree(s.block[b]);
         (void)hipFree(s.rank);
-        (void)hipFree(s.safe);
         (void)hipFree(s.count);
         (void)hipFree(s.off);
         (void)hipFree(s.d_n);
@@ -403,12 +402,23 @@ extern "C" int pic_species_add(pic_ctx* ctx, double mass, double charge, double 
         }
         s.buf[b].w = (float*)(base + 7 * stride);
     }
-    // ranks; pic_push_sort keeps 64 run bases per group of 64 particles here
-    if (e == hipSuccess) e = hipMalloc(&s.rank, (c + 63) / 64 * 64 * 4);
     if (e == hipSuccess) e = hipMalloc(&s.count, count_bytes(g));
     if (e == hipSuccess) e = hipMalloc(&s.off, ((size_t)g.ncells + 2) * 4);
     if (e == hipSuccess) e = hipMalloc(&s.d_n, 4 * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc(&s.den, (size_t)g.nn * sizeof(double));
+    // last, ranks (pic_push_sort keeps 64 run bases per group of 64 particles here),
+    // and with them pic_push_sort's flags and their bound; a species does
+    // without these where there is no memory for them
+    const size_t rank_bytes = (c + 63) / 64 * 64 * 4, safe_bytes = (c + 255) / 256 * 256;
+    if (e == hipSuccess) {
+        if (hipMalloc(&s.rank, rank_bytes + safe_bytes + 4 * sizeof(float)) == hipSuccess) {
+            s.safe = reinterpret_cast<uint8_t*>(s.rank) + rank_bytes;
+            s.safe_kick = reinterpret_cast<float*>(s.safe + safe_bytes);
+        } else {
+            (void)hipGetLastError();
+            e = hipMalloc(&s.rank, rank_bytes);
+        }
+    }
     if (e == hipSuccess) e = hipMemsetAsync(s.d_n, 0, 4 * sizeof(uint32_t), ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(s.den, 0, (size_t)g.nn * sizeof(double), ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(s.off, 0, ((size_t)g.ncells + 2) * 4, ctx->stream);
@@ -422,13 +432,6 @@ extern "C" int pic_species_add(pic_ctx* ctx, double mass, double charge, double 
         (void)hipFree(s.den);
         return pic_hip_check(ctx, e, "species allocation");
     }
-    // pic_push_sort's flags and their bound; a species does without where
-    // there is no memory for them
-    const size_t safe_bytes = (c + 255) / 256 * 256;
-    if (hipMalloc(&s.safe, safe_bytes + 4 * sizeof(float)) == hipSuccess)
-        s.safe_kick = reinterpret_cast<float*>(s.safe + safe_bytes);
-    else
-        (void)hipGetLastError();
     s.sorted = true;  // empty set is trivially sorted
     ctx->sp.push_back(s);
     *sid = (int)ctx->sp.size() - 1;

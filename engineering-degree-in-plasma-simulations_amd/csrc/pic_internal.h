@@ -178,7 +178,7 @@ struct Species {
     // drifts of at most safe_dtx cells per m/s.  They describe the arrays as
     // that call left them: every call that moves, reorders, adds or changes
     // particles clears safe_ok.
-    uint8_t* safe = nullptr;     // null: no memory for them
+    uint8_t* safe = nullptr;     // (in rank's block; null: no memory for them)
     float* safe_kick = nullptr;  // device, 3 floats (-1: no flags left)
     bool safe_ok = false;
     // the last pic_push_sort may have left flags; the last ones went unused
