@@ -302,10 +302,13 @@ extern "C" int pic_dirichlet_walls(pic_ctx* ctx) {
     if (!ctx) return PIC_ERR_ARG;
     const GridC& g = ctx->g;
     for (int k = 0; k < g.nk; k++)
-        for (int j = 0; j < g.nj; j++)
-            for (int i = 0; i < g.ni; i++)
-                if (i == 0 || i == g.ni - 1 || j == 0 || j == g.nj - 1 || k == 0 || k == g.nk - 1)
-                    ctx->node_type_in[((size_t)k * g.nj + j) * g.ni + i] = 2;
+        for (int j = 0; j < g.nj; j++) {
+            int32_t* row = ctx->node_type_in.data() + ((size_t)k * g.nj + j) * g.ni;
+            if (j == 0 || j == g.nj - 1 || k == 0 || k == g.nk - 1)
+                std::fill(row, row + g.ni, 2);
+            else
+                row[0] = row[g.ni - 1] = 2;
+        }
     ctx->ntype_dirty = true;
     return PIC_OK;
 }

@@ -214,3 +214,17 @@ def test_row_types_of_open_boxes(pg, shape, objects):
                 else:
                     assert phi[k, j, i] != old[k, j, i]
     c.close()
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (5, 3, 4), (9, 8, 7), (3, 12, 6)])
+def test_dirichlet_walls_flag_every_face_node(pg, shape):
+    L = [1e-2 * (n - 1) for n in shape]
+    c = pg.Context(*shape, [0, 0, 0], L)
+    before = c.node_flags()[1].reshape(shape[::-1])
+    c.dirichlet_walls()
+    after = c.node_flags()[1].reshape(shape[::-1])
+    face = np.ones(shape[::-1], bool)
+    face[1:-1, 1:-1, 1:-1] = False
+    assert np.all(before[face] == 1) and np.all(after[face] == 2)
+    assert np.all(before[~face] == 0) and np.all(after[~face] == 0)
+    c.close()
